@@ -5,7 +5,7 @@
 
 namespace ftdx {
 
-// Triangle tiles (32x32) per channel and 32-blocks per dimension of the gain kernel.
+// Triangle tiles (64x64) per channel and 64-blocks per dimension of the gain kernel.
 int gain_tiles(int N);
 int gain_blocks(int N);
 

@@ -765,7 +765,10 @@ int ftdx_gain_loss_grad_noalloc(const void* V, const void* M, const void* g, int
     int rc = ftdx::gain_check_args("ftdx_gain_loss_grad_noalloc", V, M, g, N, batch_count, loss, grad_g,
                                    Gamma);
     if (rc != FTDX_OK || N == 0 || batch_count == 0) return rc;
-    const size_t need = ftdx::gain_scratch_bytes(N, batch_count);
+    // the documented limit counts partials per 32-row block; the kernels' own 64-row blocks
+    // need about half of it
+    const size_t nb = ((size_t)N + 31) / 32;
+    const size_t need = 2 * (size_t)batch_count * nb * N * 8 + (size_t)batch_count * (nb * (nb + 1) / 2) * 8;
     if (need > ftdx::kGainStaticScratchBytes)
         return fail(FTDX_ERR_INVALID_ARG,
                     "ftdx_gain_loss_grad_noalloc: N=" + std::to_string(N) + ", batch=" +

@@ -207,3 +207,43 @@ def test_calibration_full_size_vs_fp64(dev):
             fd = (Lg(h * unit) - Lg(-h * unit)) / (2 * h)
             an = float(grad[0, k, 0] if unit == 1.0 else grad[0, k, 1])
             assert abs(fd - an) <= 1e-4 * float(grad64.abs().max()), (k, unit, fd, an)
+
+
+@pytest.mark.parametrize("N", [1, 2, 63, 64, 65, 127, 130, 193])
+def test_gain_tile_edges_vs_fp64(dev, N):
+    """Loss, gradient and Gamma at the edges of the 64 x 64 gain tiles (one element, one short
+    of a tile, one past it, odd last columns), next to a channel of NaNs that must not leak.
+    Bounds from the arithmetic: a term is a product of at most 4 complex factors (32 roundings),
+    a gradient the sum of N + 1 of them, so its error stays below (N + 40) 2^-24 times the sum
+    of the terms' magnitudes; the loss is summed in FP64 from residuals with 8 roundings."""
+    import torch
+    from ftd_amd import ftdx
+    P = N * (N + 1) // 2
+    gen = torch.Generator(device="cpu").manual_seed(N)
+    V, M = (torch.randn((2, P, 2), generator=gen) for _ in range(2))
+    g = torch.randn((2, N, 2), generator=gen)
+    V[1] = float("nan")
+    M[1] = float("nan")
+    i, j = np.tril_indices(N)
+    i, j = torch.from_numpy(i), torch.from_numpy(j)
+    V[0, i == j, 1] = 0.0
+    loss, grad, Gamma = ftdx.gain_loss_grad(ftdx.CutlassComplexGemm(), V.to(dev), M.to(dev), g.to(dev), N, 2)
+    torch.cuda.synchronize()
+    v, m, c = (torch.view_as_complex(x[0].double()) for x in (V, M, g))
+    p = c[i] * c[j].conj()
+    R = v - p * m
+    eps = 2.0 ** -24
+    size = v.abs() + (p * m).abs()  # of the residual's operands
+    want = float((R.abs() ** 2).sum())
+    assert abs(float(loss[0]) - want) <= 32 * eps * float((size ** 2).sum())
+    G = -2.0 * R * p.conj()
+    err = (torch.view_as_complex(Gamma[0].double().cpu()) - G).abs()
+    assert bool((err <= 64 * eps * size * p.abs()).all())
+    ref = torch.zeros(N, dtype=torch.complex128)
+    mag = torch.zeros(N, dtype=torch.float64)
+    for k, t, s in ((i, -2.0 * R * m.conj() * c[j], c[j]), (j, -2.0 * R.conj() * m * c[i], c[i])):
+        ref.index_add_(0, k, t)
+        mag.index_add_(0, k, 2.0 * size * m.abs() * s.abs())
+    err = (torch.view_as_complex(grad[0].double().cpu()) - ref).abs()
+    assert bool((err <= 2 * (N + 40) * eps * mag).all())
+    assert bool(torch.isnan(grad[1]).all()) and bool(torch.isnan(loss[1]))
