@@ -581,6 +581,12 @@ struct TileRunner {
     // baseline i(i+1)/2 + j; UV in wavelengths = float(uv_m / lambda) (double division);
     // cell = roundf(u / cell + Ng/2); the visibility alpha * C_ij (Im = 0 on the diagonal)
     // is added there and, for i != j, its conjugate at (-u, -v).
+    static __device__ __forceinline__ int64_t grid_cell(const TileJob& j, float u_lam, float v_lam, float half_ng) {
+        const int iu = (int)__builtin_roundf(u_lam / j.cell + half_ng);
+        const int iv = (int)__builtin_roundf(v_lam / j.cell + half_ng);
+        return iu >= 0 && iu < j.Ng && iv >= 0 && iv < j.Ng ? (int64_t)iv * j.Ng + iu : -1;
+    }
+
     static __device__ __forceinline__ void epilogue_grid(const TileJob& j, const v16f (&acc_re)[Cfg::FM][Cfg::FN],
                                                          const v16f (&acc_im)[Cfg::FM][Cfg::FN], int wrow0,
                                                          int wcol0, int lane) {
@@ -595,28 +601,18 @@ struct TileRunner {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int gi = wrow0 + a * 32 + (r >> 2) * 8 + g4 + (r & 3);
-                    if (gi >= j.N || gj > gi) continue;
                     const float vre = acc_re[a][b][r] * j.alpha;
                     const float vim = gi == gj ? 0.0f : acc_im[a][b][r] * j.alpha;
-                    const int64_t k = tri_index(gi, gj);
-                    const float u_lam = (float)((double)j.uv[2 * k] / j.lambda);
-                    const float v_lam = (float)((double)j.uv[2 * k + 1] / j.lambda);
-                    const int iu = (int)__builtin_roundf(u_lam / j.cell + half_ng);
-                    const int iv = (int)__builtin_roundf(v_lam / j.cell + half_ng);
-                    if (iu >= 0 && iu < j.Ng && iv >= 0 && iv < j.Ng) {
-                        float* g = grid + 2 * ((int64_t)iv * j.Ng + iu);
-                        unsafeAtomicAdd(g, vre);
-                        unsafeAtomicAdd(g + 1, vim);
+                    int64_t cell = -1, conj = -1;
+                    if (gi < j.N && gj <= gi) {
+                        const int64_t k = tri_index(gi, gj);
+                        const float u_lam = (float)((double)j.uv[2 * k] / j.lambda);
+                        const float v_lam = (float)((double)j.uv[2 * k + 1] / j.lambda);
+                        cell = grid_cell(j, u_lam, v_lam, half_ng);
+                        if (gi != gj) conj = grid_cell(j, -u_lam, -v_lam, half_ng);
                     }
-                    if (gi != gj) {
-                        const int iuc = (int)__builtin_roundf(-u_lam / j.cell + half_ng);
-                        const int ivc = (int)__builtin_roundf(-v_lam / j.cell + half_ng);
-                        if (iuc >= 0 && iuc < j.Ng && ivc >= 0 && ivc < j.Ng) {
-                            float* g = grid + 2 * ((int64_t)ivc * j.Ng + iuc);
-                            unsafeAtomicAdd(g, vre);
-                            unsafeAtomicAdd(g + 1, -vim);
-                        }
-                    }
+                    grid_add(grid, cell, vre, vim);
+                    grid_add(grid, conj, vre, -vim);
                 }
             }
     }

@@ -13,7 +13,7 @@
 //                        pillbox_grid_scatter_fp32_fp32grid_kernel,
 //                        include/kernels/imaging_kernels.cuh:219-270).
 //
-// Both are HBM/atomic-bound, one grid-stride pass.  The UV cell arithmetic keeps the
+// Both are HBM/atomic-bound, one grid-stride pass (grid_add in herk_common.h on the atomics).  The UV cell arithmetic keeps the
 // reference's float / double steps (wavelength in double, u_lambda rounded to float,
 // roundf of u_lambda / cell + Ng/2), so the cells agree.  The baseline index is decoded
 // exactly in integers (the reference decodes it in float, which loses the diagonal
@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include "herk_common.h"
 #include "imaging.h"
 
 namespace ftdx {
@@ -74,30 +75,33 @@ pillbox_grid_kernel(const T* __restrict__ vis, const float* __restrict__ uv_m,
     const int64_t plane = (int64_t)Ng * Ng;
     const float half_ng = 0.5f * Ng;
     const int64_t stride = (int64_t)gridDim.x * IM_THREADS;
-    for (int64_t i = (int64_t)blockIdx.x * IM_THREADS + threadIdx.x; i < total; i += stride) {
-        const int64_t f = i / n_bl, k = i - f * n_bl;
-        int row, col;
-        tri_row_col(k, row, col);
-        const float vre = to_f(vis[2 * i]), vim = to_f(vis[2 * i + 1]);
-        const double lambda = C_LIGHT / freq_hz[freq_offset + f];
-        const float u_lam = (float)((double)uv_m[2 * k] / lambda);
-        const float v_lam = (float)((double)uv_m[2 * k + 1] / lambda);
-        const int iu = (int)roundf(u_lam / cell + half_ng);
-        const int iv = (int)roundf(v_lam / cell + half_ng);
-        if (iu >= 0 && iu < Ng && iv >= 0 && iv < Ng) {
-            float* g = grid + 2 * (f * plane + (int64_t)iv * Ng + iu);
-            unsafeAtomicAdd(g, vre);
-            unsafeAtomicAdd(g + 1, vim);
-        }
-        if (row != col) {
-            const int iuc = (int)roundf(-u_lam / cell + half_ng);
-            const int ivc = (int)roundf(-v_lam / cell + half_ng);
-            if (iuc >= 0 && iuc < Ng && ivc >= 0 && ivc < Ng) {
-                float* g = grid + 2 * (f * plane + (int64_t)ivc * Ng + iuc);
-                unsafeAtomicAdd(g, vre);
-                unsafeAtomicAdd(g + 1, -vim);
+    auto cell_of = [&](float u, float v) -> int64_t {
+        const int iu = (int)roundf(u / cell + half_ng), iv = (int)roundf(v / cell + half_ng);
+        return iu >= 0 && iu < Ng && iv >= 0 && iv < Ng ? (int64_t)iv * Ng + iu : -1;
+    };
+    // whole waves per pass: grid_add exchanges values between lanes
+    for (int64_t i0 = (int64_t)blockIdx.x * IM_THREADS; i0 < total; i0 += stride) {
+        const int64_t i = i0 + threadIdx.x;
+        float vre = 0.0f, vim = 0.0f;
+        int64_t at = -1, conj = -1;  // cells of all channels' planes as one grid
+        if (i < total) {
+            const int64_t f = i / n_bl, k = i - f * n_bl;
+            int row, col;
+            tri_row_col(k, row, col);
+            vre = to_f(vis[2 * i]);
+            vim = to_f(vis[2 * i + 1]);
+            const double lambda = C_LIGHT / freq_hz[freq_offset + f];
+            const float u_lam = (float)((double)uv_m[2 * k] / lambda);
+            const float v_lam = (float)((double)uv_m[2 * k + 1] / lambda);
+            at = cell_of(u_lam, v_lam);
+            if (at >= 0) at += f * plane;
+            if (row != col) {
+                conj = cell_of(-u_lam, -v_lam);
+                if (conj >= 0) conj += f * plane;
             }
         }
+        grid_add(grid, at, vre, vim);
+        grid_add(grid, conj, vre, -vim);
     }
 }
 

@@ -187,6 +187,32 @@ def test_fused_herk_pol_grid_bit_exact(oracle, dev, N, K, n_ch, n_pol, cfg):
     assert np.array_equal(_bits(unfused.cpu().numpy()), _bits(ref))
 
 
+@pytest.mark.parametrize("N", [1, 2, 3, 11, 23])
+def test_gridding_of_partial_waves(oracle, dev, N):
+    """Baseline counts that fill no wave (1, 3, 6, 66, 276): the gridding kernels pair lanes
+    to add a cell's two components, so lanes past the last baseline, off-grid cells and
+    autocorrelations must leave their partner's cell alone.  Integer sums: bit-exact."""
+    import torch
+    from ftd_amd import ftdx
+    K, n_ch, n_pol, Ng, cell = 48, 2, 2, 33, 2e-3
+    qc = oracle.gen_qc_uniform(N, N * K * n_ch * n_pol)
+    rng = np.random.default_rng(N)
+    uv = (rng.standard_normal((N * (N + 1) // 2, 2)) * 0.02).astype(np.float32)
+    uv[::2] *= 3.0  # every other baseline near or past the edge of the grid
+    freqs = np.array([0.8e9, 1.3e9])
+    ref = _grid_ref(oracle, qc, N, K, n_ch, n_pol, uv, freqs, Ng, cell, 0, 1.0)
+    g = ftdx.CutlassComplexGemm()
+    A, uv_d, f_d = (torch.from_numpy(x).to(dev) for x in (qc, uv, freqs))
+    fused = torch.zeros((n_ch, Ng, Ng, 2), dtype=torch.float32, device=dev)
+    ftdx.herk_pol_grid(g, A, N, K, n_ch, n_pol, uv_d, f_d, fused, Ng, cell)
+    tri = ftdx.herk_pol_reduce(g, A, N, K, n_ch, n_pol, 1)
+    unfused = torch.zeros_like(fused)
+    ftdx.pillbox_grid(tri, uv_d, f_d, unfused, N * (N + 1) // 2, Ng, n_ch, cell)
+    torch.cuda.synchronize()
+    assert np.array_equal(fused.cpu().numpy(), ref)
+    assert np.array_equal(unfused.cpu().numpy(), ref)
+
+
 def test_fused_herk_pol_grid_accumulates_and_validates(oracle, dev):
     """The grid is accumulated into (two calls give twice the values) and bad arguments
     are rejected before any launch."""
