@@ -20,6 +20,8 @@
 #include "ftdx_tune.h"
 #include "herk_fp8.h"
 #include "herk_mx.h"
+#include "herk_direct.h"
+#include "herk_pipe.h"
 #include "calib.h"
 #include "stages.h"
 #include "imaging.h"
@@ -51,6 +53,16 @@ struct ftdx_context {
     // pre-cast FP8 operand rows for the unfused / FP16-input paths
     uint8_t* precast = nullptr;
     size_t precast_cap = 0;
+    // fragment rows of the pipelined HERK, one buffer per stream that called it (calls on
+    // different streams may overlap, as the fused tile needs no scratch); a fifth stream
+    // takes the fused tile
+    struct FragScratch {
+        bool used = false;
+        void* stream = nullptr;
+        uint8_t* rows = nullptr;
+        size_t cap = 0;
+    };
+    FragScratch frag[4];
     // plain-path graph replay (set_direct_herk_graph): small LRU of captured calls
     struct GraphEntry {
         bool used = false;
@@ -193,10 +205,8 @@ int precast_chunk_cap(int N, int K, int batch) {
 
 // units_out: output batches per unit of `batch` (a unit is one group of polarization
 // segments on the polarization-sum path)
-int pick_chunk(int cfg, int N, int batch, int cmax, int units_out = 1) {
+int pick_chunk_of(int64_t slots, int64_t tiles, int batch, int cmax) {
     if (cmax >= batch) return std::max(batch, 1);
-    const int64_t slots = (int64_t)std::max(device_cu_count(), 1) * tile_config_wg_per_cu(cfg);
-    const int64_t tiles = herk_tiles(cfg, N) * units_out;
     double best = 1e30;
     int pick = cmax;
     for (int c = cmax; c >= 1; --c) {
@@ -212,6 +222,11 @@ int pick_chunk(int cfg, int N, int batch, int cmax, int units_out = 1) {
         }
     }
     return pick;
+}
+
+int pick_chunk(int cfg, int N, int batch, int cmax, int units_out = 1) {
+    const int64_t slots = (int64_t)std::max(device_cu_count(), 1) * tile_config_wg_per_cu(cfg);
+    return pick_chunk_of(slots, (int64_t)herk_tiles(cfg, N) * units_out, batch, cmax);
 }
 
 // The pre-cast path of one call: per chunk of batches, convert A's rows into the
@@ -319,6 +334,112 @@ hipError_t run_padded(ftdx_context* ctx, const HerkPlainArgs& a, int cfg, int ou
     return hipSuccess;
 }
 
+// ---- pipelined HERK over E3M2 fragment rows (herk_pipe.h) ----
+// Chunks of batches as on the pre-cast paths, for the same reason; at most 160 MB, so that a
+// chunk's rows and its output share the 256 MB memory-side cache and the next chunk's rows
+// overwrite them there (headline 4.13 ms; 320 MB 4.23, 96 MB 4.21, 48 MB 4.58; 1024 inputs x
+// 286, K = 2048: 1.02 against 1.12 ms for 320 MB).
+constexpr size_t kFragChunkBytes = size_t(160) << 20;
+
+int frag_chunk_cap(int N, int K, int nseg, int batch) {
+    const size_t per = (size_t)frag_rows_bytes(N, K, nseg);
+    const int cap = (int)std::max<size_t>(1, std::min<size_t>(kFragChunkBytes / per, (size_t)std::max(batch, 1)));
+    return std::min(cap, 65535 / std::max(nseg, 1));
+}
+
+size_t frag_scratch_bytes(const HerkPlainArgs& a) {
+    const int grp = std::max(a.seg_group, 1);
+    return (size_t)frag_rows_bytes(a.N, a.K, a.nseg) * grp * frag_chunk_cap(a.N, a.K, a.nseg * grp, a.batch / grp);
+}
+
+// Fragment-row scratch of this stream, or NULL where the call has to do without: under
+// capture (a captured call must not depend on a buffer that a later call may replace), with
+// four other streams holding theirs, or when memory is short.
+uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    ftdx_context::FragScratch* slot = nullptr;
+    for (auto& f : ctx->frag)
+        if (f.used && f.stream == s) slot = &f;
+    for (auto& f : ctx->frag)
+        if (!slot && !f.used) slot = &f;
+    if (!slot) return nullptr;
+    if (slot->cap < need) {
+        if (slot->rows) {
+            if (hipDeviceSynchronize() != hipSuccess) return nullptr;
+            (void)hipFree(slot->rows);
+        }
+        *slot = ftdx_context::FragScratch();
+        if (hipMalloc(&slot->rows, need) != hipSuccess) {
+            (void)hipGetLastError();
+            slot->rows = nullptr;
+            return nullptr;
+        }
+        slot->cap = need;
+    }
+    slot->used = true;
+    slot->stream = s;
+    return slot->rows;
+}
+
+// Converts and multiplies chunk by chunk; a.A holds QC rows, `rows` frag_scratch_bytes(a).
+hipError_t run_pipe(uint8_t* rows, const HerkPlainArgs& a, bool fp16, hipStream_t st) {
+    const int grp = std::max(a.seg_group, 1), in_per = a.nseg * grp, units = a.batch / grp;
+    const int64_t slots = (int64_t)std::max(device_cu_count(), 1) * pipe_wg_per_cu();
+    const int chunk = pick_chunk_of(slots, (int64_t)pipe_tiles(a.N) * grp, units, frag_chunk_cap(a.N, a.K, in_per, units));
+    for (int u0 = 0; u0 < units; u0 += chunk) {
+        const int nu = std::min(chunk, units - u0);
+        hipError_t e = launch_qc_frag_rows(a.A + (int64_t)u0 * in_per * a.a_bstride, rows, a.N, a.K, nu * in_per,
+                                           a.nseg, grp, st);
+        if (e != hipSuccess) return e;
+        HerkPlainArgs b = a;
+        b.A = rows;
+        b.C = static_cast<uint8_t*>(a.C) + (int64_t)u0 * grp * a.c_bstride * (fp16 ? 2 : 4);
+        b.batch = nu * grp;
+        b.a_bstride = frag_rows_bytes(a.N, a.K, a.nseg);
+        if ((e = launch_herk_pipe(b, fp16, st)) != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+// Whether the direct kernel can be the fastest: up to a few rounds of its workgroups.
+bool worth_direct(int N, int K, int batch) {
+    return direct_supported(N, K, batch) && (int64_t)direct_tiles(N) * batch <= 8192;
+}
+
+// The kernel of an INT4 call that nobody tuned or forced: the direct one, the pipelined one, or
+// the fused 128 x 128 tile, by estimates in microseconds.  Each kernel is its launches, then the
+// longest of one workgroup's chain of 64-sample stages, all workgroups' stages over the chip's
+// 512 workgroup slots, and the output at the rate it stores (faster while it fits the memory-side cache);
+// the conversion and padding passes move their bytes at 5 TB/s.  The constants are fits to (us: direct / pipelined / fused)
+//   128 x 20, K 1024:   7.8 /  18 /  21     512 x 5,  K 4000:   30 / 47 / 59
+//   2000 x 1, K 1024:    20 /  20 /  21     2000 x 1, K 4000:   89 / 45 / 60
+//   512 x 20, K 1024:     - /  29 /  22     512 x 1144, K 1024:  - / 824 / 744
+//   1024 x 286, K 2048:   - / 1022 / 1098   2624 x 43, K 128:    - / 295 / 320
+//   4096 x 96, K 2048:    - / 4134 / 5460
+// Rows that 16-byte loads cannot take cost the fused tile a padding pass.
+int choose_kernel(const void* A, int N, int K, int batch, bool fp16) {
+    const double st = (K + 63) / 64, t128 = (double)pipe_tiles(N) * batch, in = (double)N * K * batch;
+    const double out = (double)N * (N + 1) / 2 * (fp16 ? 4.0 : 8.0) * batch;
+    double best = 5.0 + std::max({0.87 * st + 3.0, t128 / 512.0 * (1.55 * st + 6.0), out / 3.6e6});
+    if (!rows_take_vector_loads(A, K)) best += 4.0 + in * 2.0 / 5e6;
+    int pick = TILE_128x128_K64_P2;
+    if (pipe_supported(N, K)) {
+        const double t = 8.0 + in * 2.5 / 5e6 +
+                         std::max({0.45 * st + 3.0, t128 / 512.0 * (0.92 * st + 5.7), out / (out < 2e8 ? 5.5e6 : 4.1e6)});
+        if (t < best) {
+            best = t;
+            pick = TILE_PIPE;
+        }
+    }
+    if (worth_direct(N, K, batch) && 4.0 + std::max(0.68e-3 * direct_tiles(N) * batch * st, out / 2.8e6) < best)
+        pick = TILE_DIRECT;
+    return pick;
+}
+
 // Times every (tile configuration, workgroup order) on this call's buffers and
 // stores the fastest (cutlass_interface/strategy_cache.hpp:504-800: warm-up, then
 // event-timed repeats, failures skipped).  With beta != 0 the timing runs use a
@@ -326,7 +447,7 @@ hipError_t run_padded(ftdx_context* ctx, const HerkPlainArgs& a, int cfg, int ou
 // flag = TILE_BF6: the E3M2 variants, each timed with its conversion pass into the
 // context's pre-cast rows (already sized by the caller).
 int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStream_t s,
-             const TuneKey& key, TuneEntry& best, int flag) {
+             const TuneKey& key, TuneEntry& best, int flag, const HerkPlainArgs* qc_args, uint8_t* frag) {
     HerkPlainArgs a = a0;
     void* scratch = nullptr;
     hipError_t e;
@@ -346,6 +467,11 @@ int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStrea
     (void)hipEventCreate(&t0);
     (void)hipEventCreate(&t1);
     auto launch = [&](int cfg, int remap) -> hipError_t {
+        if (cfg == TILE_PIPE || cfg == TILE_DIRECT) {  // these take the call's own rows
+            HerkPlainArgs b = *qc_args;
+            b.C = a.C;
+            return cfg == TILE_PIPE ? run_pipe(frag, b, out_fp16, s) : launch_herk_direct(b, out_fp16, s);
+        }
         if (!(cfg & TILE_BF6)) return launch_herk_int4_plain(a, cfg, out_fp16, remap, s);
         return run_precast(ctx, a, FTDX_INPUT_INT4, true, tile_base(cfg), out_fp16, remap, s);
     };
@@ -382,6 +508,13 @@ int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStrea
                 std::printf("ftdx tune:   %-16s xcd_remap=%d  %.4f ms\n", tile_config_name(cfg), remap, ms);
             cands.push_back({cfg, remap, ms});
         }
+    for (int cfg : {TILE_PIPE, TILE_DIRECT}) {
+        if (!qc_args || (cfg == TILE_PIPE && !frag) ||
+            (cfg == TILE_DIRECT && !worth_direct(a.N, qc_args->K, qc_args->batch)) || time_cand(cfg, 1, 1) < 0.0f)
+            continue;
+        const float ms = time_cand(cfg, 1, 3);
+        if (ms >= 0.0f) cands.push_back({cfg, 1, ms});
+    }
     best.ms = 1e30f;
     best.cfg = kDefaultCfg | flag;
     best.xcd_remap = kDefaultRemap;
@@ -682,7 +815,6 @@ int ftdx_herk_query_config(ftdx_context* ctx, int N, int K, int batch_count, int
 }
 
 int ftdx_init_herk(ftdx_context* ctx, int N, int K, int batch_count, void* stream) {
-    (void)stream;
     if (!ctx) return fail(FTDX_ERR_INVALID_ARG, "ftdx_init_herk: NULL context");
     if (N < 0 || K < 0 || batch_count < 0)
         return fail(FTDX_ERR_INVALID_ARG, "ftdx_init_herk: negative size");
@@ -707,6 +839,16 @@ int ftdx_init_herk(ftdx_context* ctx, int N, int K, int batch_count, void* strea
         int rc = ftdx::grow_precast(ctx, need, "ftdx_init_herk: scratch");
         if (rc != FTDX_OK) return rc;
     }
+    // fragment rows of the pipelined path, for calls on this stream (which do without when
+    // there is no memory for them)
+    if (ctx->device >= 0 && ctx->herk_mode == FTDX_HERK_AUTO && ctx->forced_cfg < 0 &&
+        ctx->direct_tile == FTDX_DIRECT_TILE_AUTO && batch_count > 0 && ftdx::pipe_supported(N, K)) {
+        ftdx::HerkPlainArgs a{};
+        a.N = N;
+        a.K = K;
+        a.batch = batch_count;
+        (void)ftdx::frag_scratch(ctx, ftdx::frag_scratch_bytes(a), static_cast<hipStream_t>(stream));
+    }
     return FTDX_OK;
 }
 
@@ -715,9 +857,15 @@ int ftdx_end_herk(ftdx_context* ctx) {
     ctx->init_N = ctx->init_K = ctx->init_batch = 0;
     bool any_graph = false;
     for (auto& gph : ctx->graphs) any_graph = any_graph || gph.used;
-    if (ctx->mx_codes || ctx->cal_part || ctx->cal_herm || ctx->precast ||
+    bool any_frag = false;
+    for (auto& f : ctx->frag) any_frag = any_frag || f.rows;
+    if (ctx->mx_codes || ctx->cal_part || ctx->cal_herm || ctx->precast || any_frag ||
         any_graph) {
         (void)hipDeviceSynchronize();
+        for (auto& f : ctx->frag) {
+            if (f.rows) (void)hipFree(f.rows);
+            f = ftdx_context::FragScratch();
+        }
         if (ctx->mx_codes) (void)hipFree(ctx->mx_codes);
         if (ctx->cal_part) (void)hipFree(ctx->cal_part);
         if (ctx->cal_herm) (void)hipFree(ctx->cal_herm);
@@ -998,22 +1146,30 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
     bool cached;
     ftdx::pick_config(ctx, key, cfg, remap, cached);
     const bool explicit_cfg = ctx->forced_cfg >= 0 || ctx->direct_tile != FTDX_DIRECT_TILE_AUTO;
+    // INT4 calls without an explicit tile or mode may take the pipelined or the direct kernel:
+    // where the tuning cache says so, or untuned by choose_kernel
+    const bool may_route = !e3m2 && !precast && !explicit_cfg && ctx->herk_mode == FTDX_HERK_AUTO;
+    const bool may_pipe = may_route && ftdx::pipe_supported(N, K);
+    const bool tune_now = tune && !cached && !explicit_cfg && !precast;
+    if (may_route && !cached) cfg = ftdx::choose_kernel(A, N, K, batch_count, fp16);
+    uint8_t* frag = nullptr;
+    if (may_pipe && (cfg == ftdx::TILE_PIPE || tune_now))
+        frag = ftdx::frag_scratch(ctx, ftdx::frag_scratch_bytes(a), s);
+    if ((cfg == ftdx::TILE_PIPE && !frag) ||
+        (cfg == ftdx::TILE_DIRECT && !(may_route && ftdx::direct_supported(N, K, batch_count))))
+        cfg = ftdx::TILE_128x128_K64_P2;
     const int Kp = ftdx::precast_row_samples(K);
     const size_t rows_need = (size_t)N * ftdx::precast_chunk_cap(N, K, batch_count) * 2 * Kp;
-    if (precast) {
-        int rc = ftdx::grow_precast(ctx, rows_need, "ftdx_herk: scratch");
-        if (rc != FTDX_OK) return rc;
-    }
-    if (e3m2) {
+    if (precast || e3m2) {
         int rc = ftdx::grow_precast(ctx, rows_need, "ftdx_herk: scratch");
         if (rc != FTDX_OK) return rc;
     }
     const size_t pad_need = (size_t)N * ftdx::padded_chunk_cap(N, K, batch_count) * ftdx::padded_row_cap(K);
-    if (padded) {
+    if (padded && ((cfg != ftdx::TILE_PIPE && cfg != ftdx::TILE_DIRECT) || tune_now)) {
         int rc = ftdx::grow_precast(ctx, pad_need, "ftdx_herk: scratch");
         if (rc != FTDX_OK) return rc;
     }
-    if (tune && !cached && !explicit_cfg && !precast) {
+    if (tune_now) {
         ftdx::TuneEntry best;
         ftdx::HerkPlainArgs t = a;
         if (padded) {
@@ -1026,11 +1182,14 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
             t.K = Kt;
             t.a_bstride = (int64_t)N * Kt;
         }
-        if (ftdx::autotune(ctx, t, fp16, s, key, best, e3m2 ? ftdx::TILE_BF6 : 0) == FTDX_OK) {
+        ftdx::HerkPlainArgs tp = a;
+        tp.batch = t.batch;
+        if (ftdx::autotune(ctx, t, fp16, s, key, best, e3m2 ? ftdx::TILE_BF6 : 0, may_route ? &tp : nullptr, frag) == FTDX_OK) {
             cfg = best.cfg;
             if (ctx->forced_remap < 0) remap = best.xcd_remap;
         }
     }
+    const bool pipe = cfg == ftdx::TILE_PIPE, direct = cfg == ftdx::TILE_DIRECT;
     // E3M2 operand tiles: FP6 compute on INT4 input, or an INT4 FP8 call whose tile
     // configuration carries the FTDX_TILE_BF6 flag (explicit choice or cache entry)
     const bool bf6 = e3m2 || (!precast && (cfg & ftdx::TILE_BF6));
@@ -1040,6 +1199,8 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
         if (rc != FTDX_OK) return rc;
     }
     auto run = [&](hipStream_t st) -> hipError_t {
+        if (pipe) return ftdx::run_pipe(frag, a, fp16, st);
+        if (direct) return ftdx::launch_herk_direct(a, fp16, st);
         if (precast || bf6) return ftdx::run_precast(ctx, a, input, bf6, cfg, fp16, remap, st);
         if (padded)
             return ftdx::run_padded(ctx, a, cfg, fp16 ? 2 : 4, st, [&](const ftdx::HerkPlainArgs& b) {

@@ -20,6 +20,8 @@ const char* tile_config_name(int cfg) {
          "t256x128_k64_p2"},
         {"t128x128_k64_bf6", "t128x128_k128_bf6", "t64x64_k64_bf6", "t256x128_k64_bf6",
          "t128x128_k64_p2_bf6", "t256x128_k64_p2_bf6"}};
+    if (cfg == TILE_PIPE) return "pipe_e3m2";
+    if (cfg == TILE_DIRECT) return "direct32";
     if (!valid_tile_config(cfg)) return "unknown";
     return names[(cfg & TILE_BF6) ? 1 : 0][tile_base(cfg)];
 }

@@ -65,7 +65,7 @@ int TuneCache::load(const std::string& path, int* skipped) {
         TuneEntry e{};
         if (!(ss >> kind >> k.N >> k.K >> k.batch >> k.out_fp16 >> k.vec >> e.cfg >> e.xcd_remap >>
               e.ms) ||
-            kind != "herk" || !valid_tile_config(e.cfg) || k.N < 0 || k.K < 0 ||
+            kind != "herk" || !valid_tuned_config(e.cfg) || k.N < 0 || k.K < 0 ||
             k.batch < 0) {
             ++bad;
             continue;

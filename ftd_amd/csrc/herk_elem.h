@@ -1,0 +1,67 @@
+// herk_elem.h -- output elements and QC row loads shared by the pipelined and the direct HERK.
+#pragma once
+#include "herk_common.h"
+
+namespace ftdx {
+
+template <typename OutT>
+struct Elem;  // one complex output element
+template <>
+struct Elem<float> {
+    typedef float v2 __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ v2 make(float r, float i) {
+        v2 v;
+        v[0] = r;
+        v[1] = i;
+        return v;
+    }
+};
+template <>
+struct Elem<_Float16> {
+    typedef _Float16 v2 __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ v2 make(float r, float i) {
+        v2 v;
+        v[0] = (_Float16)r;
+        v[1] = (_Float16)i;
+        return v;
+    }
+};
+
+// C = alpha * (r, i) + beta * C for one element: alpha first, then fma(beta, old, .), one
+// rounding each, as the other HERK kernels.
+template <typename OutT>
+__device__ __forceinline__ void put_element(typename Elem<OutT>::v2* c, float r, float i, float alpha, float beta) {
+    r *= alpha;
+    i *= alpha;
+    if (beta != 0.0f) {
+        const typename Elem<OutT>::v2 old = *c;
+        r = __builtin_fmaf(beta, (float)old[0], r);
+        i = __builtin_fmaf(beta, (float)old[1], i);
+    }
+    *c = Elem<OutT>::make(r, i);
+}
+
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+
+// Samples k .. k + 15 of a row of K >= 16 samples at any address; zeros past K.  A segment that
+// crosses the row's end is taken from its last 16 bytes and shifted down, so nothing past the
+// row is read.
+__device__ __forceinline__ uint4 row_segment(const uint8_t* row, int k, int K) {
+    const int over = k + 16 - K;
+    if (over >= 16) return make_uint4(0u, 0u, 0u, 0u);
+    const u32x4_any v = *reinterpret_cast<const u32x4_any*>(row + (over > 0 ? K - 16 : k));
+    uint64_t lo = ((uint64_t)v[1] << 32) | v[0], hi = ((uint64_t)v[3] << 32) | v[2];
+    if (over > 0) {
+        const int s = over * 8;
+        if (s >= 64) {
+            lo = hi >> (s - 64);
+            hi = 0;
+        } else {
+            lo = (lo >> s) | (hi << (64 - s));
+            hi >>= s;
+        }
+    }
+    return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
+
+}  // namespace ftdx

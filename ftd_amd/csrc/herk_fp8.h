@@ -23,7 +23,12 @@ enum TileConfigId {
 constexpr int TILE_BF6 = 16;
 inline bool valid_tile_config(int c) { return c >= 0 && (c & ~TILE_BF6) < NUM_TILE_CONFIGS; }
 inline int tile_base(int c) { return c & ~TILE_BF6; }
-
+// Not tiles of this family: the pipelined HERK over E3M2 fragment rows (herk_pipe.h) and the
+// direct HERK for small problems (herk_direct.h), which ftdx_herk takes by its own rule or because
+// the autotuner found them fastest.  Stored in tuning caches, not accepted as explicit settings.
+constexpr int TILE_PIPE = 64;
+constexpr int TILE_DIRECT = 65;
+inline bool valid_tuned_config(int c) { return valid_tile_config(c) || c == TILE_PIPE || c == TILE_DIRECT; }
 
 const char* tile_config_name(int cfg);
 int tile_config_rows(int cfg);   // TM

@@ -1,0 +1,42 @@
+// herk_pipe.h -- host-side launch interface of the pipelined HERK (internal).
+//
+// The HERK of QC voltages over E3M2 fragment rows: every QC value is exact in E3M2, and
+// the matrix cores take 6-bit operands at twice the FP8 rate.  Layout of the rows of one
+// batch: [group of 32 rows][step of 32 samples][1536 bytes], the operand of one 32x32x64
+// MFMA in lane order.  Lane l holds row l % 32, samples 16 (l / 32) .. + 15 of the step: 16
+// six-bit Re codes then 16 Im codes (code k at bits 6k), six dwords, the first four of all
+// lanes at 16 l, the last two at 1024 + 8 l.  So a wave copies whole kilobytes from memory
+// to LDS and reads its operands from there without bank conflicts, 48 bytes per 32 samples.
+// Rows past N and samples past K are zero.
+#pragma once
+#include "herk_fp8.h"
+
+namespace ftdx {
+
+constexpr int kFragBytes = 1536;
+
+// 32-sample steps of a row of K samples (whole 64-sample stages).
+inline int frag_steps(int K) { return (K + 63) / 64 * 2; }
+// Bytes of one batch's fragment rows (nseg segments of K samples per row).
+inline int64_t frag_rows_bytes(int N, int K, int nseg = 1) {
+    return (int64_t)((N + 31) / 32) * frag_steps(K) * nseg * kFragBytes;
+}
+
+// Whether the pipelined HERK takes this problem: 16-byte row loads (K >= 16) and one
+// batch's fragment rows within a 32-bit buffer offset.
+bool pipe_supported(int N, int K, int nseg = 1);
+
+// QC rows [batches][N][K] (any K >= 16, any alignment) -> fragment rows.  Input batch
+// (ob * nseg + s) * seg_group + i becomes segment s of output batch ob * seg_group + i.
+hipError_t launch_qc_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, int batches, int nseg, int seg_group,
+                               hipStream_t stream);
+
+// The HERK over fragment rows: a.A the rows, a.a_bstride their bytes per batch, a.K the
+// samples of one segment (a.nseg of them); packed lower triangle as launch_herk_int4_plain.
+hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t stream);
+
+// Tiles per batch and resident workgroups per CU of the launch above.
+int pipe_tiles(int N);
+int pipe_wg_per_cu();
+
+}  // namespace ftdx

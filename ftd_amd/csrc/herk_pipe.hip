@@ -1,0 +1,427 @@
+// herk_pipe.hip -- HERK of QC voltages on E3M2 MFMA over fragment rows (layout: herk_pipe.h).
+//
+// What bounds it: at 4096 x 96, K = 2048 the matrix cores are busy about 60% of the cycles, and
+// under that load the chip runs at 1.5 - 1.9 instead of 2.4 GHz: the time is the energy of the
+// MFMAs, then of the operand traffic.  So the operands are the smallest exact ones (6 bits,
+// half the MFMA time of FP8 and 0.75 of its bytes), tiles go in square blocks that one XCD's L2
+// serves, and the loop keeps both pipes fed:
+//   * 128 x 128 tile, 4 waves of 64 x 64, two workgroups per CU, so that one workgroup's
+//     stores overlap the other's MFMAs (256 x 128 with one per CU: 4.39 against 4.25 ms);
+//   * stages of 64 samples in three LDS buffers, copied by buffer_load ... lds.  (The
+//     global_load form is a FLAT instruction to the compiler, which then waits for every
+//     outstanding LDS and memory operation at the next use of either.)
+//   * operands one 32-sample step ahead in a second register set, across the barrier too: a
+//     stage's first step is read during the previous stage, whose barrier already published
+//     it, so no MFMA waits for an LDS read that was not issued a step earlier.
+// Stores go to the packed rows straight from the accumulators: 32-lane runs, plain (not
+// non-temporal) so that the L2 joins the partial lines of neighbouring runs (1664 inputs x
+// 128, K = 128: 303 against 478 us; 64-byte write requests within 1% of the output bytes).
+#include "herk_common.h"
+#include "herk_elem.h"
+#include "herk_pipe.h"
+
+namespace ftdx {
+
+namespace {
+
+constexpr int PT = 128;                      // tile rows and columns
+constexpr int P_THREADS = 256;               // 4 waves, 2 x 2
+constexpr int P_GROUPS = 2 * PT / 32;        // row groups of a stage: 4 of the rows, 4 of the columns
+constexpr int P_GSTRIDE = 2 * kFragBytes + 16;  // LDS bytes per group and stage; not a multiple of
+                                             // 512, or the compiler pairs the 8-byte reads of two
+                                             // groups and copies the halves into place
+constexpr int P_STAGE = P_GROUPS * P_GSTRIDE;
+constexpr int P_BUFS = 3;
+constexpr int P_LOADS = P_GROUPS * 3 / 4;    // kilobyte copies per wave and stage
+constexpr int P_WG_PER_CU = 2;
+constexpr int P_BLOCK = 4;                   // tile order: blocks of 4 x 4 tiles
+static_assert(P_BUFS * P_STAGE * P_WG_PER_CU <= 160 * 1024, "LDS of the resident workgroups");
+
+typedef int v6i __attribute__((ext_vector_type(6)));
+typedef v6i Frags[2];
+
+__device__ __forceinline__ v8i op8(v6i a) { return __builtin_shufflevector(a, a, 0, 1, 2, 3, 4, 5, -1, -1); }
+
+// v = [im | -re] of u = [re | im]: the halves swapped, bit 5 of every Re code flipped
+__device__ __forceinline__ v6i conj6(v6i a) {
+    v6i r;
+    r[0] = a[3];
+    r[1] = a[4];
+    r[2] = a[5];
+    r[3] = a[0] ^ (int)0x20820820u;
+    r[4] = a[1] ^ (int)0x08208208u;
+    r[5] = a[2] ^ (int)0x82082082u;
+    return r;
+}
+
+template <int VM>
+__device__ __forceinline__ void wait_vm() {  // vmcnt(VM), other counters free
+    __builtin_amdgcn_s_waitcnt((VM & 0xF) | (0x7 << 4) | (0xF << 8) | (((VM >> 4) & 0x3) << 14));
+}
+
+template <int L>
+__device__ __forceinline__ void wait_lgkm() {  // lgkmcnt(L), other counters free
+    __builtin_amdgcn_s_waitcnt(0xF | (0x7 << 4) | (L << 8) | (3 << 14));
+}
+
+__device__ __forceinline__ void wg_barrier() {
+    __asm__ __volatile__("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ __volatile__("" ::: "memory");
+}
+
+// The operands of step ks (0, 1) of a stage: two groups at `a`, two at `b`.
+__device__ __forceinline__ void read_frags(const uint8_t* __restrict__ st, int a, int b, int lane, int ks, Frags& fa,
+                                           Frags& fb) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            const int off = (m ? b : a) + x * P_GSTRIDE + ks * kFragBytes;
+            const uint4 u = *reinterpret_cast<const uint4*>(st + off + lane * 16);
+            const uint2 v = *reinterpret_cast<const uint2*>(st + off + 1024 + lane * 8);
+            v6i& f = m ? fb[x] : fa[x];
+            f[0] = (int)u.x;
+            f[1] = (int)u.y;
+            f[2] = (int)u.z;
+            f[3] = (int)u.w;
+            f[4] = (int)v.x;
+            f[5] = (int)v.y;
+        }
+}
+
+// One step: 8 MFMAs.  The empty asm keeps each operand in six consecutive registers here.
+__device__ __forceinline__ void mfma_step(Frags& fa, Frags& fb, v16f (&re)[2][2], v16f (&im)[2][2]) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        __asm__ __volatile__("" : "+v"(fa[x]));
+        __asm__ __volatile__("" : "+v"(fb[x]));
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        const v6i v = conj6(fa[x]);
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+            re[x][y] = mfma_32x32x64<OPF_BF6>(op8(fa[x]), op8(fb[y]), re[x][y]);
+            im[x][y] = mfma_32x32x64<OPF_BF6>(op8(v), op8(fb[y]), im[x][y]);
+        }
+    }
+}
+
+// This wave's share of one stage: kilobyte q * 4 + wave of the stage's 24, three per group.
+__device__ __forceinline__ void copy_stage(__amdgpu_buffer_rsrc_t rows, int at, uint8_t* st, int wave,
+                                           const uint32_t (&off)[P_LOADS]) {
+#pragma unroll
+    for (int q = 0; q < P_LOADS; ++q) {
+        const int p = q * 4 + wave;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rows, (void __attribute__((address_space(3)))*)(st + (p / 3) * P_GSTRIDE + (p % 3) * 1024), 16, off[q], at,
+            0, 0);
+    }
+}
+
+// Stage s in `cur`: its second step's operands are read while the first step (f0, read a stage
+// ago) multiplies, the next stage's first step while the second one does.  The copies of
+// stage s + 2 go into `fre`, the buffer of stage s - 1, which every wave finished reading
+// before this stage's barrier.
+template <bool ACTIVE>
+__device__ __forceinline__ void stage_body(const uint8_t* __restrict__ cur, const uint8_t* __restrict__ nxt,
+                                           uint8_t* __restrict__ fre, __amdgpu_buffer_rsrc_t rows, int at,
+                                           const uint32_t (&off)[P_LOADS], int lane, int wave, int a, int b, Frags& a0,
+                                           Frags& b0, Frags& a1, Frags& b1, v16f (&re)[2][2], v16f (&im)[2][2]) {
+    copy_stage(rows, at, fre, wave, off);
+    if constexpr (ACTIVE) {
+        read_frags(cur, a, b, lane, 1, a1, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lgkm<8>();  // all but the eight reads just issued
+        mfma_step(a0, b0, re, im);
+        __builtin_amdgcn_sched_barrier(0);
+        read_frags(nxt, a, b, lane, 0, a0, b0);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lgkm<8>();
+        mfma_step(a1, b1, re, im);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+template <bool ACTIVE>
+__device__ __forceinline__ void tile_loop(__amdgpu_buffer_rsrc_t rows, uint8_t* lds, int nst,
+                                          const uint32_t (&off)[P_LOADS], int lane, int wave, int a, int b,
+                                          v16f (&re)[2][2], v16f (&im)[2][2]) {
+    constexpr int SRC = 2 * kFragBytes;  // bytes of one group and stage
+    copy_stage(rows, 0, lds, wave, off);
+    copy_stage(rows, nst > 1 ? SRC : 0, lds + P_STAGE, wave, off);
+    Frags a0, b0, a1, b1;
+    wait_vm<P_LOADS>();  // stage 0 landed
+    wg_barrier();
+    if constexpr (ACTIVE) read_frags(lds, a, b, lane, 0, a0, b0);
+    int c = 0;  // buffer of stage s
+    for (int s = 0; s < nst; ++s) {
+        wait_vm<0>();  // this wave's copies of stage s + 1
+        wg_barrier();
+        const int n = c == P_BUFS - 1 ? 0 : c + 1, f = c == 0 ? P_BUFS - 1 : c - 1;
+        // past the end the last stage is copied again, into a buffer that is not read
+        const int t = s + 2 < nst ? s + 2 : nst - 1;
+        stage_body<ACTIVE>(lds + c * P_STAGE, lds + n * P_STAGE, lds + f * P_STAGE, rows, t * SRC, off, lane, wave, a,
+                           b, a0, b0, a1, b1, re, im);
+        c = n;
+    }
+    wait_vm<0>();  // no copy may land after the workgroup's LDS is given back
+}
+
+// A block wholly below the diagonal and inside the matrix, beta = 0: no element is tested, and a
+// row's offset is the last row's plus a lane constant (row d of a block starting at row w lies
+// d w + d (d + 1) / 2 elements after row 0).  The general form below spends about 15 VALU
+// operations per element, 5 of them on 64-bit index arithmetic (K = 128, FP16 output: 214
+// against 269 us for the whole launch).
+template <typename OutT, bool SCALE, bool NT>
+__device__ __forceinline__ void store_inside(OutT* C, int w, int col, float alpha, const v16f (&re)[2][2],
+                                             const v16f (&im)[2][2], int lane) {
+    typedef typename Elem<OutT>::v2 v2;
+    constexpr uint32_t ES = sizeof(v2);
+    const int n = lane & 31, g4 = (lane >> 5) * 4;
+    uint8_t* base = reinterpret_cast<uint8_t*>(reinterpret_cast<v2*>(C) + tri_index(w, col));
+    uint32_t off = (uint32_t)(g4 * w + g4 * (g4 + 1) / 2 + n) * ES;
+    const uint32_t step = (uint32_t)(w + g4) * ES;  // row d + g4 -> d + 1 + g4 adds step + (d + 1) ES
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int d = x * 32 + (q >> 2) * 8 + (q & 3);
+            v2* p = reinterpret_cast<v2*>(base + off);
+#pragma unroll
+            for (int y = 0; y < 2; ++y) {
+                const v2 e = SCALE ? Elem<OutT>::make(re[x][y][q] * alpha, im[x][y][q] * alpha)
+                                  : Elem<OutT>::make(re[x][y][q], im[x][y][q]);
+                if constexpr (NT) __builtin_nontemporal_store(e, p + y * 32);
+                else p[y * 32] = e;
+            }
+            off += (q & 3) != 3 ? step + (uint32_t)(d + 1) * ES : 5 * step + (uint32_t)(5 * d + 15) * ES;
+        }
+}
+
+// Any block: elements (i, j <= i) with i < N; Im = 0 on the diagonal, then alpha, then
+// fma(beta, old, .), as the other HERK kernels.
+template <typename OutT>
+__device__ __forceinline__ void store_any(OutT* C, int N, int w, int col, float alpha, float beta,
+                                          const v16f (&re)[2][2], const v16f (&im)[2][2], int lane) {
+    typedef typename Elem<OutT>::v2 v2;
+    const int n = lane & 31, g4 = (lane >> 5) * 4;
+    v2* base = reinterpret_cast<v2*>(C);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int i = w + x * 32 + (q >> 2) * 8 + g4 + (q & 3);
+            v2* row = base + tri_index(i, 0);
+#pragma unroll
+            for (int y = 0; y < 2; ++y) {
+                const int j = col + y * 32 + n;
+                if (i < N && j <= i)
+                    put_element<OutT>(row + j, re[x][y][q], i == j ? 0.0f : im[x][y][q], alpha, beta);
+            }
+        }
+}
+
+// Tile t of the lower triangle of nb x nb tiles, in square blocks of H x H tiles (row-major
+// inside a block, blocks row-major): the tiles that one XCD runs together then share H row and
+// H column blocks in its L2 instead of one and many.
+__device__ __forceinline__ void tri_decode_blocked(int t, int nb, int H, int& I, int& J) {
+    const int full = H * H, diag = H * (H + 1) / 2;
+    // block row S starts at full S (S - 1) / 2 + diag S
+    const float a = 0.5f * full, b = diag - a;
+    int S = (int)((__builtin_sqrtf(b * b + 4.0f * a * (float)t) - b) / (2.0f * a));
+    while (S > 0 && full * S * (S - 1) / 2 + diag * S > t) --S;
+    while (full * (S + 1) * S / 2 + diag * (S + 1) <= t) ++S;
+    int u = t - (full * S * (S - 1) / 2 + diag * S);
+    const int h = nb - S * H < H ? nb - S * H : H;  // rows of this block row
+    if (u < h * H * S) {
+        const int SJ = u / (h * H), v = u - SJ * (h * H);
+        I = S * H + v / H;
+        J = SJ * H + v % H;
+    } else {
+        int i;
+        tri_decode(u - h * H * S, i, u);
+        I = S * H + i;
+        J = S * H + u;
+    }
+}
+
+template <typename OutT, bool NT>
+__global__ void __launch_bounds__(P_THREADS, 2) herk_pipe_kernel(HerkPlainArgs p, int steps, int tiles) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[P_BUFS * P_STAGE];
+    const int w = xcd_logical((int)blockIdx.x, tiles * p.batch);
+    const int b = w / tiles, t = w - b * tiles;
+    int I, J;
+    tri_decode_blocked(t, (p.N + PT - 1) / PT, P_BLOCK, I, J);
+    // wave index in an SGPR: the conditions on it are scalar branches
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int wrow = I * PT + wm * 64, wcol = J * PT + wn * 64;
+    const bool active = wrow < p.N && wrow + 63 >= wcol;
+    // groups past N (edge tiles) read the last group; their products are not stored
+    const int ng = (p.N + 31) / 32;
+    uint32_t off[P_LOADS];
+#pragma unroll
+    for (int q = 0; q < P_LOADS; ++q) {
+        const int k = q * 4 + wave, g = k / 3;
+        const int want = g < P_GROUPS / 2 ? I * (PT / 32) + g : J * (PT / 32) + g - P_GROUPS / 2;
+        off[q] = (uint32_t)(want < ng ? want : ng - 1) * (uint32_t)(steps * kFragBytes) + (uint32_t)((k % 3) * 1024 + lane * 16);
+    }
+    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(p.A) + (int64_t)b * p.a_bstride, 0, (int)((uint32_t)ng * (uint32_t)(steps * kFragBytes)),
+        0x00027000);
+    v16f re[2][2], im[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                re[x][y][r] = 0.0f;
+                im[x][y][r] = 0.0f;
+            }
+    const int a = wm * 2 * P_GSTRIDE, bo = (P_GROUPS / 2 + wn * 2) * P_GSTRIDE;
+    if (!active) {
+        tile_loop<false>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
+        return;
+    }
+    tile_loop<true>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
+    OutT* C = static_cast<OutT*>(p.C) + (int64_t)b * p.c_bstride;
+    if (wcol + 63 < wrow && wrow + 64 <= p.N && p.beta == 0.0f) {
+        if (p.alpha == 1.0f) store_inside<OutT, false, NT>(C, wrow, wcol, p.alpha, re, im, lane);
+        else store_inside<OutT, true, NT>(C, wrow, wcol, p.alpha, re, im, lane);
+    } else {
+        store_any<OutT>(C, p.N, wrow, wcol, p.alpha, p.beta, re, im, lane);
+    }
+}
+
+// ---- QC rows -> fragment rows ----
+// HBM-bound (1 byte read, 1.5 written per sample).  A thread converts 16 samples of one row; a
+// wave covers S segments x 64 / S rows, so it reads runs of 16 S bytes and writes runs of
+// 64 / S x 16 bytes.
+
+// 4 QC bytes -> E3M2 codes of their Re and Im nibbles, one per byte (bits 5:0)
+__device__ __forceinline__ void qc4_codes(uint32_t x, uint32_t& re, uint32_t& im) {
+    const uint32_t TLO = 0x12100C00u;  // e3m2(0..3)
+    const uint32_t THI = 0x17161514u;  // e3m2(4..7)
+    re = __builtin_amdgcn_perm(THI, TLO, (x >> 4) & 0x07070707u) | ((x >> 2) & 0x20202020u);
+    im = __builtin_amdgcn_perm(THI, TLO, x & 0x07070707u) | ((x << 2) & 0x20202020u);
+}
+
+__device__ __forceinline__ uint32_t pack4(uint32_t c) {  // four byte-wide codes -> 24 bits
+    return (c & 0x3Fu) | ((c >> 2) & 0xFC0u) | ((c >> 4) & 0x3F000u) | ((c >> 6) & 0xFC0000u);
+}
+
+__device__ __forceinline__ void pack16(const uint32_t (&c)[4], uint32_t& d0, uint32_t& d1, uint32_t& d2) {
+    const uint32_t p0 = pack4(c[0]), p1 = pack4(c[1]), p2 = pack4(c[2]), p3 = pack4(c[3]);
+    d0 = p0 | (p1 << 24);
+    d1 = (p1 >> 8) | (p2 << 16);
+    d2 = (p2 >> 16) | (p3 << 8);
+}
+
+// VEC: K % 16 == 0 and 16-byte aligned rows
+template <bool VEC, int S>
+__global__ void __launch_bounds__(256)
+qc_frag_rows_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int N, int K, int steps, int nseg,
+                    int grp) {
+    constexpr int R = 64 / S;
+    const int ng = (N + 31) / 32, segs = steps * 2;
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x, v = t / 64u;
+    const uint32_t sb = v % (uint32_t)(segs / S), rb = v / (uint32_t)(segs / S);
+    const int s = (int)sb * S + (int)(t % S), r = (int)rb * R + (int)(t / S % R);
+    if (r >= ng * 32) return;
+    const int ib = (int)blockIdx.y, ob = ib / (nseg * grp), sg = ib / grp - ob * nseg;
+    const int64_t dst_batch = (int64_t)ob * grp + ib % grp;
+    uint4 w = make_uint4(0u, 0u, 0u, 0u);
+    if (r < N) {
+        const uint8_t* row = in + ((int64_t)ib * N + r) * K;
+        if constexpr (VEC) {
+            if (s * 16 < K) w = *reinterpret_cast<const uint4*>(row + s * 16);
+        } else {
+            w = row_segment(row, s * 16, K);
+        }
+    }
+    uint32_t re[4], im[4];
+    qc4_codes(w.x, re[0], im[0]);
+    qc4_codes(w.y, re[1], im[1]);
+    qc4_codes(w.z, re[2], im[2]);
+    qc4_codes(w.w, re[3], im[3]);
+    uint4 a;
+    uint2 b;
+    pack16(re, a.x, a.y, a.z);
+    pack16(im, a.w, b.x, b.y);
+    const int lane = (r & 31) + 32 * (s & 1);
+    uint8_t* dst = out + ((dst_batch * ng + (r >> 5)) * (int64_t)(steps * nseg) + sg * steps + (s >> 1)) * kFragBytes;
+    *reinterpret_cast<uint4*>(dst + lane * 16) = a;
+    *reinterpret_cast<uint2*>(dst + 1024 + lane * 8) = b;
+}
+
+}  // namespace
+
+bool pipe_supported(int N, int K, int nseg) {
+    return N > 0 && K >= 16 && nseg >= 1 && (int64_t)K * nseg <= 0x7FFFFFFF - 64 * (int64_t)nseg &&
+           frag_rows_bytes(N, K, nseg) <= 0x7FFFFFFFll;
+}
+
+int pipe_tiles(int N) {
+    const int nb = (N + PT - 1) / PT;
+    return nb * (nb + 1) / 2;
+}
+
+int pipe_wg_per_cu() { return P_WG_PER_CU; }
+
+hipError_t launch_qc_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, int batches, int nseg, int seg_group,
+                               hipStream_t stream) {
+    if (N <= 0 || batches <= 0) return hipSuccess;
+    if (!pipe_supported(N, K, nseg) || batches > 65535) return hipErrorInvalidValue;
+    const int steps = frag_steps(K), segs = steps * 2, rows = (N + 31) / 32 * 32;
+    const bool vec = K % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
+    const dim3 grid((unsigned)(((int64_t)rows * segs + 255) / 256), (unsigned)batches), block(256);
+    // 8 segments per wave where a row's segments allow it (whole stages have 4)
+    if (segs % 8 == 0) {
+        if (vec)
+            hipLaunchKernelGGL((qc_frag_rows_kernel<true, 8>), grid, block, 0, stream, in, out, N, K, steps, nseg,
+                               seg_group);
+        else
+            hipLaunchKernelGGL((qc_frag_rows_kernel<false, 8>), grid, block, 0, stream, in, out, N, K, steps, nseg,
+                               seg_group);
+    } else {
+        if (vec)
+            hipLaunchKernelGGL((qc_frag_rows_kernel<true, 4>), grid, block, 0, stream, in, out, N, K, steps, nseg,
+                               seg_group);
+        else
+            hipLaunchKernelGGL((qc_frag_rows_kernel<false, 4>), grid, block, 0, stream, in, out, N, K, steps, nseg,
+                               seg_group);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t stream) {
+    if (a.N <= 0 || a.batch <= 0) return hipSuccess;
+    const int tiles = pipe_tiles(a.N);
+    const int64_t blocks = (int64_t)tiles * a.batch;
+    if (blocks > 0x7FFFFFFF || !pipe_supported(a.N, a.K, a.nseg)) return hipErrorInvalidValue;
+    const int steps = frag_steps(a.K) * a.nseg;
+    const dim3 grid((unsigned)blocks), block(P_THREADS);
+    // Plain stores let the L2 join the partial lines at the ends of the runs, and fill it with
+    // output in place of operand rows: they pay where the launch writes more than it multiplies.
+    // Both at 4096 inputs x 17, FP32: K = 256 295 (plain) / 382 us (non-temporal), 384 336 / 378,
+    // 512 402 / 371, 1024 566 / 423; FP16: 128 142 / 245, 256 202 / 237, 384 245 / 221, 512
+    // 286 / 233 us.
+    const int samples = a.K * a.nseg;
+    if (out_fp16) {
+        if (samples > 320)
+            hipLaunchKernelGGL((herk_pipe_kernel<_Float16, true>), grid, block, 0, stream, a, steps, tiles);
+        else
+            hipLaunchKernelGGL((herk_pipe_kernel<_Float16, false>), grid, block, 0, stream, a, steps, tiles);
+    } else {
+        if (samples > 448)
+            hipLaunchKernelGGL((herk_pipe_kernel<float, true>), grid, block, 0, stream, a, steps, tiles);
+        else
+            hipLaunchKernelGGL((herk_pipe_kernel<float, false>), grid, block, 0, stream, a, steps, tiles);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace ftdx

@@ -123,9 +123,15 @@ int ftdx_destroy(ftdx_context* ctx);
 /* Replaces CutlassComplexGemm::herk (cutlass_interface/cutlass_gemm_api.h:750-760;
  * cutlass_gemm_api.cu:1707-1878).  input/compute/output/format take the FTDX_*
  * values above; `tune` != 0 consults (and on a miss fills) the tile-config cache.
- * INT4 rows of K % 16 != 0, or at an address that is not 16-byte aligned, are copied
+ * INT4 input with FP8 compute, no forced mode or tile: small problems run a kernel that splits K
+ * over the waves of a workgroup, larger ones convert each chunk of channels to 6-bit E3M2 operand
+ * rows (every QC value is exact in E3M2, results are those of the FP8 tile bit for bit) and run a
+ * pipelined kernel over them, and the rest the fused FP8 tile.  The rows live in the context, at
+ * most 160 MB (or one channel's) for each of up to four streams that called it; a call without them --
+ * under stream capture, from a fifth stream, or when memory is short -- takes the fused tile.
+ * The fused tile copies rows of K % 16 != 0, or at an address that is not 16-byte aligned,
  * zero-padded (K rounded up to 16, or to the tile's stage) into the context's scratch (at
- * most 320 MB per chunk of channels) before the fused tile runs on them; the FP16-input, ForceBaseline and E3M2
+ * most 320 MB per chunk of channels); the FP16-input, ForceBaseline and E3M2
  * paths stage converted rows there.  The scratch grows on first need unless
  * ftdx_init_herk sized it. */
 int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch_count,
@@ -134,8 +140,8 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
 
 /* Replaces CutlassComplexGemm::init_herk / end_herk (cutlass_gemm_api.h:601-617).
  * init_herk allocates the scratch that calls of this shape need (staged rows for the
- * pre-cast paths and graph mode, padded rows when K % 16 != 0), so that they allocate
- * nothing later; end_herk releases it. */
+ * pre-cast paths and graph mode, padded rows when K % 16 != 0, E3M2 rows for calls on
+ * `stream`), so that they allocate nothing later; end_herk releases it. */
 int ftdx_init_herk(ftdx_context* ctx, int N, int K, int batch_count, void* stream);
 int ftdx_end_herk(ftdx_context* ctx);
 
@@ -171,7 +177,10 @@ int ftdx_set_launch_config(ftdx_context* ctx, int tile_config, int xcd_remap);
 int ftdx_tune_load(ftdx_context* ctx, const char* path, int* loaded, int* skipped);
 int ftdx_tune_save(ftdx_context* ctx, const char* path);
 /* Launch configuration ftdx_herk would use now for this shape without tuning
- * (explicit setting, else cache entry, else the default). */
+ * (explicit setting, else cache entry, else the default).  A cache entry may also hold 64 (the
+ * pipelined kernel over E3M2 rows) or 65 (the K-splitting kernel for small problems), which
+ * ftdx_set_launch_config does not take; without an entry or a setting INT4 calls choose between
+ * them and the fused tile by size. */
 int ftdx_herk_query_config(ftdx_context* ctx, int N, int K, int batch_count, int output,
                            int* tile_config, int* xcd_remap);
 
