@@ -15,6 +15,16 @@
 // owns, refreshed by one pad launch before the HERK launch on every run (captured in the
 // same graph), so the HERK kernel is built with the 16-byte load path only.  If that
 // buffer cannot be allocated, the plan runs the kernel that holds both load paths.
+//
+// A plan of no stated tile configuration may run the pipelined kernel instead: every run
+// converts the problems' rows (any K and alignment) to E3M2 fragment rows in a buffer of
+// the plan, then multiplies from there, one launch each.  No two problems share rows, so
+// runs of one plan on two streams only write the same bytes twice.  The tiles, problems by
+// descending K, are split over the XCDs in eight runs of equal cost, so that one XCD's L2
+// serves the tiles of few problems; inside a run the hardware hands out tiles as workgroups
+// finish.  512 problems of N, K up to 4096: 9.50 ms (persistent, 256 x 128 tiles) to 7.01;
+// in chunks of 160, 320 and 640 MB of rows that stay in the memory-side cache: 7.07, 7.16
+// and 7.02, so the rows go in one piece.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,6 +36,7 @@
 #include "ftdx_host.h"
 #include "ftdx_internal.h"
 #include "herk_fp8.h"
+#include "herk_pipe.h"
 #include "stages.h"
 
 struct ftdx_grouped_plan {
@@ -44,6 +55,11 @@ struct ftdx_grouped_plan {
     ftdx::PadRowsJob* d_pad_jobs = nullptr;
     ftdx::PadBlock* d_pad_blocks = nullptr;
     int pad_blocks = 0;
+    uint8_t* d_rows = nullptr;  // fragment rows of the pipelined kernel; none: not used
+    ftdx::PipeProblem* d_pipe = nullptr;
+    ftdx::ConvBlock* d_conv = nullptr;
+    ftdx::GroupItemDev* d_tiles = nullptr;
+    int conv_blocks = 0;
     bool use_graph = false;
     hipStream_t cap_stream = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -154,7 +170,107 @@ int grouped_build(ftdx_grouped_plan* P, const ftdx_herk_problem* problems, int c
     return FTDX_OK;
 }
 
+namespace {
+
+// The most fragment rows a plan holds (beyond that, or half of what is free, it runs the
+// persistent kernel).
+constexpr size_t kGroupRowsMax = size_t(8) << 30;
+
+template <typename T>
+hipError_t upload(T** dst, const std::vector<T>& v) {
+    hipError_t e = hipMalloc(dst, sizeof(T) * std::max<size_t>(v.size(), 1));
+    if (e == hipSuccess && !v.empty()) e = hipMemcpy(*dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
+    return e;
+}
+
+// Cost of a tile in 64-sample stages: its stages and the share of its stores and its start.
+double pipe_cost(const PipeProblem& p) { return p.steps / 2 + 6.0; }
+
+}  // namespace
+
+// The plan over fragment rows.  FTDX_ERR_UNSUPPORTED: sizes or memory that it does not take (the
+// caller builds the fused plan).
+int grouped_build_pipe(ftdx_grouped_plan* P, const ftdx_herk_problem* problems, int count, int cfg, int out_fp16) {
+    std::vector<PipeProblem> probs;
+    size_t total = 0;
+    int64_t items = 0;
+    for (int i = 0; i < count; ++i) {
+        const ftdx_herk_problem& q = problems[i];
+        if (q.N <= 0) continue;
+        const int kq = std::max(q.K, 16);
+        if (!pipe_supported(q.N, kq)) return FTDX_ERR_UNSUPPORTED;
+        PipeProblem p;
+        p.A = static_cast<const uint8_t*>(q.A);
+        p.rows = nullptr;
+        p.C = q.C;
+        p.N = q.N;
+        p.K = q.K;
+        p.steps = frag_steps(kq);
+        p.nt = pipe_nontemporal(q.K, out_fp16 != 0);
+        p.alpha = q.alpha;
+        p.beta = q.beta;
+        probs.push_back(p);
+        total += (size_t)frag_rows_bytes(q.N, kq);
+        items += pipe_tiles(q.N);
+    }
+    size_t free_bytes = 0, all_bytes = 0;
+    if (probs.empty() || items > 0x0FFFFFFF || total > kGroupRowsMax) return FTDX_ERR_UNSUPPORTED;
+    if (hipMemGetInfo(&free_bytes, &all_bytes) != hipSuccess || total > free_bytes / 2 ||
+        hipMalloc(&P->d_rows, total) != hipSuccess) {
+        (void)hipGetLastError();
+        P->d_rows = nullptr;
+        return FTDX_ERR_UNSUPPORTED;
+    }
+    std::stable_sort(probs.begin(), probs.end(),
+                     [](const PipeProblem& a, const PipeProblem& b) { return a.steps > b.steps; });
+    std::vector<ConvBlock> conv;
+    std::vector<GroupItemDev> run[8], tiles;
+    uint8_t* at = P->d_rows;
+    double cost = 0.0, done = 0.0, load[8] = {};
+    for (size_t p = 0; p < probs.size(); ++p) {
+        PipeProblem& q = probs[p];
+        q.rows = at;
+        at += (size_t)((q.N + 31) / 32) * q.steps * kFragBytes;
+        cost += pipe_cost(q) * pipe_tiles(q.N);
+        const int64_t segs = (int64_t)(q.N + 31) / 32 * 64 * q.steps;  // < 2^31: its rows' bytes / 24
+        for (int64_t f = 0; f < segs; f += kConvThreads) conv.push_back({(int)p, (uint32_t)f});
+    }
+    for (size_t p = 0; p < probs.size(); ++p) {
+        const double one = pipe_cost(probs[p]);
+        const int n = pipe_tiles(probs[p].N);
+        for (int t = 0; t < n; ++t, done += one) {
+            const int x = std::min(7, (int)(8.0 * done / cost));
+            run[x].push_back({(int)p, t});
+            load[x] += one;
+        }
+    }
+    size_t len = 0;
+    for (const auto& r : run) len = std::max(len, r.size());
+    for (size_t k = 0; k < len; ++k)
+        for (const auto& r : run) tiles.push_back(k < r.size() ? r[k] : GroupItemDev{-1, 0});
+    hipError_t e;
+    if ((e = upload(&P->d_pipe, probs)) != hipSuccess || (e = upload(&P->d_conv, conv)) != hipSuccess ||
+        (e = upload(&P->d_tiles, tiles)) != hipSuccess) {
+        (void)hipGetLastError();
+        return FTDX_ERR_UNSUPPORTED;
+    }
+    P->items = items;
+    P->max_load = *std::max_element(load, load + 8);
+    P->mean_load = cost / 8.0;
+    P->num_wg = (int)tiles.size();  // at most 8 items: < 2^31
+    P->conv_blocks = (int)conv.size();
+    P->cfg = cfg;
+    P->out_fp16 = out_fp16;
+    P->count = count;
+    return FTDX_OK;
+}
+
 hipError_t grouped_launch(ftdx_grouped_plan* P, hipStream_t s) {
+    if (P->d_rows) {
+        hipError_t e = launch_qc_frag_rows_multi(P->d_pipe, P->d_conv, P->conv_blocks, s);
+        if (e != hipSuccess) return e;
+        return launch_herk_pipe_grouped(P->d_pipe, P->d_tiles, P->num_wg, P->out_fp16 != 0, s);
+    }
     if (P->pad_blocks > 0) {
         hipError_t e = launch_pad_qc_rows_multi(P->d_pad_jobs, P->d_pad_blocks, P->pad_blocks, s);
         if (e != hipSuccess) return e;
@@ -173,6 +289,14 @@ void grouped_release(ftdx_grouped_plan* P) {
     if (P->d_pad) (void)hipFree(P->d_pad);
     if (P->d_pad_jobs) (void)hipFree(P->d_pad_jobs);
     if (P->d_pad_blocks) (void)hipFree(P->d_pad_blocks);
+    if (P->d_rows) (void)hipFree(P->d_rows);
+    if (P->d_pipe) (void)hipFree(P->d_pipe);
+    if (P->d_conv) (void)hipFree(P->d_conv);
+    if (P->d_tiles) (void)hipFree(P->d_tiles);
+    P->d_rows = nullptr;
+    P->d_pipe = nullptr;
+    P->d_conv = nullptr;
+    P->d_tiles = nullptr;
     P->d_pad = nullptr;
     P->d_pad_jobs = nullptr;
     P->d_pad_blocks = nullptr;
@@ -205,17 +329,20 @@ int grouped_capture(ftdx_grouped_plan* P) {
     return FTDX_OK;
 }
 
-// Times each tile configuration's plan on the problems' own buffers (outputs are
-// overwritten: only used when every beta is 0) and returns the fastest.
-int grouped_autotune(const ftdx_herk_problem* problems, int count, int out16, int cus, int& best,
-                     float& best_ms) {
+// Times each tile configuration's plan, and the pipelined one, on the problems' own buffers
+// (outputs are overwritten: only used when every beta is 0): the fastest tile configuration,
+// and whether the pipelined plan beat it.
+int grouped_autotune(const ftdx_herk_problem* problems, int count, int out16, int cus, int& best, bool& pipe) {
     hipEvent_t t0, t1;
     (void)hipEventCreate(&t0);
     (void)hipEventCreate(&t1);
-    best_ms = 1e30f;
-    for (int cfg = 0; cfg < NUM_TILE_CONFIGS; ++cfg) {
+    float best_ms = 1e30f;
+    pipe = false;
+    for (int cfg = 0; cfg <= NUM_TILE_CONFIGS; ++cfg) {
         ftdx_grouped_plan P;
-        int rc = grouped_build(&P, problems, count, cfg, out16, cus);
+        const bool rows = cfg == NUM_TILE_CONFIGS;
+        int rc = rows ? grouped_build_pipe(&P, problems, count, best, out16)
+                      : grouped_build(&P, problems, count, cfg, out16, cus);
         if (rc != FTDX_OK) {
             grouped_release(&P);
             continue;
@@ -235,7 +362,8 @@ int grouped_autotune(const ftdx_herk_problem* problems, int count, int out16, in
         grouped_release(&P);
         if (ms < best_ms) {
             best_ms = ms;
-            best = cfg;
+            if (rows) pipe = true;
+            else best = cfg;
         }
     }
     (void)hipEventDestroy(t0);
@@ -279,14 +407,18 @@ int ftdx_herk_grouped_plan_create(ftdx_context* ctx, const ftdx_herk_problem* pr
     int cfg = tile_config >= 0 ? tile_config : ftdx::TILE_128x128_K64;
     bool all_beta0 = true;
     for (int p = 0; p < count; ++p) all_beta0 = all_beta0 && problems[p].beta == 0.0f;
+    bool pipe = false;
     if (tile_config < 0 && all_beta0 && count > 0) {
-        float best_ms = 0.0f;
-        int rc = ftdx::grouped_autotune(problems, count, out16, cus, cfg, best_ms);
+        int rc = ftdx::grouped_autotune(problems, count, out16, cus, cfg, pipe);
         if (rc != FTDX_OK) return rc;
     }
     auto* P = new ftdx_grouped_plan();
     P->device = dev;
-    int rc = ftdx::grouped_build(P, problems, count, cfg, out16, cus);
+    int rc = pipe ? ftdx::grouped_build_pipe(P, problems, count, cfg, out16) : FTDX_ERR_UNSUPPORTED;
+    if (rc != FTDX_OK) {  // also when the rows' memory went to someone else meanwhile
+        ftdx::grouped_release(P);
+        rc = ftdx::grouped_build(P, problems, count, cfg, out16, cus);
+    }
     if (rc == FTDX_OK && use_graph && P->items > 0) rc = ftdx::grouped_capture(P);
     if (rc != FTDX_OK) {
         ftdx::grouped_release(P);

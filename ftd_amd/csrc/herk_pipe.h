@@ -39,4 +39,28 @@ hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t s
 int pipe_tiles(int N);
 int pipe_wg_per_cu();
 
+// Whether the stores of the launch above are non-temporal (samples: of all segments).
+bool pipe_nontemporal(int samples, bool out_fp16);
+
+// ---- many problems of different sizes ----
+struct PipeProblem {
+    const uint8_t* A;  // QC rows [N][K], any K >= 0 and alignment
+    uint8_t* rows;     // their fragment rows, 16-byte aligned
+    void* C;
+    int N, K, steps;   // steps: max(frag_steps(K), 2)
+    int nt;            // pipe_nontemporal
+    float alpha, beta;
+};
+// Segments from `first` of problem `prob`: (N rounded up to 32) * 2 steps of them in all.
+constexpr int kConvThreads = 2048;
+struct ConvBlock {
+    int prob;
+    uint32_t first;  // a multiple of kConvThreads
+};
+// All arrays in device memory.  tiles[b]: problem and tile (0 .. pipe_tiles(N) - 1) of
+// workgroup b, prob < 0 for none; workgroup b runs on XCD b mod 8.
+hipError_t launch_qc_frag_rows_multi(const PipeProblem* probs, const ConvBlock* blocks, int nblocks, hipStream_t stream);
+hipError_t launch_herk_pipe_grouped(const PipeProblem* probs, const GroupItemDev* tiles, int ntiles, bool out_fp16,
+                                    hipStream_t stream);
+
 }  // namespace ftdx

@@ -247,20 +247,17 @@ __device__ __forceinline__ void tri_decode_blocked(int t, int nb, int H, int& I,
     }
 }
 
-template <typename OutT, bool NT>
-__global__ void __launch_bounds__(P_THREADS, 2) herk_pipe_kernel(HerkPlainArgs p, int steps, int tiles) {
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[P_BUFS * P_STAGE];
-    const int w = xcd_logical((int)blockIdx.x, tiles * p.batch);
-    const int b = w / tiles, t = w - b * tiles;
-    int I, J;
-    tri_decode_blocked(t, (p.N + PT - 1) / PT, P_BLOCK, I, J);
+// Tile (I, J) of one problem: `base` its fragment rows, `steps` per row.
+template <typename OutT>
+__device__ __forceinline__ void pipe_tile(uint8_t* lds, const uint8_t* base, int N, int steps, int I, int J, OutT* C,
+                                          float alpha, float beta, bool nt) {
     // wave index in an SGPR: the conditions on it are scalar branches
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int wrow = I * PT + wm * 64, wcol = J * PT + wn * 64;
-    const bool active = wrow < p.N && wrow + 63 >= wcol;
+    const bool active = wrow < N && wrow + 63 >= wcol;
     // groups past N (edge tiles) read the last group; their products are not stored
-    const int ng = (p.N + 31) / 32;
+    const int ng = (N + 31) / 32;
     uint32_t off[P_LOADS];
 #pragma unroll
     for (int q = 0; q < P_LOADS; ++q) {
@@ -269,8 +266,7 @@ __global__ void __launch_bounds__(P_THREADS, 2) herk_pipe_kernel(HerkPlainArgs p
         off[q] = (uint32_t)(want < ng ? want : ng - 1) * (uint32_t)(steps * kFragBytes) + (uint32_t)((k % 3) * 1024 + lane * 16);
     }
     const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(p.A) + (int64_t)b * p.a_bstride, 0, (int)((uint32_t)ng * (uint32_t)(steps * kFragBytes)),
-        0x00027000);
+        const_cast<uint8_t*>(base), 0, (int)((uint32_t)ng * (uint32_t)(steps * kFragBytes)), 0x00027000);
     v16f re[2][2], im[2][2];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
@@ -287,13 +283,41 @@ __global__ void __launch_bounds__(P_THREADS, 2) herk_pipe_kernel(HerkPlainArgs p
         return;
     }
     tile_loop<true>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
-    OutT* C = static_cast<OutT*>(p.C) + (int64_t)b * p.c_bstride;
-    if (wcol + 63 < wrow && wrow + 64 <= p.N && p.beta == 0.0f) {
-        if (p.alpha == 1.0f) store_inside<OutT, false, NT>(C, wrow, wcol, p.alpha, re, im, lane);
-        else store_inside<OutT, true, NT>(C, wrow, wcol, p.alpha, re, im, lane);
+    if (wcol + 63 < wrow && wrow + 64 <= N && beta == 0.0f) {
+        if (nt) {
+            if (alpha == 1.0f) store_inside<OutT, false, true>(C, wrow, wcol, alpha, re, im, lane);
+            else store_inside<OutT, true, true>(C, wrow, wcol, alpha, re, im, lane);
+        } else {
+            if (alpha == 1.0f) store_inside<OutT, false, false>(C, wrow, wcol, alpha, re, im, lane);
+            else store_inside<OutT, true, false>(C, wrow, wcol, alpha, re, im, lane);
+        }
     } else {
-        store_any<OutT>(C, p.N, wrow, wcol, p.alpha, p.beta, re, im, lane);
+        store_any<OutT>(C, N, wrow, wcol, alpha, beta, re, im, lane);
     }
+}
+
+template <typename OutT, bool NT>
+__global__ void __launch_bounds__(P_THREADS, 2) herk_pipe_kernel(HerkPlainArgs p, int steps, int tiles) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[P_BUFS * P_STAGE];
+    const int w = xcd_logical((int)blockIdx.x, tiles * p.batch);
+    const int b = w / tiles, t = w - b * tiles;
+    int I, J;
+    tri_decode_blocked(t, (p.N + PT - 1) / PT, P_BLOCK, I, J);
+    pipe_tile<OutT>(lds, p.A + (int64_t)b * p.a_bstride, p.N, steps, I, J,
+                    static_cast<OutT*>(p.C) + (int64_t)b * p.c_bstride, p.alpha, p.beta, NT);
+}
+
+// Tiles of many problems: workgroup b runs tiles[b].
+template <typename OutT>
+__global__ void __launch_bounds__(P_THREADS, 2)
+herk_pipe_grouped_kernel(const PipeProblem* __restrict__ probs, const GroupItemDev* __restrict__ tiles) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[P_BUFS * P_STAGE];
+    const GroupItemDev it = tiles[blockIdx.x];
+    if (it.prob < 0) return;  // this XCD's list is shorter than the longest
+    const PipeProblem p = probs[it.prob];
+    int I, J;
+    tri_decode_blocked(it.tile, (p.N + PT - 1) / PT, P_BLOCK, I, J);
+    pipe_tile<OutT>(lds, p.rows, p.N, p.steps, I, J, static_cast<OutT*>(p.C), p.alpha, p.beta, p.nt != 0);
 }
 
 // ---- QC rows -> fragment rows ----
@@ -320,16 +344,37 @@ __device__ __forceinline__ void pack16(const uint32_t (&c)[4], uint32_t& d0, uin
     d2 = (p2 >> 16) | (p3 << 8);
 }
 
+// 16 samples -> their place in the fragment step at dst (lane as in herk_pipe.h)
+__device__ __forceinline__ void put_frag(uint4 w, uint8_t* dst, int lane) {
+    uint32_t re[4], im[4];
+    qc4_codes(w.x, re[0], im[0]);
+    qc4_codes(w.y, re[1], im[1]);
+    qc4_codes(w.z, re[2], im[2]);
+    qc4_codes(w.w, re[3], im[3]);
+    uint4 a;
+    uint2 b;
+    pack16(re, a.x, a.y, a.z);
+    pack16(im, a.w, b.x, b.y);
+    *reinterpret_cast<uint4*>(dst + lane * 16) = a;
+    *reinterpret_cast<uint2*>(dst + 1024 + lane * 8) = b;
+}
+
+// Row and 16-sample segment of conversion thread t: waves of S segments x 64 / S rows.
+__device__ __forceinline__ void conv_place(uint32_t t, int segs, int S, int& r, int& s) {
+    const uint32_t v = t / 64u, per = (uint32_t)(segs / S);
+    const uint32_t rb = v / per, sb = v - rb * per;
+    s = (int)sb * S + (int)(t % S);
+    r = (int)rb * (64 / S) + (int)(t / S % (64 / S));
+}
+
 // VEC: K % 16 == 0 and 16-byte aligned rows
 template <bool VEC, int S>
 __global__ void __launch_bounds__(256)
 qc_frag_rows_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int N, int K, int steps, int nseg,
                     int grp) {
-    constexpr int R = 64 / S;
-    const int ng = (N + 31) / 32, segs = steps * 2;
-    const uint32_t t = blockIdx.x * 256u + threadIdx.x, v = t / 64u;
-    const uint32_t sb = v % (uint32_t)(segs / S), rb = v / (uint32_t)(segs / S);
-    const int s = (int)sb * S + (int)(t % S), r = (int)rb * R + (int)(t / S % R);
+    const int ng = (N + 31) / 32;
+    int r, s;
+    conv_place(blockIdx.x * 256u + threadIdx.x, steps * 2, S, r, s);
     if (r >= ng * 32) return;
     const int ib = (int)blockIdx.y, ob = ib / (nseg * grp), sg = ib / grp - ob * nseg;
     const int64_t dst_batch = (int64_t)ob * grp + ib % grp;
@@ -342,19 +387,36 @@ qc_frag_rows_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, i
             w = row_segment(row, s * 16, K);
         }
     }
-    uint32_t re[4], im[4];
-    qc4_codes(w.x, re[0], im[0]);
-    qc4_codes(w.y, re[1], im[1]);
-    qc4_codes(w.z, re[2], im[2]);
-    qc4_codes(w.w, re[3], im[3]);
-    uint4 a;
-    uint2 b;
-    pack16(re, a.x, a.y, a.z);
-    pack16(im, a.w, b.x, b.y);
-    const int lane = (r & 31) + 32 * (s & 1);
-    uint8_t* dst = out + ((dst_batch * ng + (r >> 5)) * (int64_t)(steps * nseg) + sg * steps + (s >> 1)) * kFragBytes;
-    *reinterpret_cast<uint4*>(dst + lane * 16) = a;
-    *reinterpret_cast<uint2*>(dst + 1024 + lane * 8) = b;
+    put_frag(w, out + ((dst_batch * ng + (r >> 5)) * (int64_t)(steps * nseg) + sg * steps + (s >> 1)) * kFragBytes,
+             (r & 31) + 32 * (s & 1));
+}
+
+// The rows of many problems: workgroup b converts up to kConvThreads segments of one problem.
+__global__ void __launch_bounds__(256)
+qc_frag_rows_multi_kernel(const PipeProblem* __restrict__ probs, const ConvBlock* __restrict__ blocks) {
+    const ConvBlock cb = blocks[blockIdx.x];
+    const PipeProblem p = probs[cb.prob];
+    const int ng = (p.N + 31) / 32, segs = p.steps * 2, S = segs % 8 == 0 ? 8 : 4;
+    const bool vec = p.K % 16 == 0 && (reinterpret_cast<uintptr_t>(p.A) & 15u) == 0;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kConvThreads; i += 256u) {
+        int r, s;
+        conv_place(cb.first + i, segs, S, r, s);
+        if (r >= ng * 32) return;
+        uint4 w = make_uint4(0u, 0u, 0u, 0u);
+        if (r < p.N) {
+            const uint8_t* row = p.A + (int64_t)r * p.K;
+            if (vec) {
+                if (s * 16 < p.K) w = *reinterpret_cast<const uint4*>(row + s * 16);
+            } else if (p.K >= 16) {
+                w = row_segment(row, s * 16, p.K);
+            } else if (s == 0) {
+                uint32_t d[4] = {0u, 0u, 0u, 0u};
+                for (int k = 0; k < p.K; ++k) d[k >> 2] |= (uint32_t)row[k] << (8 * (k & 3));
+                w = make_uint4(d[0], d[1], d[2], d[3]);
+            }
+        }
+        put_frag(w, p.rows + ((int64_t)(r >> 5) * p.steps + (s >> 1)) * kFragBytes, (r & 31) + 32 * (s & 1));
+    }
 }
 
 }  // namespace
@@ -370,6 +432,29 @@ int pipe_tiles(int N) {
 }
 
 int pipe_wg_per_cu() { return P_WG_PER_CU; }
+
+// Plain stores let the L2 join the partial lines at the ends of the runs, and fill it with
+// output in place of operand rows: they pay where the launch writes more than it multiplies.
+// Both at 4096 inputs x 17, FP32: K = 256 295 (plain) / 382 us (non-temporal), 384 336 / 378,
+// 512 402 / 371, 1024 566 / 423; FP16: 128 142 / 245, 256 202 / 237, 384 245 / 221, 512
+// 286 / 233 us.
+bool pipe_nontemporal(int samples, bool out_fp16) { return samples > (out_fp16 ? 320 : 448); }
+
+hipError_t launch_qc_frag_rows_multi(const PipeProblem* probs, const ConvBlock* blocks, int nblocks, hipStream_t s) {
+    if (nblocks <= 0) return hipSuccess;
+    hipLaunchKernelGGL(qc_frag_rows_multi_kernel, dim3((unsigned)nblocks), dim3(256), 0, s, probs, blocks);
+    return hipGetLastError();
+}
+
+hipError_t launch_herk_pipe_grouped(const PipeProblem* probs, const GroupItemDev* tiles, int ntiles, bool out_fp16,
+                                    hipStream_t s) {
+    if (ntiles <= 0) return hipSuccess;
+    if (out_fp16)
+        hipLaunchKernelGGL(herk_pipe_grouped_kernel<_Float16>, dim3((unsigned)ntiles), dim3(P_THREADS), 0, s, probs, tiles);
+    else
+        hipLaunchKernelGGL(herk_pipe_grouped_kernel<float>, dim3((unsigned)ntiles), dim3(P_THREADS), 0, s, probs, tiles);
+    return hipGetLastError();
+}
 
 hipError_t launch_qc_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, int batches, int nseg, int seg_group,
                                hipStream_t stream) {
@@ -404,19 +489,14 @@ hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t s
     if (blocks > 0x7FFFFFFF || !pipe_supported(a.N, a.K, a.nseg)) return hipErrorInvalidValue;
     const int steps = frag_steps(a.K) * a.nseg;
     const dim3 grid((unsigned)blocks), block(P_THREADS);
-    // Plain stores let the L2 join the partial lines at the ends of the runs, and fill it with
-    // output in place of operand rows: they pay where the launch writes more than it multiplies.
-    // Both at 4096 inputs x 17, FP32: K = 256 295 (plain) / 382 us (non-temporal), 384 336 / 378,
-    // 512 402 / 371, 1024 566 / 423; FP16: 128 142 / 245, 256 202 / 237, 384 245 / 221, 512
-    // 286 / 233 us.
-    const int samples = a.K * a.nseg;
+    const bool nt = pipe_nontemporal(a.K * a.nseg, out_fp16);
     if (out_fp16) {
-        if (samples > 320)
+        if (nt)
             hipLaunchKernelGGL((herk_pipe_kernel<_Float16, true>), grid, block, 0, stream, a, steps, tiles);
         else
             hipLaunchKernelGGL((herk_pipe_kernel<_Float16, false>), grid, block, 0, stream, a, steps, tiles);
     } else {
-        if (samples > 448)
+        if (nt)
             hipLaunchKernelGGL((herk_pipe_kernel<float, true>), grid, block, 0, stream, a, steps, tiles);
         else
             hipLaunchKernelGGL((herk_pipe_kernel<float, false>), grid, block, 0, stream, a, steps, tiles);

@@ -190,7 +190,11 @@ int ftdx_herk_query_config(ftdx_context* ctx, int N, int K, int batch_count, int
  * of uneven size.  A plan uploads the problem list and a static tile schedule;
  * with use_graph != 0 the launch is captured once in a hipGraph and replayed.
  * tile_config = FTDX_TILE_AUTO times the configurations on the problems' own
- * buffers when every beta is 0 (C is overwritten), else uses the default.
+ * buffers when every beta is 0 (C is overwritten), else uses the default.  Such a
+ * timed plan may instead convert all rows to 6-bit rows (1.5 bytes per sample, at
+ * most 8 GiB and half of the free memory, owned by the plan) and run one workgroup
+ * per tile over them; plan_info then gives those workgroups, and as tile_config the
+ * fastest of the fused configurations.
  * All outputs share one precision.  The plan keeps the pointers: buffers must
  * outlive it.  Problems whose rows 16-byte loads cannot take (K % 16 != 0, or A
  * not 16-byte aligned) run on zero-padded copies (K rounded up to 16) in device

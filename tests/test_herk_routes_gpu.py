@@ -192,3 +192,46 @@ def test_choice_by_size_bit_exact(oracle, dev):
         torch.cuda.synchronize()
         ref = oracle.herk_f32(qc, N, K, B) if K else np.zeros(C.shape, np.float32)
         assert np.array_equal(_bits(C.cpu().numpy()), _bits(ref)), (N, K, B)
+
+
+# A plan of large problems runs the pipelined kernel; the small ones among them take its edges
+# (no samples, rows shorter than one 16-byte segment, tile and stage remainders, unaligned rows).
+GROUP_EDGES = [(1, 5), (40, 0), (33, 15), (64, 16), (65, 17), (127, 65), (129, 64), (257, 449), (31, 1000)]
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("fp16", [False, True])
+def test_grouped_fragment_rows_bit_exact(oracle, dev, graph, fp16):
+    import torch
+    from ftd_amd import ftdx
+    out = ftdx.OutputPrecision.FP16 if fp16 else ftdx.OutputPrecision.FP32
+    dt = torch.float16 if fp16 else torch.float32
+    ctx, probs, refs = ftdx.CutlassComplexGemm(), [], []
+    for i, (N, K) in enumerate(GROUP_EDGES):
+        qc = oracle.gen_bytes(70 + i, max(N * K, 1))
+        buf = torch.zeros(qc.size + i, dtype=torch.uint8, device=dev)
+        buf[i:].copy_(torch.from_numpy(qc))
+        C = torch.full((N * (N + 1) // 2, 2), float("nan"), dtype=dt, device=dev)
+        probs.append((buf[i:], C, N, K, 0.5 if i % 2 else 1.0, 0.0))
+        alpha = probs[-1][4]
+        ref = (oracle.herk_f16 if fp16 else oracle.herk_f32)(qc[:N * K], N, K, 1, alpha=alpha) if K else None
+        refs.append(None if ref is None else ref[0])
+    big = [(2048, 2048)] * 24
+    Ab = torch.randint(0, 256, (2048 * 2048,), dtype=torch.uint8, device=dev)
+    Cb = [torch.empty((2048 * 2049 // 2, 2), dtype=dt, device=dev) for _ in big]
+    probs += [(Ab, C, N, K, 1.0, 0.0) for C, (N, K) in zip(Cb, big)]
+    plan = ftdx.GroupedPlan(ctx, probs, output=out, use_graph=graph)
+    assert plan.info()["workgroups"] > 24 * 136  # a workgroup per tile: not the persistent kernel
+    fused = torch.empty_like(Cb[0])
+    one = ftdx.GroupedPlan(ctx, [(Ab, fused, 2048, 2048, 1.0, 0.0)], output=out, tile_config=0, use_graph=False)
+    one.run()
+    for _ in range(3):
+        for p in probs:
+            p[1].fill_(float("nan"))
+        plan.run()
+        torch.cuda.synchronize()
+        for p, ref in zip(probs, refs):
+            got = p[1].cpu().numpy()
+            assert np.array_equal(_bits(got), _bits(np.zeros_like(got) if ref is None else ref)), (p[2], p[3])
+        for C in Cb:
+            assert torch.equal(C, fused)
