@@ -25,8 +25,8 @@ namespace ftdx {
 int xengine_cfg(int forced, int N, int batch);
 // Bytes of pre-cast operand rows for batch x N rows of K samples.
 size_t rows_bytes(int N, int K, int batch);
-// One GGP payload: convert to pre-cast rows, then HERK into `out` in layout `fmt`
-// (OUT_UPPER_PACKED or OUT_HERM_FULL), FP32 or FP64.
+// One GGP payload: convert to operand rows, then HERK into `out` in layout `fmt`
+// (OUT_UPPER_PACKED or OUT_HERM_FULL), FP32 or FP64.  cfg < 0: no forced tile.
 hipError_t run_ggp_payload(const uint8_t* in, void* out, uint8_t* rows, int N, int K, int batch,
                            int fmt, bool fp64, int cfg, int remap, hipStream_t s);
 // Pre-cast conj(B) rows of a context whose prepare_b ran with FP8 compute and this

@@ -6,11 +6,12 @@
 //   the full N x N M^H M -> triangulateFromHerm (upper triangle, row-major),
 // and its TCC branch runs convertQcSmToFtd -> reorder -> libtcc -> int2-to-float
 // (lib/tcc_interface.cu:124-314).  Here both are two launches per payload:
-//   1. a transposing converter writes the pre-cast FP8 operand rows of every
-//      batch (stages.hip: ggp_to_fp8_rows / ftd_to_fp8_rows);
-//   2. the HERK tile kernel computes only the lower-triangle tiles and writes the
-//      caller's layout from its epilogue (GGP upper packed, GGP full Hermitian, or
-//      the HERK lower packed), in FP32 or FP64.
+//   1. a transposing converter writes the operand rows of every batch: E3M2 fragment
+//      rows (herk_pipe.hip) for GGP payloads where they pay, else pre-cast FP8 rows
+//      (stages.hip: ggp_to_fp8_rows / ftd_to_fp8_rows);
+//   2. the pipelined HERK or the FP8 tile kernel computes only the lower-triangle
+//      tiles and writes the caller's layout from its epilogue (GGP upper packed, GGP
+//      full Hermitian, or the HERK lower packed), in FP32 or FP64.
 // Integer inputs make every product exact: FP32 accumulation is exact while the
 // sum stays below 2^24 (128 K for [-8, 7] nibbles); FP64 output longer than that
 // is accumulated in K chunks with beta = 1 (exact in double).
@@ -18,12 +19,14 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <new>
 #include <string>
 
 #include "ftdx_internal.h"
 #include "herk_fp8.h"
+#include "herk_pipe.h"
 #include "stages.h"
 
 namespace ftdx {
@@ -38,13 +41,31 @@ int heuristic_cfg(int N, int batch) {
     return (N <= 128 || tiles < 512) ? TILE_64x64_K64 : TILE_128x128_K64;
 }
 
+// Whether a GGP payload takes the pipelined kernel over E3M2 fragment rows, which holds every
+// [-8, 7] nibble exactly: where one pass is exact, the rows need at most 64 MB more scratch than
+// the FP8 ones (groups of 32 rows: few antennas waste them), and except for full FP64 matrices
+// of few tiles, whose scattered lower-half stores one workgroup then waits for.  us per call,
+// FP8 tile / pipelined, both polarizations:
+//   upper FP32:  64 x 2, K 64  26 / 24     1024 x 32, K 256  96 / 56     2048 x 8, K 1024  127 / 90
+//   full FP32:   64 x 2, K 64  28 / 25     1024 x 32, K 256 430 / 77     2048 x 8, K 1024  393 / 131
+//   upper FP64: 512 x 8, K 64  29 / 27     1024 x 32, K 256 124 / 75     2048 x 8, K 1024  148 / 113
+//   full FP64:  256 x 8, K 512 36 / 39      512 x 4, K 1024  45 / 45     2048 x 8, K 1024  541 / 191
+bool ggp_pipe(int N, int K, int batch, bool herm, bool fp64) {
+    const int64_t tiles = pipe_supported(N, K) ? (int64_t)pipe_tiles(N) * batch : 0;
+    return K <= kExactK && tiles > 0 && tiles <= 0x7FFFFFFF &&
+           (size_t)frag_rows_bytes(N, K) * batch <= rows_bytes(N, K, batch) + (size_t(64) << 20) &&
+           !(herm && fp64 && N > 128 && tiles < 64);
+}
+
 }  // namespace
 
 int xengine_cfg(int forced, int N, int batch) { return forced >= 0 ? forced : heuristic_cfg(N, batch); }
 
 hipError_t run_ggp_payload(const uint8_t* in, void* out, uint8_t* rows, int N, int K, int batch,
                            int fmt, bool fp64, int cfg, int remap, hipStream_t s) {
-    hipError_t e = launch_ggp_to_fp8_rows(in, rows, N, K, batch, s);
+    const bool pipe = cfg < 0 && ggp_pipe(N, K, batch, fmt == OUT_HERM_FULL, fp64);
+    hipError_t e = pipe ? launch_ggp_frag_rows(in, rows, N, K, batch, s)
+                        : launch_ggp_to_fp8_rows(in, rows, N, K, batch, s);
     if (e != hipSuccess) return e;
     const int Kp = precast_row_samples(K);
     HerkPlainArgs a;
@@ -56,6 +77,12 @@ hipError_t run_ggp_payload(const uint8_t* in, void* out, uint8_t* rows, int N, i
     a.beta = 0.0f;
     a.a_bstride = (int64_t)N * Kp * 2;
     a.c_bstride = fmt == OUT_HERM_FULL ? (int64_t)N * N * 2 : (int64_t)N * (N + 1);
+    if (pipe) {
+        a.K = K;
+        a.a_bstride = frag_rows_bytes(N, K);
+        return launch_herk_pipe_ggp(a, fmt, fp64, s);
+    }
+    cfg = xengine_cfg(cfg, N, batch);
     a.precast = 1;
     a.lda = (int64_t)Kp * 2;
     if (K <= kExactK || !fp64) {
@@ -107,7 +134,7 @@ struct ftdx_xengine {
     size_t in_payload = 0, out_payload = 0;
     uint8_t* d_in = nullptr;   // device copy of a host input payload
     uint8_t* d_out = nullptr;  // device output of a payload bound for the host
-    uint8_t* rows = nullptr;   // pre-cast FP8 operand rows of one payload
+    uint8_t* rows = nullptr;   // operand rows of one payload
     int cfg = -1, remap = -1;
 };
 
@@ -221,7 +248,10 @@ int ftdx_xengine_create(const ftdx_xengine_param* param, ftdx_xengine** out) {
         delete xe;
         return hip_fail(e, "xengine_create: output copy");
     }
-    if ((e = hipMalloc(&xe->rows, ftdx::rows_bytes(xe->N, xe->K, xe->batch) + 16)) != hipSuccess) {
+    size_t rows = ftdx::rows_bytes(xe->N, xe->K, xe->batch) + 16;
+    if (!xe->tcc && ftdx::ggp_pipe(xe->N, xe->K, xe->batch, xe->herm, xe->fp64))
+        rows = std::max(rows, (size_t)ftdx::frag_rows_bytes(xe->N, xe->K) * xe->batch);
+    if ((e = hipMalloc(&xe->rows, rows)) != hipSuccess) {
         release(xe);
         delete xe;
         return hip_fail(e, "xengine_create: operand rows");
@@ -254,7 +284,6 @@ int ftdx_xengine_compute(ftdx_xengine* xe, void* output, const void* input, void
     if (!xe || !output || !input) return fail(FTDX_ERR_INVALID_ARG, "xengine_compute: NULL argument");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const ftdx_xengine_param& p = xe->p;
-    const int cfg = ftdx::xengine_cfg(xe->cfg, xe->N, xe->batch);
     const int remap = xe->remap >= 0 ? xe->remap : 1;
     hipError_t e;
     for (size_t i = 0; i < p.n_payload; ++i) {
@@ -269,10 +298,11 @@ int ftdx_xengine_compute(ftdx_xengine* xe, void* output, const void* input, void
         if (xe->tcc)
             e = ftdx::run_ftd_payload(src, static_cast<float*>(res), xe->rows, xe->N,
                                       (int)p.n_channels_per_payload, (int)p.n_time_per_payload,
-                                      (int)p.n_time_inner, (int)p.n_polarizations, false, cfg, remap, s);
+                                      (int)p.n_time_inner, (int)p.n_polarizations, false,
+                                      ftdx::xengine_cfg(xe->cfg, xe->N, xe->batch), remap, s);
         else
             e = ftdx::run_ggp_payload(src, res, xe->rows, xe->N, xe->K, xe->batch,
-                                      xe->herm ? ftdx::OUT_HERM_FULL : ftdx::OUT_UPPER_PACKED, xe->fp64, cfg,
+                                      xe->herm ? ftdx::OUT_HERM_FULL : ftdx::OUT_UPPER_PACKED, xe->fp64, xe->cfg,
                                       remap, s);
         if (e != hipSuccess) return hip_fail(e, "xengine_compute: kernels");
         if (p.out_location == FTDX_LOCATION_HOST &&

@@ -107,6 +107,20 @@ __device__ __forceinline__ int xcd_logical(int w, int total) {
     return x * q + (x < r ? x : r) + local;
 }
 
+// d0..d3: one dword per sample holding 4 antennas' bytes -> one dword per antenna
+// holding its 4 samples' bytes (byte a of dword s goes to byte s of output a).
+__device__ __forceinline__ void transpose4x4_bytes(uint32_t d0, uint32_t d1, uint32_t d2, uint32_t d3,
+                                                   uint32_t (&o)[4]) {
+    const uint32_t l01 = __builtin_amdgcn_perm(d1, d0, 0x05010400u);  // d0.b0 d1.b0 d0.b1 d1.b1
+    const uint32_t h01 = __builtin_amdgcn_perm(d1, d0, 0x07030602u);  // d0.b2 d1.b2 d0.b3 d1.b3
+    const uint32_t l23 = __builtin_amdgcn_perm(d3, d2, 0x05010400u);
+    const uint32_t h23 = __builtin_amdgcn_perm(d3, d2, 0x07030602u);
+    o[0] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
+    o[1] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
+    o[2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
+    o[3] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
+}
+
 // lower-triangle tile index t -> (bi, bj), bj <= bi, t = bi(bi+1)/2 + bj
 __device__ __forceinline__ void tri_decode(int t, int& bi, int& bj) {
     int r = (int)((__builtin_sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);

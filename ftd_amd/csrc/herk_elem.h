@@ -26,6 +26,16 @@ struct Elem<_Float16> {
         return v;
     }
 };
+template <>
+struct Elem<double> {
+    typedef double v2 __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ v2 make(float r, float i) {
+        v2 v;
+        v[0] = r;
+        v[1] = i;
+        return v;
+    }
+};
 
 // C = alpha * (r, i) + beta * C for one element: alpha first, then fma(beta, old, .), one
 // rounding each, as the other HERK kernels.

@@ -35,6 +35,11 @@ hipError_t launch_qc_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, in
 // samples of one segment (a.nseg of them); packed lower triangle as launch_herk_int4_plain.
 hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t stream);
 
+// GGP bytes [batches][K][N], any alignment -> fragment rows; the HERK over them with the GGP
+// layouts of launch_herk_ggp (OUT_UPPER_PACKED or OUT_HERM_FULL, FP32 or FP64), alpha 1, beta 0.
+hipError_t launch_ggp_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, int batches, hipStream_t stream);
+hipError_t launch_herk_pipe_ggp(const HerkPlainArgs& a, int fmt, bool out_fp64, hipStream_t stream);
+
 // Tiles per batch and resident workgroups per CU of the launch above.
 int pipe_tiles(int N);
 int pipe_wg_per_cu();

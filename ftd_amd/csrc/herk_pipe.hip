@@ -90,7 +90,9 @@ __device__ __forceinline__ void read_frags(const uint8_t* __restrict__ st, int a
         }
 }
 
-// One step: 8 MFMAs.  The empty asm keeps each operand in six consecutive registers here.
+// One step: 8 MFMAs; TRANS: the accumulators hold the transposed block, same values.  The empty
+// asm keeps each operand in six consecutive registers here.
+template <bool TRANS>
 __device__ __forceinline__ void mfma_step(Frags& fa, Frags& fb, v16f (&re)[2][2], v16f (&im)[2][2]) {
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
@@ -102,8 +104,10 @@ __device__ __forceinline__ void mfma_step(Frags& fa, Frags& fb, v16f (&re)[2][2]
         const v6i v = conj6(fa[x]);
 #pragma unroll
         for (int y = 0; y < 2; ++y) {
-            re[x][y] = mfma_32x32x64<OPF_BF6>(op8(fa[x]), op8(fb[y]), re[x][y]);
-            im[x][y] = mfma_32x32x64<OPF_BF6>(op8(v), op8(fb[y]), im[x][y]);
+            re[x][y] = TRANS ? mfma_32x32x64<OPF_BF6>(op8(fb[y]), op8(fa[x]), re[x][y])
+                             : mfma_32x32x64<OPF_BF6>(op8(fa[x]), op8(fb[y]), re[x][y]);
+            im[x][y] = TRANS ? mfma_32x32x64<OPF_BF6>(op8(fb[y]), op8(v), im[x][y])
+                             : mfma_32x32x64<OPF_BF6>(op8(v), op8(fb[y]), im[x][y]);
         }
     }
 }
@@ -124,7 +128,7 @@ __device__ __forceinline__ void copy_stage(__amdgpu_buffer_rsrc_t rows, int at, 
 // ago) multiplies, the next stage's first step while the second one does.  The copies of
 // stage s + 2 go into `fre`, the buffer of stage s - 1, which every wave finished reading
 // before this stage's barrier.
-template <bool ACTIVE>
+template <bool ACTIVE, bool TRANS>
 __device__ __forceinline__ void stage_body(const uint8_t* __restrict__ cur, const uint8_t* __restrict__ nxt,
                                            uint8_t* __restrict__ fre, __amdgpu_buffer_rsrc_t rows, int at,
                                            const uint32_t (&off)[P_LOADS], int lane, int wave, int a, int b, Frags& a0,
@@ -134,17 +138,17 @@ __device__ __forceinline__ void stage_body(const uint8_t* __restrict__ cur, cons
         read_frags(cur, a, b, lane, 1, a1, b1);
         __builtin_amdgcn_sched_barrier(0);
         wait_lgkm<8>();  // all but the eight reads just issued
-        mfma_step(a0, b0, re, im);
+        mfma_step<TRANS>(a0, b0, re, im);
         __builtin_amdgcn_sched_barrier(0);
         read_frags(nxt, a, b, lane, 0, a0, b0);
         __builtin_amdgcn_sched_barrier(0);
         wait_lgkm<8>();
-        mfma_step(a1, b1, re, im);
+        mfma_step<TRANS>(a1, b1, re, im);
         __builtin_amdgcn_sched_barrier(0);
     }
 }
 
-template <bool ACTIVE>
+template <bool ACTIVE, bool TRANS>
 __device__ __forceinline__ void tile_loop(__amdgpu_buffer_rsrc_t rows, uint8_t* lds, int nst,
                                           const uint32_t (&off)[P_LOADS], int lane, int wave, int a, int b,
                                           v16f (&re)[2][2], v16f (&im)[2][2]) {
@@ -162,8 +166,8 @@ __device__ __forceinline__ void tile_loop(__amdgpu_buffer_rsrc_t rows, uint8_t* 
         const int n = c == P_BUFS - 1 ? 0 : c + 1, f = c == 0 ? P_BUFS - 1 : c - 1;
         // past the end the last stage is copied again, into a buffer that is not read
         const int t = s + 2 < nst ? s + 2 : nst - 1;
-        stage_body<ACTIVE>(lds + c * P_STAGE, lds + n * P_STAGE, lds + f * P_STAGE, rows, t * SRC, off, lane, wave, a,
-                           b, a0, b0, a1, b1, re, im);
+        stage_body<ACTIVE, TRANS>(lds + c * P_STAGE, lds + n * P_STAGE, lds + f * P_STAGE, rows, t * SRC, off, lane,
+                                  wave, a, b, a0, b0, a1, b1, re, im);
         c = n;
     }
     wait_vm<0>();  // no copy may land after the workgroup's LDS is given back
@@ -223,6 +227,69 @@ __device__ __forceinline__ void store_any(OutT* C, int N, int w, int col, float 
         }
 }
 
+// ---- GGP layouts (herk_tile.h), from the transposed accumulators: lane = row i ----
+// Block x, y, register q: i = w + 32 x + lane % 32, j = col + 32 y + 8 (q / 4) + 4 (lane / 32) + q % 4.
+// Upper packed rows (j, i >= j) are 32-lane runs, so is the upper half of the full matrix; its
+// lower half takes the four consecutive j of a lane at a time, which the L2 joins to lines.
+template <typename OutT, int FMT>
+__device__ __forceinline__ void store_ggp_inside(OutT* C, int N, int w, int col, const v16f (&re)[2][2],
+                                                 const v16f (&im)[2][2], int lane) {
+    typedef typename Elem<OutT>::v2 v2;
+    constexpr uint32_t ES = sizeof(v2);
+    constexpr bool TRI = FMT == OUT_UPPER_PACKED;
+    const int n = lane & 31, g4 = (lane >> 5) * 4;
+    const int64_t row = (int64_t)col * N - (TRI ? (int64_t)col * (col + 1) / 2 : 0);
+    uint8_t* base = reinterpret_cast<uint8_t*>(reinterpret_cast<v2*>(C) + row + w);
+    // row col + d starts d (N - col) - d (d + 1) / 2 elements on (TRI), d N (full)
+    const uint32_t pitch = (uint32_t)(N - (TRI ? col + g4 : 0)) * ES;  // row d + g4 -> d + 1 + g4: less (d + 1) ES
+    uint32_t off = (uint32_t)(TRI ? g4 * (N - col) - g4 * (g4 + 1) / 2 + n : g4 * N + n) * ES;
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int d = y * 32 + (q >> 2) * 8 + (q & 3);
+            v2* p = reinterpret_cast<v2*>(base + off);
+#pragma unroll
+            for (int x = 0; x < 2; ++x) p[x * 32] = Elem<OutT>::make(re[x][y][q], im[x][y][q]);
+            const bool next = (q & 3) != 3;
+            off += (next ? 1u : 5u) * pitch - (TRI ? (uint32_t)(next ? d + 1 : 5 * d + 15) * ES : 0u);
+        }
+    if constexpr (FMT == OUT_HERM_FULL) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            v2* p = reinterpret_cast<v2*>(C) + (int64_t)(w + x * 32 + n) * N + col + g4;
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int q = 0; q < 16; ++q)
+                    p[y * 32 + (q >> 2) * 8 + (q & 3)] = Elem<OutT>::make(re[x][y][q], -im[x][y][q]);
+        }
+    }
+}
+
+template <typename OutT, int FMT>
+__device__ __forceinline__ void store_ggp_any(OutT* C, int N, int w, int col, const v16f (&re)[2][2],
+                                              const v16f (&im)[2][2], int lane) {
+    typedef typename Elem<OutT>::v2 v2;
+    const int n = lane & 31, g4 = (lane >> 5) * 4;
+    v2* base = reinterpret_cast<v2*>(C);
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int j = col + y * 32 + (q >> 2) * 8 + g4 + (q & 3);
+            v2* row = base + ((int64_t)j * N - (FMT == OUT_UPPER_PACKED ? (int64_t)j * (j + 1) / 2 : 0));
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                const int i = w + x * 32 + n;
+                if (i >= N || j > i) continue;
+                const float r = re[x][y][q], m = i == j ? 0.0f : im[x][y][q];
+                row[i] = Elem<OutT>::make(r, m);
+                if (FMT == OUT_HERM_FULL && i != j) base[(int64_t)i * N + j] = Elem<OutT>::make(r, -m);
+            }
+        }
+}
+
 // Tile t of the lower triangle of nb x nb tiles, in square blocks of H x H tiles (row-major
 // inside a block, blocks row-major): the tiles that one XCD runs together then share H row and
 // H column blocks in its L2 instead of one and many.
@@ -247,8 +314,8 @@ __device__ __forceinline__ void tri_decode_blocked(int t, int nb, int H, int& I,
     }
 }
 
-// Tile (I, J) of one problem: `base` its fragment rows, `steps` per row.
-template <typename OutT>
+// Tile (I, J) of one problem: `base` its fragment rows, `steps` per row.  GGP layouts: alpha 1, beta 0.
+template <typename OutT, int FMT = OUT_LOWER_PACKED>
 __device__ __forceinline__ void pipe_tile(uint8_t* lds, const uint8_t* base, int N, int steps, int I, int J, OutT* C,
                                           float alpha, float beta, bool nt) {
     // wave index in an SGPR: the conditions on it are scalar branches
@@ -279,11 +346,15 @@ __device__ __forceinline__ void pipe_tile(uint8_t* lds, const uint8_t* base, int
             }
     const int a = wm * 2 * P_GSTRIDE, bo = (P_GROUPS / 2 + wn * 2) * P_GSTRIDE;
     if (!active) {
-        tile_loop<false>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
+        tile_loop<false, false>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
         return;
     }
-    tile_loop<true>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
-    if (wcol + 63 < wrow && wrow + 64 <= N && beta == 0.0f) {
+    tile_loop<true, FMT != OUT_LOWER_PACKED>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
+    const bool inside = wcol + 63 < wrow && wrow + 64 <= N;
+    if constexpr (FMT != OUT_LOWER_PACKED) {
+        if (inside) store_ggp_inside<OutT, FMT>(C, N, wrow, wcol, re, im, lane);
+        else store_ggp_any<OutT, FMT>(C, N, wrow, wcol, re, im, lane);
+    } else if (inside && beta == 0.0f) {
         if (nt) {
             if (alpha == 1.0f) store_inside<OutT, false, true>(C, wrow, wcol, alpha, re, im, lane);
             else store_inside<OutT, true, true>(C, wrow, wcol, alpha, re, im, lane);
@@ -296,15 +367,15 @@ __device__ __forceinline__ void pipe_tile(uint8_t* lds, const uint8_t* base, int
     }
 }
 
-template <typename OutT, bool NT>
+template <typename OutT, bool NT, int FMT = OUT_LOWER_PACKED>
 __global__ void __launch_bounds__(P_THREADS, 2) herk_pipe_kernel(HerkPlainArgs p, int steps, int tiles) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[P_BUFS * P_STAGE];
     const int w = xcd_logical((int)blockIdx.x, tiles * p.batch);
     const int b = w / tiles, t = w - b * tiles;
     int I, J;
     tri_decode_blocked(t, (p.N + PT - 1) / PT, P_BLOCK, I, J);
-    pipe_tile<OutT>(lds, p.A + (int64_t)b * p.a_bstride, p.N, steps, I, J,
-                    static_cast<OutT*>(p.C) + (int64_t)b * p.c_bstride, p.alpha, p.beta, NT);
+    pipe_tile<OutT, FMT>(lds, p.A + (int64_t)b * p.a_bstride, p.N, steps, I, J,
+                         static_cast<OutT*>(p.C) + (int64_t)b * p.c_bstride, p.alpha, p.beta, NT);
 }
 
 // Tiles of many problems: workgroup b runs tiles[b].
@@ -344,19 +415,34 @@ __device__ __forceinline__ void pack16(const uint32_t (&c)[4], uint32_t& d0, uin
     d2 = (p2 >> 16) | (p3 << 8);
 }
 
-// 16 samples -> their place in the fragment step at dst (lane as in herk_pipe.h)
-__device__ __forceinline__ void put_frag(uint4 w, uint8_t* dst, int lane) {
-    uint32_t re[4], im[4];
-    qc4_codes(w.x, re[0], im[0]);
-    qc4_codes(w.y, re[1], im[1]);
-    qc4_codes(w.z, re[2], im[2]);
-    qc4_codes(w.w, re[3], im[3]);
+// Four two's complement nibbles, one per byte -> their E3M2 codes: a 16-entry table over two
+// lookups (0 .. 7, -8 .. -1) and a select on bit 3.
+__device__ __forceinline__ uint32_t ggp_nib4_codes(uint32_t nib) {
+    const uint32_t sel = nib & 0x07070707u;
+    const uint32_t pos = __builtin_amdgcn_perm(0x17161514u, 0x12100C00u, sel);  // 4 .. 7, 0 .. 3
+    const uint32_t neg = __builtin_amdgcn_perm(0x2C303234u, 0x35363738u, sel);  // -4 .. -1, -8 .. -5
+    const uint32_t m = ((nib >> 3) & 0x01010101u) * 0xFFu;
+    return (pos & ~m) | (neg & m);
+}
+
+// 16 samples' codes -> their place in the fragment step at dst (lane as in herk_pipe.h)
+__device__ __forceinline__ void put_codes(const uint32_t (&re)[4], const uint32_t (&im)[4], uint8_t* dst, int lane) {
     uint4 a;
     uint2 b;
     pack16(re, a.x, a.y, a.z);
     pack16(im, a.w, b.x, b.y);
     *reinterpret_cast<uint4*>(dst + lane * 16) = a;
     *reinterpret_cast<uint2*>(dst + 1024 + lane * 8) = b;
+}
+
+// 16 QC samples -> their place in the fragment step at dst 
+__device__ __forceinline__ void put_frag(uint4 w, uint8_t* dst, int lane) {
+    uint32_t re[4], im[4];
+    qc4_codes(w.x, re[0], im[0]);
+    qc4_codes(w.y, re[1], im[1]);
+    qc4_codes(w.z, re[2], im[2]);
+    qc4_codes(w.w, re[3], im[3]);
+    put_codes(re, im, dst, lane);
 }
 
 // Row and 16-sample segment of conversion thread t: waves of S segments x 64 / S rows.
@@ -417,6 +503,62 @@ qc_frag_rows_multi_kernel(const PipeProblem* __restrict__ probs, const ConvBlock
         }
         put_frag(w, p.rows + ((int64_t)(r >> 5) * p.steps + (s >> 1)) * kFragBytes, (r & 31) + 32 * (s & 1));
     }
+}
+
+// GGP bytes [batch][K][N] (low nibble Re, high Im, two's complement) -> fragment rows.  A thread
+// converts 16 samples of four rows; in a wave 16 lanes run along the rows (64-byte reads of
+// each sample's run, 1-kilobyte runs of a group's operands) and 4 along the samples.
+// ALIGNED: N % 4 == 0 and 4-byte aligned input.
+template <bool ALIGNED>
+__global__ void __launch_bounds__(256)
+ggp_frag_rows_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int N, int K, int steps, int batches) {
+    const int tid = threadIdx.x, ng = (N + 31) / 32;
+    const int r0 = ((int)blockIdx.y * 64 + (tid & 15) + 16 * (tid >> 6)) * 4;
+    const int s = (int)blockIdx.x * 4 + ((tid >> 4) & 3);  // whole stages: s < 2 steps
+    if (r0 >= ng * 32) return;
+    for (int b = blockIdx.z; b < batches; b += gridDim.z) {
+        const uint8_t* src = in + (int64_t)b * K * N + r0;
+        uint32_t d[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int k = s * 16 + e;
+            uint32_t v = 0u;
+            if (k < K && r0 < N) {
+                const uint8_t* run = src + (int64_t)k * N;
+                if (ALIGNED) {
+                    v = *reinterpret_cast<const uint32_t*>(run);
+                } else {
+#pragma unroll
+                    for (int a = 0; a < 4; ++a)
+                        if (r0 + a < N) v |= (uint32_t)run[a] << (8 * a);
+                }
+            }
+            d[e] = v;
+        }
+        uint32_t t[4][4];  // [sample quad][row]
+#pragma unroll
+        for (int g = 0; g < 4; ++g) transpose4x4_bytes(d[4 * g], d[4 * g + 1], d[4 * g + 2], d[4 * g + 3], t[g]);
+        uint8_t* dst = out + (((int64_t)b * ng + (r0 >> 5)) * steps + (s >> 1)) * kFragBytes;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            uint32_t re[4], im[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                re[g] = ggp_nib4_codes(t[g][a] & 0x0F0F0F0Fu);
+                im[g] = ggp_nib4_codes((t[g][a] >> 4) & 0x0F0F0F0Fu);
+            }
+            put_codes(re, im, dst, ((r0 + a) & 31) + 32 * (s & 1));
+        }
+    }
+}
+
+template <typename OutT>
+void launch_ggp(const HerkPlainArgs& a, int fmt, int steps, int tiles, hipStream_t stream) {
+    const dim3 grid((unsigned)((int64_t)tiles * a.batch)), block(P_THREADS);
+    if (fmt == OUT_UPPER_PACKED)
+        hipLaunchKernelGGL((herk_pipe_kernel<OutT, false, OUT_UPPER_PACKED>), grid, block, 0, stream, a, steps, tiles);
+    else
+        hipLaunchKernelGGL((herk_pipe_kernel<OutT, false, OUT_HERM_FULL>), grid, block, 0, stream, a, steps, tiles);
 }
 
 }  // namespace
@@ -501,6 +643,26 @@ hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t s
         else
             hipLaunchKernelGGL((herk_pipe_kernel<float, false>), grid, block, 0, stream, a, steps, tiles);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_ggp_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, int batches, hipStream_t stream) {
+    if (N <= 0 || K <= 0 || batches <= 0) return hipSuccess;
+    const int steps = frag_steps(K);
+    const dim3 grid((unsigned)(steps / 2), (unsigned)((N + 255) / 256), (unsigned)(batches < 65535 ? batches : 65535));
+    if (N % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 3u) == 0)
+        hipLaunchKernelGGL(ggp_frag_rows_kernel<true>, grid, dim3(256), 0, stream, in, out, N, K, steps, batches);
+    else
+        hipLaunchKernelGGL(ggp_frag_rows_kernel<false>, grid, dim3(256), 0, stream, in, out, N, K, steps, batches);
+    return hipGetLastError();
+}
+
+hipError_t launch_herk_pipe_ggp(const HerkPlainArgs& a, int fmt, bool out_fp64, hipStream_t stream) {
+    if (a.N <= 0 || a.batch <= 0) return hipSuccess;
+    const int tiles = pipe_tiles(a.N), steps = frag_steps(a.K);
+    if ((int64_t)tiles * a.batch > 0x7FFFFFFF || !pipe_supported(a.N, a.K)) return hipErrorInvalidValue;
+    if (out_fp64) launch_ggp<double>(a, fmt, steps, tiles, stream);
+    else launch_ggp<float>(a, fmt, steps, tiles, stream);
     return hipGetLastError();
 }
 

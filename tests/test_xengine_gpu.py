@@ -70,6 +70,32 @@ def test_xengine_every_tile_config(oracle, dev, cfg, fmt, n_time):
     xe.close()
 
 
+# one row group (32), tile (128) and stage (64) to either side, unaligned input runs (N % 4), and
+# enough tiles for the full FP64 matrix to take the pipelined kernel (64)
+@pytest.mark.parametrize("n_ant,K,batch", [(1, 16, 3), (31, 17, 2), (33, 64, 1), (127, 63, 2), (128, 65, 1),
+                                           (129, 33, 22), (191, 128, 22), (260, 192, 11)])
+@pytest.mark.parametrize("prec", ["single", "double"])
+@pytest.mark.parametrize("fmt", ["tri", "herm"])
+def test_xengine_fragment_row_edges(oracle, dev, n_ant, K, batch, prec, fmt):
+    import torch
+    from ftd_amd import ftdx
+    qp = ftdx.QPREC_SINGLE if prec == "single" else ftdx.QPREC_DOUBLE
+    mf = ftdx.XENGINE_MAT_TRI if fmt == "tri" else ftdx.XENGINE_MAT_HERM
+    xe = ftdx.XEngine(_param(ftdx, n_ant, batch, K, 1, 1, qp, mf, loc=ftdx.LOCATION_DEVICE))
+    data = oracle.gen_bytes(n_ant + K, xe.in_payload_bytes)
+    dt, it = (torch.float32, torch.int32) if prec == "single" else (torch.float64, torch.int64)
+    n_out = xe.out_payload_bytes // (4 if prec == "single" else 8)
+    out, tile = (torch.full((n_out,), float("nan"), dtype=dt, device=dev) for _ in range(2))
+    A = torch.from_numpy(data).to(dev)
+    xe.compute(out, A)
+    ref = _oracle_payloads(oracle, data, xe, 1, fmt == "herm")[0]
+    assert np.array_equal(out.cpu().numpy().reshape(ref.shape), ref.astype(out.cpu().numpy().dtype))
+    xe.set_launch_config(2, 1)  # the FP8 tile kernel: every bit alike, signs of zero too
+    xe.compute(tile, A)
+    assert torch.equal(out.view(it), tile.view(it))
+    xe.close()
+
+
 def _torch_gram(data, B, K, N):
     import torch
     d = data.reshape(B, K, N)
