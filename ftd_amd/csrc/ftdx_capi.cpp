@@ -21,6 +21,7 @@
 #include "herk_fp8.h"
 #include "herk_mx.h"
 #include "herk_direct.h"
+#include "herk_mxpipe.h"
 #include "herk_pipe.h"
 #include "calib.h"
 #include "stages.h"
@@ -194,8 +195,8 @@ int device_cu_count() {
 constexpr size_t kPrecastChunkBytes = size_t(320) << 20;
 
 // batches of `per` scratch bytes each that fit one chunk
-int chunk_cap_bytes(size_t per, int batch) {
-    const size_t cap = per > 0 ? kPrecastChunkBytes / per : (size_t)batch;
+int chunk_cap_bytes(size_t per, int batch, size_t limit = kPrecastChunkBytes) {
+    const size_t cap = per > 0 ? limit / per : (size_t)batch;
     return (int)std::max<size_t>(1, std::min<size_t>(cap, (size_t)std::max(batch, 1)));
 }
 
@@ -343,8 +344,7 @@ constexpr size_t kFragChunkBytes = size_t(160) << 20;
 
 int frag_chunk_cap(int N, int K, int nseg, int batch) {
     const size_t per = (size_t)frag_rows_bytes(N, K, nseg);
-    const int cap = (int)std::max<size_t>(1, std::min<size_t>(kFragChunkBytes / per, (size_t)std::max(batch, 1)));
-    return std::min(cap, 65535 / std::max(nseg, 1));
+    return std::min(chunk_cap_bytes(per, batch, kFragChunkBytes), 65535 / std::max(nseg, 1));
 }
 
 size_t frag_scratch_bytes(const HerkPlainArgs& a) {
@@ -401,6 +401,44 @@ hipError_t run_pipe(uint8_t* rows, const HerkPlainArgs& a, bool fp16, hipStream_
         b.batch = nu * grp;
         b.a_bstride = frag_rows_bytes(a.N, a.K, a.nseg);
         if ((e = launch_herk_pipe(b, fp16, st)) != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+// ---- block-scaled HERK over operand fragments (herk_mxpipe.h) ----
+// The pipelined kernel is the faster one at every size tried, with the same bits (us, tile / pipelined):
+//   E3M2   33 x 1, K 100  16 / 14    256 x 2, K 4096  90 / 59   1024 x 32, K 1024  141 / 114
+//        4096 x 8, K 256 178 / 149  4096 x 8, K 4096 1060 / 902
+//   E2M1   33 x 1, K 100  15 / 13    256 x 2, K 4096  62 / 46   1024 x 32, K 1024  118 / 95
+//        4096 x 8, K 256 174 / 141  4096 x 8, K 4096  738 / 686
+// (chunks of 320 MB, or all in one; of 160 MB: 929 and 695 in the last rows).  Not where a batch's
+// fragments (groups of 32 rows) take 64 MB more than the tile kernel's rows of the whole call.
+bool mxpipe_takes(int N, int K, int batch, int fmt) {
+    return mxpipe_supported(N, K, fmt) && (int64_t)pipe_tiles(N) * batch <= 0x7FFFFFFF &&
+           mxfrag_rows_bytes(N, K, fmt) <= (int64_t)N * batch * mx_padded_blocks(K) * 64 + (64 << 20);
+}
+
+// Quantizes and multiplies chunk by chunk, as run_pipe; rows: cap batches of fragments.
+hipError_t run_mxpipe(uint8_t* rows, const void* A, void* C, int N, int K, int batch, int cap, int input, int fmt,
+                      int rounding, bool fp16, float alpha, float beta, hipStream_t s) {
+    const int64_t slots = (int64_t)std::max(device_cu_count(), 1) * pipe_wg_per_cu();
+    const int chunk = pick_chunk_of(slots, pipe_tiles(N), batch, cap);
+    HerkPlainArgs a{};
+    a.A = rows;
+    a.N = N;
+    a.K = K;
+    a.alpha = alpha;
+    a.beta = beta;
+    a.a_bstride = mxfrag_rows_bytes(N, K, fmt);
+    a.c_bstride = (int64_t)N * (N + 1);
+    for (int b0 = 0; b0 < batch; b0 += chunk) {
+        a.batch = std::min(chunk, batch - b0);
+        a.C = static_cast<uint8_t*>(C) + (int64_t)b0 * a.c_bstride * (fp16 ? 2 : 4);
+        const uint8_t* src = static_cast<const uint8_t*>(A) + (int64_t)b0 * N * K * (input == FTDX_INPUT_FP16 ? 4 : 1);
+        hipError_t e = launch_mx_frag_rows(src, input == FTDX_INPUT_INT4 ? MX_IN_INT4 : MX_IN_FP16, fmt, rounding, rows,
+                                           N, K, a.batch, s);
+        if (e == hipSuccess) e = launch_herk_mxpipe(a, fmt, fp16, s);
+        if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
@@ -1017,6 +1055,15 @@ int ftdx_herk_mx(ftdx_context* ctx, const void* A, void* C, int N, int K, int ba
     const int remap = ctx->forced_remap >= 0 ? ctx->forced_remap : ftdx::kDefaultRemap;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int fmt = ftdx::mx_format(compute);
+    if (ctx->forced_cfg < 0 && ftdx::mxpipe_takes(N, K, batch_count, fmt)) {
+        const int64_t per = ftdx::mxfrag_rows_bytes(N, K, fmt);
+        const int cap = std::min(ftdx::chunk_cap_bytes((size_t)per, batch_count), 65535);
+        int rc = ftdx::ensure_scratch(ctx->mx_codes, ctx->mx_codes_cap, (size_t)per * cap, "ftdx_herk_mx: scratch");
+        if (rc != FTDX_OK) return rc;
+        e = ftdx::run_mxpipe(ctx->mx_codes, A, C, N, K, batch_count, cap, input, fmt, ctx->mx_rounding,
+                             output == FTDX_OUTPUT_FP16, alpha, beta, s);
+        return e == hipSuccess ? FTDX_OK : hip_fail(e, "ftdx_herk_mx: kernel launch");
+    }
     // E2M1 on a configuration whose tiles are all interior: dense rows (32 bytes per
     // block, scales apart), twice the samples per stage of the inline-scale rows.
     const int nblkd = ftdx::mx_dense_blocks(K);

@@ -34,6 +34,7 @@
 
 #include "herk_common.h"
 #include "herk_mx.h"
+#include "herk_mxpipe.h"
 #include "herk_tile.h"
 
 namespace ftdx {
@@ -110,31 +111,11 @@ __device__ __forceinline__ float qc_nibble_value(uint32_t n) {
     return (float)((n & 8u) ? -m : m);
 }
 
-// One thread per (row, 32-sample block): reads 32 complex samples, writes the
-// Re and Im code blocks and their two scale bytes.  Blocks past K (and the
-// padding block) quantize as zeros with scale 0.
-// MX_IN_FP16_PLANAR: X holds the Re halves, X2 the Im halves, both [rows][K].  conj:
-// the Im codes are stored negated (sign bit flipped after encoding, which is exact
-// since the encoding is symmetric), i.e. the codes of conj(X).
-// ROWS: the operand-row layout of the HERK tile instead (codes = rows, scales unused):
-// per (row, block) the Re part then the Im part, 32 bytes each: codes, scale byte, zeros.
-// DENSE (E2M1, with ROWS): codes = rows [rows][nblkp][2][16] (the 16 code bytes of the Re
-// part, then of the Im part), scales = [rows / nrow][nblkp / 4][nrow][8]: per stage of 4
-// blocks, each row's (Re, Im) scale bytes of those blocks.
-template <int FMT, int IN, int RND, bool ROWS = false, bool DENSE = false>
-__global__ void __launch_bounds__(256) mx_quantize_kernel(const void* __restrict__ X,
-                                                          const void* __restrict__ X2,
-                                                          uint8_t* __restrict__ codes,
-                                                          uint8_t* __restrict__ scales,
-                                                          int64_t rows, int K, int nblkp, int conj, int vec,
-                                                          int64_t nrow = 0) {
-    using F = MxFmt<FMT>;
-    const int64_t total = rows * nblkp;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    float v[2][32];
-    if (t >= total) return;
-    const int64_t row = t / nblkp;
-    const int blk = (int)(t - row * nblkp);
+// The 32 samples of block blk of a row: Re to v[0], Im to v[1]; zeros past K.  vec: rows of whole
+// 16-byte units, 16-byte aligned.
+template <int IN>
+__device__ __forceinline__ void mx_load_block(const void* __restrict__ X, const void* __restrict__ X2, int64_t row,
+                                              int blk, int K, int vec, float (&v)[2][32]) {
     if (vec && blk * 32 + 32 <= K) {
         // whole block, 16-byte aligned rows: wide loads of the block's contiguous bytes
         if constexpr (IN == MX_IN_INT4) {
@@ -209,49 +190,86 @@ __global__ void __launch_bounds__(256) mx_quantize_kernel(const void* __restrict
         v[1][i] = im;
     }
     }
+}
+
+// One part of a block -> its packed codes; returns the scale byte.
+template <int FMT, int RND>
+__device__ __forceinline__ uint32_t mx_encode_block(const float (&v)[32], uint32_t (&w)[6]) {
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[i]));
+    const uint32_t se = mx_scale_exponent<FMT>(amax);
+    const float inv = __builtin_ldexpf(1.0f, 127 - (int)se);
+    // v * inv is exact (a power of two within range); then either the reference's
+    // converter per element, or the gfx950 converters, which round to nearest even
+    // with subnormals and saturate (the OCP MX element rule)
+#pragma unroll
+    for (int d = 0; d < 6; ++d) w[d] = 0u;
+    if constexpr (RND == MX_ROUND_REFERENCE) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) {
+            const uint32_t c = ref_element_code<FMT>(v[i] * inv);
+            if constexpr (FMT == MX_FP4_E2M1) {
+                w[i >> 3] |= c << (4 * (i & 7));
+            } else {
+                const int p = 6 * i;
+                w[p >> 5] |= c << (p & 31);
+                if ((p & 31) > 26) w[(p >> 5) + 1] |= c >> (32 - (p & 31));
+            }
+        }
+    } else if constexpr (FMT == MX_FP4_E2M1) {
+#pragma unroll
+        for (int i = 0; i < 32; i += 2) {
+            const uint32_t b = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v[i] * inv, v[i + 1] * inv,
+                                                                        1.0f, 0) & 0xFFu;
+            w[i >> 3] |= b << (4 * (i & 7));
+        }
+    } else {
+        // the 2 x 16 form interleaves its sources: code 2i from the first, 2i + 1 from
+        // the second, code k at bits 6k .. 6k + 5
+        v16f ev, od;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            ev[i] = v[2 * i] * inv;
+            od[i] = v[2 * i + 1] * inv;
+        }
+        const v6i c = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, 1.0f);
+#pragma unroll
+        for (int d = 0; d < 6; ++d) w[d] = (uint32_t)c[d];
+    }
+    return se;
+}
+
+// One thread per (row, 32-sample block): reads 32 complex samples, writes the
+// Re and Im code blocks and their two scale bytes.  Blocks past K (and the
+// padding block) quantize as zeros with scale 0.
+// MX_IN_FP16_PLANAR: X holds the Re halves, X2 the Im halves, both [rows][K].  conj:
+// the Im codes are stored negated (sign bit flipped after encoding, which is exact
+// since the encoding is symmetric), i.e. the codes of conj(X).
+// ROWS: the operand-row layout of the HERK tile instead (codes = rows, scales unused):
+// per (row, block) the Re part then the Im part, 32 bytes each: codes, scale byte, zeros.
+// DENSE (E2M1, with ROWS): codes = rows [rows][nblkp][2][16] (the 16 code bytes of the Re
+// part, then of the Im part), scales = [rows / nrow][nblkp / 4][nrow][8]: per stage of 4
+// blocks, each row's (Re, Im) scale bytes of those blocks.
+template <int FMT, int IN, int RND, bool ROWS = false, bool DENSE = false>
+__global__ void __launch_bounds__(256) mx_quantize_kernel(const void* __restrict__ X,
+                                                          const void* __restrict__ X2,
+                                                          uint8_t* __restrict__ codes,
+                                                          uint8_t* __restrict__ scales,
+                                                          int64_t rows, int K, int nblkp, int conj, int vec,
+                                                          int64_t nrow = 0) {
+    using F = MxFmt<FMT>;
+    const int64_t total = rows * nblkp;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    float v[2][32];
+    if (t >= total) return;
+    const int64_t row = t / nblkp;
+    const int blk = (int)(t - row * nblkp);
+    mx_load_block<IN>(X, X2, row, blk, K, vec, v);
 #pragma unroll
     for (int part = 0; part < 2; ++part) {
-        float amax = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[part][i]));
-        const uint32_t se = mx_scale_exponent<FMT>(amax);
-        const float inv = __builtin_ldexpf(1.0f, 127 - (int)se);
-        // v * inv is exact (a power of two within range); then either the reference's
-        // converter per element, or the gfx950 converters, which round to nearest even
-        // with subnormals and saturate (the OCP MX element rule)
-        uint32_t w[6] = {0u, 0u, 0u, 0u, 0u, 0u};
-        if constexpr (RND == MX_ROUND_REFERENCE) {
-#pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                const uint32_t c = ref_element_code<FMT>(v[part][i] * inv);
-                if constexpr (FMT == MX_FP4_E2M1) {
-                    w[i >> 3] |= c << (4 * (i & 7));
-                } else {
-                    const int p = 6 * i;
-                    w[p >> 5] |= c << (p & 31);
-                    if ((p & 31) > 26) w[(p >> 5) + 1] |= c >> (32 - (p & 31));
-                }
-            }
-        } else if constexpr (FMT == MX_FP4_E2M1) {
-#pragma unroll
-            for (int i = 0; i < 32; i += 2) {
-                const uint32_t b = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v[part][i] * inv, v[part][i + 1] * inv,
-                                                                            1.0f, 0) & 0xFFu;
-                w[i >> 3] |= b << (4 * (i & 7));
-            }
-        } else {
-            // the 2 x 16 form interleaves its sources: code 2i from the first, 2i + 1 from
-            // the second, code k at bits 6k .. 6k + 5
-            v16f ev, od;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                ev[i] = v[part][2 * i] * inv;
-                od[i] = v[part][2 * i + 1] * inv;
-            }
-            const v6i c = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, 1.0f);
-#pragma unroll
-            for (int d = 0; d < 6; ++d) w[d] = (uint32_t)c[d];
-        }
+        uint32_t w[6];
+        const uint32_t se = mx_encode_block<FMT, RND>(v[part], w);
         if constexpr (DENSE) {
             static_assert(FMT == MX_FP4_E2M1 && ROWS, "dense rows are E2M1 operand rows");
             uint32_t o[4];
@@ -275,6 +293,61 @@ __global__ void __launch_bounds__(256) mx_quantize_kernel(const void* __restrict
             scales[(row * nblkp + blk) * 2 + part] = (uint8_t)se;
         }
     }
+}
+
+// Operand fragments for the pipelined MX HERK (layout: herk_mxpipe.h).  A wave takes 8 (or 2)
+// blocks of 8 (or 32) rows: reads of 1 KB runs, writes of 128-byte runs.  A thread's two scale
+// bytes meet its neighbour block's in one 2-byte store each.
+template <int FMT, int IN, int RND, int S>
+__global__ void __launch_bounds__(256)
+mx_frag_rows_kernel(const void* __restrict__ X, uint8_t* __restrict__ out, int N, int K, int nblkp, int vec) {
+    constexpr int FB = mxfrag_bytes(FMT), R = 64 / S;
+    const int ng = (N + 31) / 32;
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x, u = t / 64u, per = (uint32_t)(nblkp / S);
+    const uint32_t rb = u / per;
+    const int blk = (int)(u - rb * per) * S + (int)(t % S), r = (int)rb * R + (int)(t / S % R);
+    if (r >= ng * 32) return;  // whole waves: 32 rows are a multiple of R
+    float v[2][32];
+    if (r < N) {
+        mx_load_block<IN>(X, nullptr, (int64_t)blockIdx.y * N + r, blk, K, vec, v);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) v[0][i] = v[1][i] = 0.0f;
+    }
+    uint8_t* stage = out + (((int64_t)blockIdx.y * ng + (r >> 5)) * (nblkp / 2) + (blk >> 1)) * (2 * FB + 128);
+    uint32_t se[2];
+#pragma unroll
+    for (int part = 0; part < 2; ++part) {
+        uint32_t w[6];
+        se[part] = mx_encode_block<FMT, RND>(v[part], w);
+        uint8_t* frag = stage + (blk & 1) * FB;
+        const int lane = (r & 31) + 32 * part;
+        *reinterpret_cast<uint4*>(frag + lane * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+        if constexpr (FMT == MX_FP6_E3M2) *reinterpret_cast<uint2*>(frag + 1024 + lane * 8) = make_uint2(w[4], w[5]);
+    }
+    const uint32_t mine = se[0] | (se[1] << 8), other = (uint32_t)__shfl_xor((int)mine, 1);
+    const int odd = blk & 1;  // block parity = lane parity; the even lane stores Re, the odd one Im
+    const uint32_t lo = odd ? other >> 8 : mine & 0xFFu, hi = odd ? mine >> 8 : other & 0xFFu;
+    *reinterpret_cast<uint16_t*>(stage + 2 * FB + ((r & 31) + 32 * odd) * 2) = (uint16_t)(lo | (hi << 8));
+}
+
+template <int FMT, int IN, int RND>
+void frag_rows(const void* X, uint8_t* out, int N, int K, int batches, int nblkp, int vec, hipStream_t s) {
+    const int64_t threads = (int64_t)((N + 31) / 32) * 32 * nblkp;
+    const dim3 grid((unsigned)((threads + 255) / 256), (unsigned)batches);
+    if (nblkp % 8 == 0)
+        hipLaunchKernelGGL((mx_frag_rows_kernel<FMT, IN, RND, 8>), grid, dim3(256), 0, s, X, out, N, K, nblkp, vec);
+    else
+        hipLaunchKernelGGL((mx_frag_rows_kernel<FMT, IN, RND, 2>), grid, dim3(256), 0, s, X, out, N, K, nblkp, vec);
+}
+
+template <int FMT, int IN>
+void frag_rows_rnd(const void* X, uint8_t* out, int rounding, int N, int K, int batches, int nblkp, int vec,
+                   hipStream_t s) {
+    if (rounding == MX_ROUND_REFERENCE)
+        frag_rows<FMT, IN, MX_ROUND_REFERENCE>(X, out, N, K, batches, nblkp, vec, s);
+    else
+        frag_rows<FMT, IN, MX_ROUND_NEAREST_EVEN>(X, out, N, K, batches, nblkp, vec, s);
 }
 
 constexpr int MX_BLK_PER_STAGE = 2;  // 32-sample blocks per 64-sample tile stage
@@ -375,6 +448,24 @@ hipError_t launch_mx_quantize_dense(const void* X, int input, int rounding, uint
     if (rounding == MX_ROUND_NEAREST_EVEN)
         return quantize_dense_rnd<MX_ROUND_NEAREST_EVEN>(X, input, rows_out, scales, rows, nrow, K, nblkp, s);
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_mx_frag_rows(const void* X, int input, int fmt, int rounding, uint8_t* out, int N, int K,
+                               int batches, hipStream_t s) {
+    if (N <= 0 || batches <= 0) return hipSuccess;
+    if (!mxpipe_supported(N, K, fmt) || batches > 65535 || (input != MX_IN_INT4 && input != MX_IN_FP16) ||
+        (rounding != MX_ROUND_REFERENCE && rounding != MX_ROUND_NEAREST_EVEN))
+        return hipErrorInvalidValue;
+    const int nblkp = mx_padded_blocks(K);
+    const int vec = ((int64_t)K * (input == MX_IN_INT4 ? 1 : 4) % 16 == 0 && (reinterpret_cast<uintptr_t>(X) & 15u) == 0) ? 1 : 0;
+    if (fmt == MX_FP4_E2M1) {
+        if (input == MX_IN_INT4) frag_rows_rnd<MX_FP4_E2M1, MX_IN_INT4>(X, out, rounding, N, K, batches, nblkp, vec, s);
+        else frag_rows_rnd<MX_FP4_E2M1, MX_IN_FP16>(X, out, rounding, N, K, batches, nblkp, vec, s);
+    } else {
+        if (input == MX_IN_INT4) frag_rows_rnd<MX_FP6_E3M2, MX_IN_INT4>(X, out, rounding, N, K, batches, nblkp, vec, s);
+        else frag_rows_rnd<MX_FP6_E3M2, MX_IN_FP16>(X, out, rounding, N, K, batches, nblkp, vec, s);
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_mx_quantize(const void* X, int input, int fmt, int rounding, uint8_t* codes, uint8_t* scales,

@@ -19,12 +19,12 @@
 #include "herk_common.h"
 #include "herk_elem.h"
 #include "herk_pipe.h"
+#include "herk_pipe_dev.h"
 
 namespace ftdx {
 
 namespace {
 
-constexpr int PT = 128;                      // tile rows and columns
 constexpr int P_THREADS = 256;               // 4 waves, 2 x 2
 constexpr int P_GROUPS = 2 * PT / 32;        // row groups of a stage: 4 of the rows, 4 of the columns
 constexpr int P_GSTRIDE = 2 * kFragBytes + 16;  // LDS bytes per group and stage; not a multiple of
@@ -34,13 +34,9 @@ constexpr int P_STAGE = P_GROUPS * P_GSTRIDE;
 constexpr int P_BUFS = 3;
 constexpr int P_LOADS = P_GROUPS * 3 / 4;    // kilobyte copies per wave and stage
 constexpr int P_WG_PER_CU = 2;
-constexpr int P_BLOCK = 4;                   // tile order: blocks of 4 x 4 tiles
 static_assert(P_BUFS * P_STAGE * P_WG_PER_CU <= 160 * 1024, "LDS of the resident workgroups");
 
-typedef int v6i __attribute__((ext_vector_type(6)));
 typedef v6i Frags[2];
-
-__device__ __forceinline__ v8i op8(v6i a) { return __builtin_shufflevector(a, a, 0, 1, 2, 3, 4, 5, -1, -1); }
 
 // v = [im | -re] of u = [re | im]: the halves swapped, bit 5 of every Re code flipped
 __device__ __forceinline__ v6i conj6(v6i a) {
@@ -54,20 +50,9 @@ __device__ __forceinline__ v6i conj6(v6i a) {
     return r;
 }
 
-template <int VM>
-__device__ __forceinline__ void wait_vm() {  // vmcnt(VM), other counters free
-    __builtin_amdgcn_s_waitcnt((VM & 0xF) | (0x7 << 4) | (0xF << 8) | (((VM >> 4) & 0x3) << 14));
-}
-
 template <int L>
 __device__ __forceinline__ void wait_lgkm() {  // lgkmcnt(L), other counters free
     __builtin_amdgcn_s_waitcnt(0xF | (0x7 << 4) | (L << 8) | (3 << 14));
-}
-
-__device__ __forceinline__ void wg_barrier() {
-    __asm__ __volatile__("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    __asm__ __volatile__("" ::: "memory");
 }
 
 // The operands of step ks (0, 1) of a stage: two groups at `a`, two at `b`.
@@ -173,60 +158,6 @@ __device__ __forceinline__ void tile_loop(__amdgpu_buffer_rsrc_t rows, uint8_t* 
     wait_vm<0>();  // no copy may land after the workgroup's LDS is given back
 }
 
-// A block wholly below the diagonal and inside the matrix, beta = 0: no element is tested, and a
-// row's offset is the last row's plus a lane constant (row d of a block starting at row w lies
-// d w + d (d + 1) / 2 elements after row 0).  The general form below spends about 15 VALU
-// operations per element, 5 of them on 64-bit index arithmetic (K = 128, FP16 output: 214
-// against 269 us for the whole launch).
-template <typename OutT, bool SCALE, bool NT>
-__device__ __forceinline__ void store_inside(OutT* C, int w, int col, float alpha, const v16f (&re)[2][2],
-                                             const v16f (&im)[2][2], int lane) {
-    typedef typename Elem<OutT>::v2 v2;
-    constexpr uint32_t ES = sizeof(v2);
-    const int n = lane & 31, g4 = (lane >> 5) * 4;
-    uint8_t* base = reinterpret_cast<uint8_t*>(reinterpret_cast<v2*>(C) + tri_index(w, col));
-    uint32_t off = (uint32_t)(g4 * w + g4 * (g4 + 1) / 2 + n) * ES;
-    const uint32_t step = (uint32_t)(w + g4) * ES;  // row d + g4 -> d + 1 + g4 adds step + (d + 1) ES
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int d = x * 32 + (q >> 2) * 8 + (q & 3);
-            v2* p = reinterpret_cast<v2*>(base + off);
-#pragma unroll
-            for (int y = 0; y < 2; ++y) {
-                const v2 e = SCALE ? Elem<OutT>::make(re[x][y][q] * alpha, im[x][y][q] * alpha)
-                                  : Elem<OutT>::make(re[x][y][q], im[x][y][q]);
-                if constexpr (NT) __builtin_nontemporal_store(e, p + y * 32);
-                else p[y * 32] = e;
-            }
-            off += (q & 3) != 3 ? step + (uint32_t)(d + 1) * ES : 5 * step + (uint32_t)(5 * d + 15) * ES;
-        }
-}
-
-// Any block: elements (i, j <= i) with i < N; Im = 0 on the diagonal, then alpha, then
-// fma(beta, old, .), as the other HERK kernels.
-template <typename OutT>
-__device__ __forceinline__ void store_any(OutT* C, int N, int w, int col, float alpha, float beta,
-                                          const v16f (&re)[2][2], const v16f (&im)[2][2], int lane) {
-    typedef typename Elem<OutT>::v2 v2;
-    const int n = lane & 31, g4 = (lane >> 5) * 4;
-    v2* base = reinterpret_cast<v2*>(C);
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int i = w + x * 32 + (q >> 2) * 8 + g4 + (q & 3);
-            v2* row = base + tri_index(i, 0);
-#pragma unroll
-            for (int y = 0; y < 2; ++y) {
-                const int j = col + y * 32 + n;
-                if (i < N && j <= i)
-                    put_element<OutT>(row + j, re[x][y][q], i == j ? 0.0f : im[x][y][q], alpha, beta);
-            }
-        }
-}
-
 // ---- GGP layouts (herk_tile.h), from the transposed accumulators: lane = row i ----
 // Block x, y, register q: i = w + 32 x + lane % 32, j = col + 32 y + 8 (q / 4) + 4 (lane / 32) + q % 4.
 // Upper packed rows (j, i >= j) are 32-lane runs, so is the upper half of the full matrix; its
@@ -288,30 +219,6 @@ __device__ __forceinline__ void store_ggp_any(OutT* C, int N, int w, int col, co
                 if (FMT == OUT_HERM_FULL && i != j) base[(int64_t)i * N + j] = Elem<OutT>::make(r, -m);
             }
         }
-}
-
-// Tile t of the lower triangle of nb x nb tiles, in square blocks of H x H tiles (row-major
-// inside a block, blocks row-major): the tiles that one XCD runs together then share H row and
-// H column blocks in its L2 instead of one and many.
-__device__ __forceinline__ void tri_decode_blocked(int t, int nb, int H, int& I, int& J) {
-    const int full = H * H, diag = H * (H + 1) / 2;
-    // block row S starts at full S (S - 1) / 2 + diag S
-    const float a = 0.5f * full, b = diag - a;
-    int S = (int)((__builtin_sqrtf(b * b + 4.0f * a * (float)t) - b) / (2.0f * a));
-    while (S > 0 && full * S * (S - 1) / 2 + diag * S > t) --S;
-    while (full * (S + 1) * S / 2 + diag * (S + 1) <= t) ++S;
-    int u = t - (full * S * (S - 1) / 2 + diag * S);
-    const int h = nb - S * H < H ? nb - S * H : H;  // rows of this block row
-    if (u < h * H * S) {
-        const int SJ = u / (h * H), v = u - SJ * (h * H);
-        I = S * H + v / H;
-        J = SJ * H + v % H;
-    } else {
-        int i;
-        tri_decode(u - h * H * S, i, u);
-        I = S * H + i;
-        J = S * H + u;
-    }
 }
 
 // Tile (I, J) of one problem: `base` its fragment rows, `steps` per row.  GGP layouts: alpha 1, beta 0.

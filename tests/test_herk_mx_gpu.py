@@ -344,6 +344,38 @@ def test_reference_precision_study(oracle, dev, reference_study_input):
             assert err / max_ref < thr
 
 
+# one row group (32), wave (64) and tile (128) to either side; blocks (32) and stages (64) too; K of
+# 3 stages (3 buffers) and 4; per-block scales far apart
+@pytest.mark.parametrize("compute", ["FP6", "FP4"])
+@pytest.mark.parametrize("rounding", [0, 1])
+@pytest.mark.parametrize("N,K,B", [(1, 1, 2), (31, 32, 3), (33, 33, 2), (65, 64, 2), (127, 65, 1), (129, 192, 2),
+                                   (200, 256, 2), (257, 100, 1)])
+def test_mx_fragment_kernel_equals_tile(dev, compute, rounding, N, K, B):
+    import torch
+    from ftd_amd import ftdx
+    g = torch.Generator(device=dev).manual_seed(N + K)
+    x = torch.randn((B, N, K, 2), generator=g, device=dev)
+    x *= torch.exp2(torch.randint(-8, 9, (B, N, K, 2), generator=g, device=dev).float())
+    x = x.half()
+    comp = getattr(ftdx.ComputePrecision, compute)
+    got = []
+    for cfg in (-1, 2):  # the 64 x 64 tile reads rows with inline scales
+        ctx = ftdx.CutlassComplexGemm()
+        ctx.set_mx_rounding(ftdx.MxRounding(rounding))
+        ctx.set_launch_config(cfg, -1)
+        for out, inp, A in (("fp32", "FP16", x), ("fp16", "FP16", x * 0.01),
+                            ("fp32", "INT4", x.view(torch.uint8)[..., 0].contiguous())):
+            C = ftdx.herk_mx(ctx, A, N, K, B, getattr(ftdx.InputPrecision, inp), comp, output=out, alpha=0.5)
+            got.append(C.cpu())
+            D = C.clone()
+            ftdx.herk_mx(ctx, A, N, K, B, getattr(ftdx.InputPrecision, inp), comp, output=out, alpha=0.5, beta=2.0, C=D)
+            got.append(D.cpu())
+    half = len(got) // 2
+    for a, b in zip(got[:half], got[half:]):
+        it = torch.int32 if a.dtype == torch.float32 else torch.int16
+        assert torch.equal(a.view(it), b.view(it))
+
+
 @pytest.mark.parametrize("rounding", [0, 1])
 def test_mx_fp6_one_step_sum_width(oracle, dev, rounding):
     """Where the FP6 tolerance comes from: one 32-sample block (K = 32, one scaled MFMA step
