@@ -669,10 +669,10 @@ int gemm_run(ftdx_context* ctx, const uint8_t* brows, GemmInput kind, const void
     g.b_bstride = (int64_t)N * Kp * 2;
     g.ldc = N;
     g.c_bstride = (int64_t)M * N;
-    // 256x128 tiles, one workgroup per CU, whose direct loads run two stages ahead in three
-    // LDS buffers: fastest at the beamformer shape (M = 256, N = 4000, K = 1664: 0.90 ms
-    // against 0.91-0.96 ms for the 128x128 tiles, two workgroups per CU)
-    const int cfg = ctx->forced_cfg >= 0 ? tile_base(ctx->forced_cfg) : TILE_256x128_K64;
+    // 128x128 tiles, two workgroups per CU, so that one's stores overlap the other's MFMAs, against
+    // 256x128, one per CU (us): M = 256, N = 4000, K = 1664 x 128 743 / 790; 128, 2000, 1000 x 32
+    // 43 / 51; 64, 4000, 1664 x 64 183 / 207; 512, 4000, 512 x 16 62 / 70; 256, 4000, 1664 x 8 48 / 47
+    const int cfg = ctx->forced_cfg >= 0 ? tile_base(ctx->forced_cfg) : TILE_128x128_K64_P2;
     const int remap = ctx->forced_remap >= 0 ? ctx->forced_remap : kDefaultRemap;
     e = launch_gemm_fp8(g, cfg, fmt, out_fp16, remap, s);
     return e == hipSuccess ? FTDX_OK : hip_fail(e, what);
@@ -1199,6 +1199,9 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
     const bool may_pipe = may_route && ftdx::pipe_supported(N, K);
     const bool tune_now = tune && !cached && !explicit_cfg && !precast;
     if (may_route && !cached) cfg = ftdx::choose_kernel(A, N, K, batch_count, fp16);
+    // pre-cast rows: loads two stages ahead (FP16 input 1664 x 16, K = 512: 67 against 73 us;
+    // 4096 x 8, K = 2048: 484 against 489; 1024 x 32, K = 300: 54 both)
+    if (precast && !cached && !explicit_cfg) cfg = ftdx::TILE_128x128_K64_P2;
     uint8_t* frag = nullptr;
     if (may_pipe && (cfg == ftdx::TILE_PIPE || tune_now))
         frag = ftdx::frag_scratch(ctx, ftdx::frag_scratch_bytes(a), s);

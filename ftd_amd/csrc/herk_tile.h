@@ -16,6 +16,7 @@
 //   LDS (double-buffered, one barrier per stage) -> ds_read_b128 -> MFMA.
 #pragma once
 #include "herk_common.h"
+#include "herk_elem.h"
 #include "herk_fp8.h"
 
 namespace ftdx {
@@ -519,6 +520,38 @@ struct TileRunner {
             __builtin_nontemporal_store((OutT)r, Cr + idx);
             __builtin_nontemporal_store((OutT)m, Ci + idx);
         }
+    }
+
+    // A block inside the matrix, beta = 0: no element is tested, and a row's offset is the last
+    // row's plus the pitch.
+    template <typename OutT, int FMT>
+    static __device__ __forceinline__ void gemm_inside(const TileJob& j, const v16f (&acc_re)[Cfg::FM][Cfg::FN],
+                                                       const v16f (&acc_im)[Cfg::FM][Cfg::FN], int wrow0, int wcol0,
+                                                       int lane) {
+        const int n = lane & 31, g4 = (lane >> 5) * 4;
+        const int64_t at = (int64_t)wrow0 * j.ldc + wcol0;
+        const uint32_t pitch = (uint32_t)j.ldc;
+        uint32_t off = (uint32_t)g4 * pitch + (uint32_t)n;
+#pragma unroll
+        for (int a = 0; a < Cfg::FM; ++a)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+#pragma unroll
+                for (int b = 0; b < Cfg::FN; ++b) {
+                    const float re = acc_re[a][b][r], im = acc_im[a][b][r];
+                    if constexpr (FMT == OUT_GEMM_POWER) {
+                        float* p = static_cast<float*>(j.C) + at + off + b * 32;
+                        const float v = j.alpha * __builtin_fmaf(re, re, im * im);
+                        __builtin_nontemporal_store(v, p);
+                    } else {
+                        OutT* cr = static_cast<OutT*>(j.C) + at + off + b * 32;
+                        OutT* ci = static_cast<OutT*>(j.C2) + at + off + b * 32;
+                        __builtin_nontemporal_store((OutT)(re * j.alpha), cr);
+                        __builtin_nontemporal_store((OutT)(im * j.alpha), ci);
+                    }
+                }
+                off += ((r & 3) != 3 ? 1u : 5u) * pitch;
+            }
     }
 
     // Beamformer epilogue (OUT_GEMM_BEAM).  Tile rows 0-63 are samples m0 .. m0 + 63 of
@@ -1313,6 +1346,10 @@ struct TileRunner {
             // B rows hold conj(B), so the HERK product A conj(B)^H = A B^T; lane =
             // column in the accumulator layout: consecutive lanes store consecutive j.
             if (!active) return;
+            if (wrow0 + Cfg::WM <= j.N && wcol0 + Cfg::WN <= j.Ncol && j.beta == 0.0f && j.ldc <= (1 << 20)) {
+                gemm_inside<OutT, FMT>(j, acc_re, acc_im, wrow0, wcol0, lane);
+                return;
+            }
             const int n = lane & 31, g4 = (lane >> 5) * 4;
 #pragma unroll
             for (int a = 0; a < Cfg::FM; ++a)
@@ -1328,7 +1365,23 @@ struct TileRunner {
                     }
                 }
             return;
-        } else if constexpr (FMT == OUT_LOWER_PACKED && Cfg::EPI_STAGED) {
+        }
+        if constexpr (FMT == OUT_LOWER_PACKED) {
+            // A tile inside the matrix and below the diagonal stores straight from its accumulators.
+            // Plain stores, which the L2 joins to whole lines, up to 1024 samples on the larger
+            // tiles; us of staged / non-temporal / plain stores, 128 x 128 tiles: FP16 rows of 1024
+            // x 32, K = 300, FP32 67 / 66 / 54; QC 1664 x 64, K = 128, FP16 129 / 145 / 109; QC
+            // 2048 x 16, K = 512, FP32 89 / 91 / 84; FP16 rows of 4096 x 8, K = 2048, FP16 504 /
+            // 484 / 491.  64 x 64 tiles write shorter runs: the second 235 / 151 / 183, the third
+            // 172 / 140 / 156.
+            if (j.beta == 0.0f && j.row0 + Cfg::TM <= j.N && j.col0 + Cfg::TN <= j.row0) {
+                OutT* C = static_cast<OutT*>(j.C);
+                if (Cfg::TM < 128 || j.K > 1024) store_inside<OutT, true, true>(C, wrow0, wcol0, j.alpha, acc_re, acc_im, lane);
+                else store_inside<OutT, true, false>(C, wrow0, wcol0, j.alpha, acc_re, acc_im, lane);
+                return;
+            }
+        }
+        if constexpr (FMT == OUT_LOWER_PACKED && Cfg::EPI_STAGED) {
             epilogue_staged<OutT>(j, lds, acc_re, acc_im, active, wrow0, wcol0, lane, wave);
             return;
         }
