@@ -21,6 +21,7 @@
 #include "herk_fp8.h"
 #include "herk_mx.h"
 #include "herk_direct.h"
+#include "herk_grid.h"
 #include "herk_mxpipe.h"
 #include "herk_pipe.h"
 #include "calib.h"
@@ -329,6 +330,7 @@ hipError_t run_padded(ftdx_context* ctx, const HerkPlainArgs& a, int cfg, int ou
         b.batch = nu * grp;
         b.K = Kq;
         b.a_bstride = (int64_t)a.N * Kq;
+        if (a.half) b.half = a.half + (int64_t)u0 * grp * 2 * half_grid_cells(a.Ng);
         b.freq_offset = a.freq_offset + u0 * grp;
         if ((e = launch(b)) != hipSuccess) return e;
     }
@@ -386,7 +388,7 @@ uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
 }
 
 // Converts and multiplies chunk by chunk; a.A holds QC rows, `rows` frag_scratch_bytes(a).
-hipError_t run_pipe(uint8_t* rows, const HerkPlainArgs& a, bool fp16, hipStream_t st) {
+hipError_t run_pipe(uint8_t* rows, const HerkPlainArgs& a, bool fp16, hipStream_t st, bool grid = false) {
     const int grp = std::max(a.seg_group, 1), in_per = a.nseg * grp, units = a.batch / grp;
     const int64_t slots = (int64_t)std::max(device_cu_count(), 1) * pipe_wg_per_cu();
     const int chunk = pick_chunk_of(slots, (int64_t)pipe_tiles(a.N) * grp, units, frag_chunk_cap(a.N, a.K, in_per, units));
@@ -400,7 +402,11 @@ hipError_t run_pipe(uint8_t* rows, const HerkPlainArgs& a, bool fp16, hipStream_
         b.C = static_cast<uint8_t*>(a.C) + (int64_t)u0 * grp * a.c_bstride * (fp16 ? 2 : 4);
         b.batch = nu * grp;
         b.a_bstride = frag_rows_bytes(a.N, a.K, a.nseg);
-        if ((e = launch_herk_pipe(b, fp16, st)) != hipSuccess) return e;
+        if (grid) {
+            b.freq_offset = a.freq_offset + u0 * grp;
+            if (a.half) b.half = a.half + (int64_t)u0 * grp * 2 * half_grid_cells(a.Ng);
+        }
+        if ((e = grid ? launch_herk_pipe_grid(b, st) : launch_herk_pipe(b, fp16, st)) != hipSuccess) return e;
     }
     return hipSuccess;
 }
@@ -459,15 +465,19 @@ bool worth_direct(int N, int K, int batch) {
 //   1024 x 286, K 2048:   - / 1022 / 1098   2624 x 43, K 128:    - / 295 / 320
 //   4096 x 96, K 2048:    - / 4134 / 5460
 // Rows that 16-byte loads cannot take cost the fused tile a padding pass.
+double fused_us(double st, double t128) { return 5.0 + std::max(0.87 * st + 3.0, t128 / 512.0 * (1.55 * st + 6.0)); }
+double pipe_us(double st, double t128, double in) {
+    return 8.0 + in * 2.5 / 5e6 + std::max(0.45 * st + 3.0, t128 / 512.0 * (0.92 * st + 5.7));
+}
+
 int choose_kernel(const void* A, int N, int K, int batch, bool fp16) {
     const double st = (K + 63) / 64, t128 = (double)pipe_tiles(N) * batch, in = (double)N * K * batch;
     const double out = (double)N * (N + 1) / 2 * (fp16 ? 4.0 : 8.0) * batch;
-    double best = 5.0 + std::max({0.87 * st + 3.0, t128 / 512.0 * (1.55 * st + 6.0), out / 3.6e6});
+    double best = std::max(fused_us(st, t128), 5.0 + out / 3.6e6);
     if (!rows_take_vector_loads(A, K)) best += 4.0 + in * 2.0 / 5e6;
     int pick = TILE_128x128_K64_P2;
     if (pipe_supported(N, K)) {
-        const double t = 8.0 + in * 2.5 / 5e6 +
-                         std::max({0.45 * st + 3.0, t128 / 512.0 * (0.92 * st + 5.7), out / (out < 2e8 ? 5.5e6 : 4.1e6)});
+        const double t = std::max(pipe_us(st, t128, in), 8.0 + in * 2.5 / 5e6 + out / (out < 2e8 ? 5.5e6 : 4.1e6));
         if (t < best) {
             best = t;
             pick = TILE_PIPE;
@@ -476,6 +486,25 @@ int choose_kernel(const void* A, int N, int K, int batch, bool fp16) {
     if (worth_direct(N, K, batch) && 4.0 + std::max(0.68e-3 * direct_tiles(N) * batch * st, out / 2.8e6) < best)
         pick = TILE_DIRECT;
     return pick;
+}
+
+// The same estimates for the gridding HERK over nseg polarizations (us, fused / pipelined: 64 x 16
+// channels, K = 2 x 1024 89 / 75; 512 x 8, 2 x 512 106 / 102; 100 x 16, 2 x 64 62 / 63).
+bool grid_pipe_pays(const HerkPlainArgs& a) {
+    const double st = (double)((a.K + 63) / 64) * a.nseg, t128 = (double)pipe_tiles(a.N) * a.batch;
+    return pipe_supported(a.N, a.K, a.nseg) && t128 <= 0x7FFFFFFF &&
+           pipe_us(st, t128, (double)a.N * a.K * a.nseg * a.batch) < fused_us(st, t128);
+}
+
+// Whether a half plane (herk_grid.h) saves more scattered atomics than its own passes cost: from
+// one baseline per five cells on, and up to 256 MB of it.  us without / with, baselines per cell:
+// 1024 x 8 channels on 1024^2 (0.50) 498 / 353; 512 x 8 on 512^2 (0.50) 133 / 106; 1536 x 2 on
+// 2048^2 (0.28) 268 / 227; 700 x 1 on 1000^2 (0.25) 74 / 65; 512 x 8 on 1024^2 (0.13) 141 / 146
+// (with the slower first form of the closing pass).
+bool half_grid_pays(int N, int Ng, int n_chan) {
+    const size_t plane = (size_t)half_grid_cells(Ng) * 8;
+    return 5 * ((int64_t)N * (N + 1) / 2) >= (int64_t)Ng * Ng && n_chan <= 65535 &&
+           plane <= (size_t(256) << 20) / n_chan;
 }
 
 // Times every (tile configuration, workgroup order) on this call's buffers and
@@ -1513,7 +1542,21 @@ int ftdx_herk_pol_grid(ftdx_context* ctx, const void* A, int N, int K, int n_cha
     const int remap = ctx->forced_remap >= 0 ? ctx->forced_remap : ftdx::kDefaultRemap;
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e;
-    if (ftdx::pol_rows_padded(A, K, n_pol, cfg)) {
+    // the half plane and the fragment rows, one after the other in this stream's scratch
+    const size_t half_bytes =
+        ftdx::half_grid_pays(N, Ng, n_chan) ? ((size_t)n_chan * ftdx::half_grid_cells(Ng) * 8 + 255) / 256 * 256 : 0;
+    const bool may_pipe = ctx->forced_cfg < 0 && ctx->direct_tile == FTDX_DIRECT_TILE_AUTO && ftdx::grid_pipe_pays(a);
+    uint8_t* scr = nullptr;
+    if (half_bytes || may_pipe)
+        scr = ftdx::frag_scratch(ctx, half_bytes + (may_pipe ? ftdx::frag_scratch_bytes(a) : 0), s);
+    if (scr && half_bytes) {
+        a.half = reinterpret_cast<float*>(scr);
+        if ((e = hipMemsetAsync(a.half, 0, half_bytes, s)) != hipSuccess)
+            return hip_fail(e, "ftdx_herk_pol_grid: half grid");
+    }
+    if (scr && may_pipe) {
+        e = ftdx::run_pipe(scr + half_bytes, a, false, s, true);
+    } else if (ftdx::pol_rows_padded(A, K, n_pol, cfg)) {
         // rows padded per chunk of channels, as ftdx_herk does
         int rc = ftdx::grow_precast(ctx, ftdx::padded_scratch_bytes(a), "ftdx_herk_pol_grid: scratch");
         if (rc != FTDX_OK) return rc;
@@ -1523,6 +1566,7 @@ int ftdx_herk_pol_grid(ftdx_context* ctx, const void* A, int N, int K, int n_cha
     } else {
         e = ftdx::launch_herk_grid(a, cfg, remap, s);
     }
+    if (e == hipSuccess && a.half) e = ftdx::launch_half_grid_add(a.half, uv_grid, Ng, n_chan, s);
     return e == hipSuccess ? FTDX_OK : hip_fail(e, "ftdx_herk_pol_grid");
 }
 

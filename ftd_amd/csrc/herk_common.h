@@ -143,20 +143,21 @@ __device__ __forceinline__ float pair_lane(float v) {
     return __int_as_float(pair_lane<Odd>(__float_as_int(v)));
 }
 
-// Adds (re, im) to grid cell `cell` ([cells][2] FP32; cell < 0: none).  Every lane of the wave
+// Adds (re, im) to the grid cell at p ([re, im] FP32; nullptr: none).  Every lane of the wave
 // calls it.  Scattered FP32 atomics run at about 21e9 cache-line requests/s on the whole chip,
 // the same for a grid of 0.1 MB as for one of 128 MB and at either scope, and the lanes of one
 // instruction that hit one line share a request.  So the two components of a cell go out as
 // two neighbouring lanes of one instruction (even lanes' cells first, odd lanes' next) rather
 // than as two instructions: 10.4e9 -> 21.0e9 cells/s.
-__device__ __forceinline__ void grid_add(float* grid, int64_t cell, float re, float im) {
+__device__ __forceinline__ void grid_add(float* p, float re, float im) {
     const bool odd = threadIdx.x & 1;
-    const int lo = (int)cell, hi = (int)(cell >> 32);
-    const int64_t c0 = ((int64_t)pair_lane<false>(hi) << 32) | (uint32_t)pair_lane<false>(lo);
-    const int64_t c1 = ((int64_t)pair_lane<true>(hi) << 32) | (uint32_t)pair_lane<true>(lo);
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    const int lo = (int)a, hi = (int)(a >> 32);
+    const uint64_t a0 = ((uint64_t)(uint32_t)pair_lane<false>(hi) << 32) | (uint32_t)pair_lane<false>(lo);
+    const uint64_t a1 = ((uint64_t)(uint32_t)pair_lane<true>(hi) << 32) | (uint32_t)pair_lane<true>(lo);
     const float im0 = pair_lane<false>(im), re1 = pair_lane<true>(re);
-    if (c0 >= 0) unsafeAtomicAdd(grid + 2 * c0 + odd, odd ? im0 : re);
-    if (c1 >= 0) unsafeAtomicAdd(grid + 2 * c1 + odd, odd ? im : re1);
+    if (a0) unsafeAtomicAdd(reinterpret_cast<float*>(a0) + odd, odd ? im0 : re);
+    if (a1) unsafeAtomicAdd(reinterpret_cast<float*>(a1) + odd, odd ? im : re1);
 }
 
 }  // namespace ftdx

@@ -94,6 +94,8 @@ struct HerkPlainArgs {
     int freq_offset = 0;
     int Ng = 0;
     float cell = 0.0f;
+    // scratch planes of half_grid_cells(Ng) cells per batch (herk_grid.h), zeroed; nullptr: none
+    float* half = nullptr;
 };
 
 // Lower-triangle tiles per problem for a configuration.

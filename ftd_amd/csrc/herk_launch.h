@@ -61,10 +61,7 @@ herk_int4_fp8_plain_kernel(HerkPlainArgs p, int tiles, int xcd_remap) {
         j.s_stage = p.s_stage;
     }
     if constexpr (FMT == OUT_GRID) {
-        j.uv = p.uv_m;
-        j.lambda = 299792458.0 / p.freq_hz[p.freq_offset + b];  // speed of light / frequency
-        j.Ng = p.Ng;
-        j.cell = p.cell;
+        j.grid = grid_job(p, b);
     }
     TileRunner<Cfg>::template run<OutT, MODE, FMT, false, TAILS>(j, lds);
 }

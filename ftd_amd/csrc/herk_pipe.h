@@ -40,6 +40,9 @@ hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t s
 hipError_t launch_ggp_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, int batches, hipStream_t stream);
 hipError_t launch_herk_pipe_ggp(const HerkPlainArgs& a, int fmt, bool out_fp64, hipStream_t stream);
 
+// The HERK over fragment rows whose epilogue grids (OUT_GRID), as launch_herk_grid.
+hipError_t launch_herk_pipe_grid(const HerkPlainArgs& a, hipStream_t stream);
+
 // Tiles per batch and resident workgroups per CU of the launch above.
 int pipe_tiles(int N);
 int pipe_wg_per_cu();

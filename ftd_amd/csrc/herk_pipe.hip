@@ -18,6 +18,7 @@
 // 128, K = 128: 303 against 478 us; 64-byte write requests within 1% of the output bytes).
 #include "herk_common.h"
 #include "herk_elem.h"
+#include "herk_grid.h"
 #include "herk_pipe.h"
 #include "herk_pipe_dev.h"
 
@@ -221,10 +222,11 @@ __device__ __forceinline__ void store_ggp_any(OutT* C, int N, int w, int col, co
         }
 }
 
-// Tile (I, J) of one problem: `base` its fragment rows, `steps` per row.  GGP layouts: alpha 1, beta 0.
+// Tile (I, J) of one problem: `base` its fragment rows, `steps` per row.  GGP layouts: alpha 1,
+// beta 0; OUT_GRID: `grid` in place of C.
 template <typename OutT, int FMT = OUT_LOWER_PACKED>
 __device__ __forceinline__ void pipe_tile(uint8_t* lds, const uint8_t* base, int N, int steps, int I, int J, OutT* C,
-                                          float alpha, float beta, bool nt) {
+                                          float alpha, float beta, bool nt, const GridJob* grid = nullptr) {
     // wave index in an SGPR: the conditions on it are scalar branches
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave >> 1, wn = wave & 1;
@@ -254,11 +256,16 @@ __device__ __forceinline__ void pipe_tile(uint8_t* lds, const uint8_t* base, int
     const int a = wm * 2 * P_GSTRIDE, bo = (P_GROUPS / 2 + wn * 2) * P_GSTRIDE;
     if (!active) {
         tile_loop<false, false>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
+        if constexpr (FMT == OUT_GRID) __syncthreads();
         return;
     }
-    tile_loop<true, FMT != OUT_LOWER_PACKED>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
+    tile_loop<true, FMT == OUT_UPPER_PACKED || FMT == OUT_HERM_FULL>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
     const bool inside = wcol + 63 < wrow && wrow + 64 <= N;
-    if constexpr (FMT != OUT_LOWER_PACKED) {
+    if constexpr (FMT == OUT_GRID) {
+        static_assert(4 * grid_lds_bytes<2>() <= P_BUFS * P_STAGE, "gridding regions");
+        __syncthreads();  // the last stage is read
+        grid_block(*grid, N, wrow, wcol, alpha, re, im, lds + wave * grid_lds_bytes<2>(), lane);
+    } else if constexpr (FMT != OUT_LOWER_PACKED) {
         if (inside) store_ggp_inside<OutT, FMT>(C, N, wrow, wcol, re, im, lane);
         else store_ggp_any<OutT, FMT>(C, N, wrow, wcol, re, im, lane);
     } else if (inside && beta == 0.0f) {
@@ -281,8 +288,14 @@ __global__ void __launch_bounds__(P_THREADS, 2) herk_pipe_kernel(HerkPlainArgs p
     const int b = w / tiles, t = w - b * tiles;
     int I, J;
     tri_decode_blocked(t, (p.N + PT - 1) / PT, P_BLOCK, I, J);
-    pipe_tile<OutT, FMT>(lds, p.A + (int64_t)b * p.a_bstride, p.N, steps, I, J,
-                         static_cast<OutT*>(p.C) + (int64_t)b * p.c_bstride, p.alpha, p.beta, NT);
+    const uint8_t* rows = p.A + (int64_t)b * p.a_bstride;
+    if constexpr (FMT == OUT_GRID) {
+        const GridJob g = grid_job(p, b);
+        pipe_tile<OutT, FMT>(lds, rows, p.N, steps, I, J, nullptr, p.alpha, 0.0f, NT, &g);
+    } else {
+        pipe_tile<OutT, FMT>(lds, rows, p.N, steps, I, J, static_cast<OutT*>(p.C) + (int64_t)b * p.c_bstride, p.alpha,
+                             p.beta, NT);
+    }
 }
 
 // Tiles of many problems: workgroup b runs tiles[b].
@@ -528,6 +541,17 @@ hipError_t launch_qc_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, in
             hipLaunchKernelGGL((qc_frag_rows_kernel<false, 4>), grid, block, 0, stream, in, out, N, K, steps, nseg,
                                seg_group);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_herk_pipe_grid(const HerkPlainArgs& a, hipStream_t stream) {
+    if (a.N <= 0 || a.batch <= 0) return hipSuccess;
+    const int tiles = pipe_tiles(a.N);
+    const int64_t blocks = (int64_t)tiles * a.batch;
+    if (blocks > 0x7FFFFFFF || !pipe_supported(a.N, a.K, a.nseg) || !a.uv_m || !a.freq_hz || a.Ng <= 0)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL((herk_pipe_kernel<float, false, OUT_GRID>), dim3((unsigned)blocks), dim3(P_THREADS), 0, stream, a,
+                       frag_steps(a.K) * a.nseg, tiles);
     return hipGetLastError();
 }
 

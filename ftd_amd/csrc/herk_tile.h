@@ -17,6 +17,7 @@
 #pragma once
 #include "herk_common.h"
 #include "herk_elem.h"
+#include "herk_grid.h"
 #include "herk_fp8.h"
 
 namespace ftdx {
@@ -105,12 +106,7 @@ struct TileJob {
     // LOAD_MX4D: this problem's scales (row 0 of stage 0) and the bytes between stages
     const uint8_t* S;
     int64_t s_stage;
-    // OUT_GRID: baseline UV (metres, packed lower index), wavelength (metres), grid size
-    // and cell (radians); C is this batch's grid plane [Ng][Ng][2]
-    const float* uv;
-    double lambda;
-    int Ng;
-    float cell;
+    GridJob grid;  // OUT_GRID
 };
 
 // 4 QC bytes (4 samples) -> u dwords: re = fp8(Re0..Re3), im = fp8(Im0..Im3).
@@ -606,48 +602,6 @@ struct TileRunner {
                 out[g] = acc;
             }
         }
-    }
-
-    // Gridding epilogue (OUT_GRID): the pillbox scatter of the reference
-    // (include/kernels/visibility_bf.cuh:269-370) applied to each element straight from
-    // the accumulators, so the triangle never reaches HBM.  Element (i, j <= i) is
-    // baseline i(i+1)/2 + j; UV in wavelengths = float(uv_m / lambda) (double division);
-    // cell = roundf(u / cell + Ng/2); the visibility alpha * C_ij (Im = 0 on the diagonal)
-    // is added there and, for i != j, its conjugate at (-u, -v).
-    static __device__ __forceinline__ int64_t grid_cell(const TileJob& j, float u_lam, float v_lam, float half_ng) {
-        const int iu = (int)__builtin_roundf(u_lam / j.cell + half_ng);
-        const int iv = (int)__builtin_roundf(v_lam / j.cell + half_ng);
-        return iu >= 0 && iu < j.Ng && iv >= 0 && iv < j.Ng ? (int64_t)iv * j.Ng + iu : -1;
-    }
-
-    static __device__ __forceinline__ void epilogue_grid(const TileJob& j, const v16f (&acc_re)[Cfg::FM][Cfg::FN],
-                                                         const v16f (&acc_im)[Cfg::FM][Cfg::FN], int wrow0,
-                                                         int wcol0, int lane) {
-        float* grid = static_cast<float*>(j.C);
-        const float half_ng = 0.5f * j.Ng;
-        const int n = lane & 31, g4 = (lane >> 5) * 4;
-#pragma unroll
-        for (int a = 0; a < Cfg::FM; ++a)
-#pragma unroll
-            for (int b = 0; b < Cfg::FN; ++b) {
-                const int gj = wcol0 + b * 32 + n;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int gi = wrow0 + a * 32 + (r >> 2) * 8 + g4 + (r & 3);
-                    const float vre = acc_re[a][b][r] * j.alpha;
-                    const float vim = gi == gj ? 0.0f : acc_im[a][b][r] * j.alpha;
-                    int64_t cell = -1, conj = -1;
-                    if (gi < j.N && gj <= gi) {
-                        const int64_t k = tri_index(gi, gj);
-                        const float u_lam = (float)((double)j.uv[2 * k] / j.lambda);
-                        const float v_lam = (float)((double)j.uv[2 * k + 1] / j.lambda);
-                        cell = grid_cell(j, u_lam, v_lam, half_ng);
-                        if (gi != gj) conj = grid_cell(j, -u_lam, -v_lam, half_ng);
-                    }
-                    grid_add(grid, cell, vre, vim);
-                    grid_add(grid, conj, vre, -vim);
-                }
-            }
     }
 
     // One stage of MFMAs on the staged rows in `st` (KC samples, all 32-sample steps).
@@ -1340,7 +1294,9 @@ struct TileRunner {
             epilogue_beam<OutT>(j, lds, acc_re, acc_im, active, wrow0, wcol0, lane, tid);
             return;
         } else if constexpr (FMT == OUT_GRID) {
-            if (active) epilogue_grid(j, acc_re, acc_im, wrow0, wcol0, lane);
+            static_assert(grid_lds_bytes<Cfg::FN>() * Cfg::WAVES_M * Cfg::WAVES_N <= Cfg::LDS_BYTES, "gridding regions");
+            if (active)
+                grid_block(j.grid, j.N, wrow0, wcol0, j.alpha, acc_re, acc_im, lds + wave * grid_lds_bytes<Cfg::FN>(), lane);
             return;
         } else if constexpr (GEMM) {
             // B rows hold conj(B), so the HERK product A conj(B)^H = A B^T; lane =

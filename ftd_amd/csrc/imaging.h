@@ -14,4 +14,8 @@ hipError_t launch_pillbox_grid(const void* vis, bool fp16, const float* uv_m, co
                                float* grid, int64_t n_bl, int Ng, int Nf, int freq_offset, float cell,
                                hipStream_t s);
 
+// Half planes [planes][half_grid_cells(Ng)] of the gridding HERK (herk_grid.h) into the grids
+// [planes][Ng][Ng][2]: each cell to itself, its conjugate to its mirror cell.
+hipError_t launch_half_grid_add(const float* half, float* grid, int Ng, int planes, hipStream_t s);
+
 }  // namespace ftdx

@@ -187,6 +187,31 @@ def test_fused_herk_pol_grid_bit_exact(oracle, dev, N, K, n_ch, n_pol, cfg):
     assert np.array_equal(_bits(unfused.cpu().numpy()), _bits(ref))
 
 
+# even and odd grids (mirror cells at Ng - i both ways), few baselines (no half plane) and many;
+# K and polarizations that the pipelined kernel takes (2 x 1024) and not; a grid that is not zero
+@pytest.mark.parametrize("N,K,n_pol,Ng", [(20, 64, 2, 64), (129, 1024, 2, 64), (129, 1000, 2, 65), (200, 40, 1, 33),
+                                          (64, 2048, 1, 16)])
+def test_gridding_by_half_planes(oracle, dev, N, K, n_pol, Ng):
+    """Pairs of mirror cells add once to a half plane: bit-exact on integer sums, also for
+    baselines on the grid's edge (no mirror cell) and exactly between two cells (rounding away
+    from zero is not symmetric about the centre)."""
+    import torch
+    from ftd_amd import ftdx
+    n_ch, cell = 3, 2e-3
+    qc = oracle.gen_qc_uniform(N + K, N * K * n_ch * n_pol)
+    rng = np.random.default_rng(Ng)
+    freqs = np.array([299792458.0, 0.5 * 299792458.0, 1.3e9])  # wavelengths 1 and 2 m
+    uv = (rng.integers(-2 * Ng, 2 * Ng + 1, (N * (N + 1) // 2, 2)) * (0.25 * cell)).astype(np.float32)  # ties among them
+    uv[np.arange(N) * (np.arange(N) + 3) // 2] = 0.0  # autocorrelations
+    ref = _grid_ref(oracle, qc, N, K, n_ch, n_pol, uv, freqs, Ng, cell, 0, 1.0)
+    A, uv_d, f_d = (torch.from_numpy(x).to(dev) for x in (qc, uv, freqs))
+    grid = torch.full((n_ch, Ng, Ng, 2), 3.0, dtype=torch.float32, device=dev)
+    ftdx.herk_pol_grid(ftdx.CutlassComplexGemm(), A, N, K, n_ch, n_pol, uv_d, f_d, grid, Ng, cell)
+    torch.cuda.synchronize()
+    assert np.abs(ref).max() < 2 ** 24 - 3 and np.abs(ref).sum() > 0
+    assert np.array_equal(grid.cpu().numpy(), ref + 3.0)
+
+
 @pytest.mark.parametrize("N", [1, 2, 3, 11, 23])
 def test_gridding_of_partial_waves(oracle, dev, N):
     """Baseline counts that fill no wave (1, 3, 6, 66, 276): the gridding kernels pair lanes
