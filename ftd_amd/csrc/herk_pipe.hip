@@ -287,7 +287,11 @@ __global__ void __launch_bounds__(P_THREADS, 2) herk_pipe_kernel(HerkPlainArgs p
     const int w = xcd_logical((int)blockIdx.x, tiles * p.batch);
     const int b = w / tiles, t = w - b * tiles;
     int I, J;
-    tri_decode_blocked(t, (p.N + PT - 1) / PT, P_BLOCK, I, J);
+    // Launches that are bound by their stores go 2 x 2 tiles at a time (longer runs of each output
+    // row together), those bound by operands 4 x 4; us for 1 / 2 / 4 / 8: 4096 x 16, K = 256 255 /
+    // 261 / 276 / 281; 2500 x 20, K = 128 122 / 124 / 129 / 130; 3000 x 20, K = 64, FP16 79 / 78 / 83 /
+    // 81; 1664 x 128, K = 128, FP16 212 / 205 / 207 / 206; 4096 x 96, K = 2048 4364 / 4203 / 4150 / 4160.
+    tri_decode_blocked(t, (p.N + PT - 1) / PT, NT ? P_BLOCK : 2, I, J);
     const uint8_t* rows = p.A + (int64_t)b * p.a_bstride;
     if constexpr (FMT == OUT_GRID) {
         const GridJob g = grid_job(p, b);
