@@ -357,6 +357,10 @@ def test_mx_fragment_kernel_equals_tile(dev, compute, rounding, N, K, B):
     x = torch.randn((B, N, K, 2), generator=g, device=dev)
     x *= torch.exp2(torch.randint(-8, 9, (B, N, K, 2), generator=g, device=dev).float())
     x = x.half()
+    # blocks of zeros of both signs, of subnormals, and of each side of the quantizers' 2^-7 line
+    x[0, 0, :32] *= 0.0
+    x[0, N // 2, -32:] *= 2.0 ** -18
+    x[-1, N - 1, :32] = x[-1, N - 1, :32].clamp(-1, 1) * (127 / 128) * 2.0 ** -7
     comp = getattr(ftdx.ComputePrecision, compute)
     got = []
     for cfg in (-1, 2):  # the 64 x 64 tile reads rows with inline scales
