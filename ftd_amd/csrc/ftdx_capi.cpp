@@ -395,7 +395,7 @@ hipError_t run_pipe(uint8_t* rows, const HerkPlainArgs& a, bool fp16, hipStream_
     for (int u0 = 0; u0 < units; u0 += chunk) {
         const int nu = std::min(chunk, units - u0);
         hipError_t e = launch_qc_frag_rows(a.A + (int64_t)u0 * in_per * a.a_bstride, rows, a.N, a.K, nu * in_per,
-                                           a.nseg, grp, st);
+                                           a.nseg, grp, !grid && pipe_nontemporal(a.K * a.nseg, fp16), st);
         if (e != hipSuccess) return e;
         HerkPlainArgs b = a;
         b.A = rows;

@@ -230,9 +230,9 @@ int grouped_build_pipe(ftdx_grouped_plan* P, const ftdx_herk_problem* problems, 
     for (size_t p = 0; p < probs.size(); ++p) {
         PipeProblem& q = probs[p];
         q.rows = at;
-        at += (size_t)((q.N + 31) / 32) * q.steps * kFragBytes;
+        at += (size_t)frag_groups(q.N) * q.steps * kFragBytes;
         cost += pipe_cost(q) * pipe_tiles(q.N);
-        const int64_t segs = (int64_t)(q.N + 31) / 32 * 64 * q.steps;  // < 2^31: its rows' bytes / 24
+        const int64_t segs = (int64_t)frag_groups(q.N) * 64 * q.steps;  // < 2^31: its rows' bytes / 24
         for (int64_t f = 0; f < segs; f += kConvThreads) conv.push_back({(int)p, (uint32_t)f});
     }
     for (size_t p = 0; p < probs.size(); ++p) {

@@ -43,7 +43,7 @@ int heuristic_cfg(int N, int batch) {
 
 // Whether a GGP payload takes the pipelined kernel over E3M2 fragment rows, which holds every
 // [-8, 7] nibble exactly: where one pass is exact, the rows need at most 64 MB more scratch than
-// the FP8 ones (groups of 32 rows: few antennas waste them), and except for full FP64 matrices
+// the FP8 ones (blocks of 64 rows: few antennas waste them), and except for full FP64 matrices
 // of few tiles, whose scattered lower-half stores one workgroup then waits for.  us per call,
 // FP8 tile / pipelined, both polarizations:
 //   upper FP32:  64 x 2, K 64  26 / 24     1024 x 32, K 256  96 / 56     2048 x 8, K 1024  127 / 90

@@ -7,7 +7,9 @@
 // six-bit Re codes then 16 Im codes (code k at bits 6k), six dwords, the first four of all
 // lanes at 16 l, the last two at 1024 + 8 l.  So a wave copies whole kilobytes from memory
 // to LDS and reads its operands from there without bank conflicts, 48 bytes per 32 samples.
-// Rows past N and samples past K are zero.
+// Rows past N and samples past K are zero.  "Paired" rows: of each 64 rows the even ones are one
+// group and the odd ones the next, so that a lane's outputs in the two column groups of its
+// wave are neighbours in memory.
 #pragma once
 #include "herk_fp8.h"
 
@@ -15,11 +17,16 @@ namespace ftdx {
 
 constexpr int kFragBytes = 1536;
 
+// Row groups of N rows (whole blocks of 64); row r's group, and its lane in it.
+__host__ __device__ inline int frag_groups(int N) { return (N + 63) / 64 * 2; }
+__host__ __device__ inline int frag_group(int r, bool paired) { return paired ? (r >> 6) * 2 + (r & 1) : r >> 5; }
+__host__ __device__ inline int frag_lane(int r, bool paired) { return paired ? (r & 63) >> 1 : r & 31; }
+
 // 32-sample steps of a row of K samples (whole 64-sample stages).
 inline int frag_steps(int K) { return (K + 63) / 64 * 2; }
 // Bytes of one batch's fragment rows (nseg segments of K samples per row).
 inline int64_t frag_rows_bytes(int N, int K, int nseg = 1) {
-    return (int64_t)((N + 31) / 32) * frag_steps(K) * nseg * kFragBytes;
+    return (int64_t)frag_groups(N) * frag_steps(K) * nseg * kFragBytes;
 }
 
 // Whether the pipelined HERK takes this problem: 16-byte row loads (K >= 16) and one
@@ -29,10 +36,11 @@ bool pipe_supported(int N, int K, int nseg = 1);
 // QC rows [batches][N][K] (any K >= 16, any alignment) -> fragment rows.  Input batch
 // (ob * nseg + s) * seg_group + i becomes segment s of output batch ob * seg_group + i.
 hipError_t launch_qc_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, int batches, int nseg, int seg_group,
-                               hipStream_t stream);
+                               bool paired, hipStream_t stream);
 
 // The HERK over fragment rows: a.A the rows, a.a_bstride their bytes per batch, a.K the
 // samples of one segment (a.nseg of them); packed lower triangle as launch_herk_int4_plain.
+// The rows are paired where pipe_nontemporal(a.K * a.nseg, out_fp16).
 hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t stream);
 
 // GGP bytes [batches][K][N], any alignment -> fragment rows; the HERK over them with the GGP
@@ -56,10 +64,10 @@ struct PipeProblem {
     uint8_t* rows;     // their fragment rows, 16-byte aligned
     void* C;
     int N, K, steps;   // steps: max(frag_steps(K), 2)
-    int nt;            // pipe_nontemporal
+    int nt;            // pipe_nontemporal: non-temporal stores, paired rows
     float alpha, beta;
 };
-// Segments from `first` of problem `prob`: (N rounded up to 32) * 2 steps of them in all.
+// Segments from `first` of problem `prob`: 32 frag_groups(N) * 2 steps of them in all.
 constexpr int kConvThreads = 2048;
 struct ConvBlock {
     int prob;

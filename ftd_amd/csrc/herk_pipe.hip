@@ -193,8 +193,12 @@ __device__ __forceinline__ void store_ggp_inside(OutT* C, int N, int w, int col,
 #pragma unroll
             for (int y = 0; y < 2; ++y)
 #pragma unroll
-                for (int q = 0; q < 16; ++q)
-                    p[y * 32 + (q >> 2) * 8 + (q & 3)] = Elem<OutT>::make(re[x][y][q], -im[x][y][q]);
+                for (int q = 0; q < 16; ++q) {
+                    float r = re[x][y][q], m = -im[x][y][q];
+                    // converted anew: kept from the first loop, FP64 values would spill
+                    if constexpr (sizeof(OutT) == 8) __asm__ __volatile__("" : "+v"(r), "+v"(m));
+                    p[y * 32 + (q >> 2) * 8 + (q & 3)] = Elem<OutT>::make(r, m);
+                }
         }
     }
 }
@@ -233,7 +237,7 @@ __device__ __forceinline__ void pipe_tile(uint8_t* lds, const uint8_t* base, int
     const int wrow = I * PT + wm * 64, wcol = J * PT + wn * 64;
     const bool active = wrow < N && wrow + 63 >= wcol;
     // groups past N (edge tiles) read the last group; their products are not stored
-    const int ng = (N + 31) / 32;
+    const int ng = frag_groups(N);
     uint32_t off[P_LOADS];
 #pragma unroll
     for (int q = 0; q < P_LOADS; ++q) {
@@ -270,12 +274,14 @@ __device__ __forceinline__ void pipe_tile(uint8_t* lds, const uint8_t* base, int
         else store_ggp_any<OutT, FMT>(C, N, wrow, wcol, re, im, lane);
     } else if (inside && beta == 0.0f) {
         if (nt) {
-            if (alpha == 1.0f) store_inside<OutT, false, true>(C, wrow, wcol, alpha, re, im, lane);
-            else store_inside<OutT, true, true>(C, wrow, wcol, alpha, re, im, lane);
+            if (alpha == 1.0f) store_pairs<OutT, false, true>(C, wrow, wcol, alpha, re, im, lane);
+            else store_pairs<OutT, true, true>(C, wrow, wcol, alpha, re, im, lane);
         } else {
             if (alpha == 1.0f) store_inside<OutT, false, false>(C, wrow, wcol, alpha, re, im, lane);
             else store_inside<OutT, true, false>(C, wrow, wcol, alpha, re, im, lane);
         }
+    } else if (nt) {
+        store_any<OutT, true>(C, N, wrow, wcol, alpha, beta, re, im, lane);
     } else {
         store_any<OutT>(C, N, wrow, wcol, alpha, beta, re, im, lane);
     }
@@ -369,22 +375,24 @@ __device__ __forceinline__ void put_frag(uint4 w, uint8_t* dst, int lane) {
     put_codes(re, im, dst, lane);
 }
 
-// Row and 16-sample segment of conversion thread t: waves of S segments x 64 / S rows.
-__device__ __forceinline__ void conv_place(uint32_t t, int segs, int S, int& r, int& s) {
+// Row and 16-sample segment of conversion thread t: waves of S segments x 64 / S rows, of one parity
+// where paired.
+__device__ __forceinline__ void conv_place(uint32_t t, int segs, int S, bool paired, int& r, int& s) {
     const uint32_t v = t / 64u, per = (uint32_t)(segs / S);
     const uint32_t rb = v / per, sb = v - rb * per;
     s = (int)sb * S + (int)(t % S);
-    r = (int)rb * (64 / S) + (int)(t / S % (64 / S));
+    const int R = 64 / S, u = (int)(t / S) % R;
+    r = paired ? (int)(rb >> 1) * 2 * R + 2 * u + (int)(rb & 1) : (int)rb * R + u;
 }
 
 // VEC: K % 16 == 0 and 16-byte aligned rows
 template <bool VEC, int S>
 __global__ void __launch_bounds__(256)
 qc_frag_rows_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int N, int K, int steps, int nseg,
-                    int grp) {
-    const int ng = (N + 31) / 32;
+                    int grp, bool paired) {
+    const int ng = frag_groups(N);
     int r, s;
-    conv_place(blockIdx.x * 256u + threadIdx.x, steps * 2, S, r, s);
+    conv_place(blockIdx.x * 256u + threadIdx.x, steps * 2, S, paired, r, s);
     if (r >= ng * 32) return;
     const int ib = (int)blockIdx.y, ob = ib / (nseg * grp), sg = ib / grp - ob * nseg;
     const int64_t dst_batch = (int64_t)ob * grp + ib % grp;
@@ -397,8 +405,9 @@ qc_frag_rows_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, i
             w = row_segment(row, s * 16, K);
         }
     }
-    put_frag(w, out + ((dst_batch * ng + (r >> 5)) * (int64_t)(steps * nseg) + sg * steps + (s >> 1)) * kFragBytes,
-             (r & 31) + 32 * (s & 1));
+    put_frag(w,
+             out + ((dst_batch * ng + frag_group(r, paired)) * (int64_t)(steps * nseg) + sg * steps + (s >> 1)) * kFragBytes,
+             frag_lane(r, paired) + 32 * (s & 1));
 }
 
 // The rows of many problems: workgroup b converts up to kConvThreads segments of one problem.
@@ -406,11 +415,11 @@ __global__ void __launch_bounds__(256)
 qc_frag_rows_multi_kernel(const PipeProblem* __restrict__ probs, const ConvBlock* __restrict__ blocks) {
     const ConvBlock cb = blocks[blockIdx.x];
     const PipeProblem p = probs[cb.prob];
-    const int ng = (p.N + 31) / 32, segs = p.steps * 2, S = segs % 8 == 0 ? 8 : 4;
+    const int ng = frag_groups(p.N), segs = p.steps * 2, S = segs % 8 == 0 ? 8 : 4;
     const bool vec = p.K % 16 == 0 && (reinterpret_cast<uintptr_t>(p.A) & 15u) == 0;
     for (uint32_t i = threadIdx.x; i < (uint32_t)kConvThreads; i += 256u) {
         int r, s;
-        conv_place(cb.first + i, segs, S, r, s);
+        conv_place(cb.first + i, segs, S, p.nt, r, s);
         if (r >= ng * 32) return;
         uint4 w = make_uint4(0u, 0u, 0u, 0u);
         if (r < p.N) {
@@ -425,7 +434,8 @@ qc_frag_rows_multi_kernel(const PipeProblem* __restrict__ probs, const ConvBlock
                 w = make_uint4(d[0], d[1], d[2], d[3]);
             }
         }
-        put_frag(w, p.rows + ((int64_t)(r >> 5) * p.steps + (s >> 1)) * kFragBytes, (r & 31) + 32 * (s & 1));
+        put_frag(w, p.rows + ((int64_t)frag_group(r, p.nt) * p.steps + (s >> 1)) * kFragBytes,
+                 frag_lane(r, p.nt) + 32 * (s & 1));
     }
 }
 
@@ -436,7 +446,7 @@ qc_frag_rows_multi_kernel(const PipeProblem* __restrict__ probs, const ConvBlock
 template <bool ALIGNED>
 __global__ void __launch_bounds__(256)
 ggp_frag_rows_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int N, int K, int steps, int batches) {
-    const int tid = threadIdx.x, ng = (N + 31) / 32;
+    const int tid = threadIdx.x, ng = frag_groups(N);
     const int r0 = ((int)blockIdx.y * 64 + (tid & 15) + 16 * (tid >> 6)) * 4;
     const int s = (int)blockIdx.x * 4 + ((tid >> 4) & 3);  // whole stages: s < 2 steps
     if (r0 >= ng * 32) return;
@@ -523,27 +533,27 @@ hipError_t launch_herk_pipe_grouped(const PipeProblem* probs, const GroupItemDev
 }
 
 hipError_t launch_qc_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, int batches, int nseg, int seg_group,
-                               hipStream_t stream) {
+                               bool paired, hipStream_t stream) {
     if (N <= 0 || batches <= 0) return hipSuccess;
     if (!pipe_supported(N, K, nseg) || batches > 65535) return hipErrorInvalidValue;
-    const int steps = frag_steps(K), segs = steps * 2, rows = (N + 31) / 32 * 32;
+    const int steps = frag_steps(K), segs = steps * 2, rows = frag_groups(N) * 32;
     const bool vec = K % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
     const dim3 grid((unsigned)(((int64_t)rows * segs + 255) / 256), (unsigned)batches), block(256);
     // 8 segments per wave where a row's segments allow it (whole stages have 4)
     if (segs % 8 == 0) {
         if (vec)
             hipLaunchKernelGGL((qc_frag_rows_kernel<true, 8>), grid, block, 0, stream, in, out, N, K, steps, nseg,
-                               seg_group);
+                               seg_group, paired);
         else
             hipLaunchKernelGGL((qc_frag_rows_kernel<false, 8>), grid, block, 0, stream, in, out, N, K, steps, nseg,
-                               seg_group);
+                               seg_group, paired);
     } else {
         if (vec)
             hipLaunchKernelGGL((qc_frag_rows_kernel<true, 4>), grid, block, 0, stream, in, out, N, K, steps, nseg,
-                               seg_group);
+                               seg_group, paired);
         else
             hipLaunchKernelGGL((qc_frag_rows_kernel<false, 4>), grid, block, 0, stream, in, out, N, K, steps, nseg,
-                               seg_group);
+                               seg_group, paired);
     }
     return hipGetLastError();
 }
