@@ -340,13 +340,16 @@ hipError_t run_padded(ftdx_context* ctx, const HerkPlainArgs& a, int cfg, int ou
 // ---- pipelined HERK over E3M2 fragment rows (herk_pipe.h) ----
 // Chunks of batches as on the pre-cast paths, for the same reason; at most 160 MB, so that a
 // chunk's rows and its output share the 256 MB memory-side cache and the next chunk's rows
-// overwrite them there (headline 4.13 ms; 320 MB 4.23, 96 MB 4.21, 48 MB 4.58; 1024 inputs x
-// 286, K = 2048: 1.02 against 1.12 ms for 320 MB).
+// overwrite them there, and at most 80 MB where that makes two chunks of what would be one.  us
+// for 160 / 80 / 48 MB, buffers in turn: 4096 x 96, K = 2048 4116 / 4253 / 4405; 1024 x 200, K = 2048
+// 744 / 891 / 892; 1152 x 66, K = 1024 (117 MB in all) 196 / 180 / 202; 700 x 60, K = 2000, FP16
+// (130 MB) 141 / 137 / 152; 1024 x 64, K = 1024 (101 MB) 150 / 147 / 171.
 constexpr size_t kFragChunkBytes = size_t(160) << 20;
 
 int frag_chunk_cap(int N, int K, int nseg, int batch) {
     const size_t per = (size_t)frag_rows_bytes(N, K, nseg);
-    return std::min(chunk_cap_bytes(per, batch, kFragChunkBytes), 65535 / std::max(nseg, 1));
+    const size_t limit = per * (size_t)std::max(batch, 1) <= kFragChunkBytes ? kFragChunkBytes / 2 : kFragChunkBytes;
+    return std::min(chunk_cap_bytes(per, batch, limit), 65535 / std::max(nseg, 1));
 }
 
 size_t frag_scratch_bytes(const HerkPlainArgs& a) {
@@ -395,7 +398,7 @@ hipError_t run_pipe(uint8_t* rows, const HerkPlainArgs& a, bool fp16, hipStream_
     for (int u0 = 0; u0 < units; u0 += chunk) {
         const int nu = std::min(chunk, units - u0);
         hipError_t e = launch_qc_frag_rows(a.A + (int64_t)u0 * in_per * a.a_bstride, rows, a.N, a.K, nu * in_per,
-                                           a.nseg, grp, !grid && pipe_nontemporal(a.K * a.nseg, fp16), st);
+                                           a.nseg, grp, !grid && pipe_nontemporal(a.N, a.K * a.nseg, fp16), st);
         if (e != hipSuccess) return e;
         HerkPlainArgs b = a;
         b.A = rows;
@@ -457,17 +460,22 @@ bool worth_direct(int N, int K, int batch) {
 // The kernel of an INT4 call that nobody tuned or forced: the direct one, the pipelined one, or
 // the fused 128 x 128 tile, by estimates in microseconds.  Each kernel is its launches, then the
 // longest of one workgroup's chain of 64-sample stages, all workgroups' stages over the chip's
-// 512 workgroup slots, and the output at the rate it stores (faster while it fits the memory-side cache);
-// the conversion and padding passes move their bytes at 5 TB/s.  The constants are fits to (us: direct / pipelined / fused)
+// 512 workgroup slots, and the output at the rate it stores (faster while it fits the memory-side
+// cache); the padding pass moves its bytes at 5 TB/s, the conversion its 2.5 per sample and what the
+// multiply then waits for its rows, 3.2 in all.  The constants are fits to (us: direct / pipelined / fused)
 //   128 x 20, K 1024:   7.8 /  18 /  21     512 x 5,  K 4000:   30 / 47 / 59
 //   2000 x 1, K 1024:    20 /  20 /  21     2000 x 1, K 4000:   89 / 45 / 60
 //   512 x 20, K 1024:     - /  29 /  22     512 x 1144, K 1024:  - / 824 / 744
 //   1024 x 286, K 2048:   - / 1022 / 1098   2624 x 43, K 128:    - / 295 / 320
 //   4096 x 96, K 2048:    - / 4134 / 5460
+// and, three sets of buffers in turn,
+//   1152 x 66, K 1024:    - / 180 / 188     1024 x 64, K 1024:   - / 147 / 145
+//   700 x 60, K 2000:     - / 137 / 132     512 x 100, K 1024:   - / 75 / 64
+//   1500 x 40, K 800:     - / 150 / 180     300 x 100, K 1000:   - / 48 / 53
 // Rows that 16-byte loads cannot take cost the fused tile a padding pass.
 double fused_us(double st, double t128) { return 5.0 + std::max(0.87 * st + 3.0, t128 / 512.0 * (1.55 * st + 6.0)); }
-double pipe_us(double st, double t128, double in) {
-    return 8.0 + in * 2.5 / 5e6 + std::max(0.45 * st + 3.0, t128 / 512.0 * (0.92 * st + 5.7));
+double pipe_us(double st, double t128, double in, double conv) {
+    return 8.0 + in * conv / 5e6 + std::max(0.45 * st + 3.0, t128 / 512.0 * (0.92 * st + 5.7));
 }
 
 int choose_kernel(const void* A, int N, int K, int batch, bool fp16) {
@@ -477,7 +485,7 @@ int choose_kernel(const void* A, int N, int K, int batch, bool fp16) {
     if (!rows_take_vector_loads(A, K)) best += 4.0 + in * 2.0 / 5e6;
     int pick = TILE_128x128_K64_P2;
     if (pipe_supported(N, K)) {
-        const double t = std::max(pipe_us(st, t128, in), 8.0 + in * 2.5 / 5e6 + out / (out < 2e8 ? 5.5e6 : 4.1e6));
+        const double t = std::max(pipe_us(st, t128, in, 3.2), 8.0 + in * 3.2 / 5e6 + out / (out < 2e8 ? 5.5e6 : 4.1e6));
         if (t < best) {
             best = t;
             pick = TILE_PIPE;
@@ -488,12 +496,13 @@ int choose_kernel(const void* A, int N, int K, int batch, bool fp16) {
     return pick;
 }
 
-// The same estimates for the gridding HERK over nseg polarizations (us, fused / pipelined: 64 x 16
+// The same estimates for the gridding HERK over nseg polarizations, whose smaller outputs leave the
+// rows in the memory-side cache: 2.5 bytes per sample (us, fused / pipelined: 64 x 16
 // channels, K = 2 x 1024 89 / 75; 512 x 8, 2 x 512 106 / 102; 100 x 16, 2 x 64 62 / 63).
 bool grid_pipe_pays(const HerkPlainArgs& a) {
     const double st = (double)((a.K + 63) / 64) * a.nseg, t128 = (double)pipe_tiles(a.N) * a.batch;
     return pipe_supported(a.N, a.K, a.nseg) && t128 <= 0x7FFFFFFF &&
-           pipe_us(st, t128, (double)a.N * a.K * a.nseg * a.batch) < fused_us(st, t128);
+           pipe_us(st, t128, (double)a.N * a.K * a.nseg * a.batch, 2.5) < fused_us(st, t128);
 }
 
 // Whether a half plane (herk_grid.h) saves more scattered atomics than its own passes cost: from
@@ -514,7 +523,7 @@ bool half_grid_pays(int N, int Ng, int n_chan) {
 // flag = TILE_BF6: the E3M2 variants, each timed with its conversion pass into the
 // context's pre-cast rows (already sized by the caller).
 int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStream_t s,
-             const TuneKey& key, TuneEntry& best, int flag, const HerkPlainArgs* qc_args, uint8_t* frag) {
+             const TuneKey& key, TuneEntry& best, int flag, const HerkPlainArgs* qc_args, uint8_t* frag, bool padded) {
     HerkPlainArgs a = a0;
     void* scratch = nullptr;
     hipError_t e;
@@ -539,6 +548,10 @@ int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStrea
             b.C = a.C;
             return cfg == TILE_PIPE ? run_pipe(frag, b, out_fp16, s) : launch_herk_direct(b, out_fp16, s);
         }
+        if (padded && qc_args) {  // the tiles' padding pass, as every call runs it
+            hipError_t pe = launch_pad_qc_rows(qc_args->A, ctx->precast, (int64_t)a.N * a.batch, qc_args->K, a.K, s);
+            if (pe != hipSuccess) return pe;
+        }
         if (!(cfg & TILE_BF6)) return launch_herk_int4_plain(a, cfg, out_fp16, remap, s);
         return run_precast(ctx, a, FTDX_INPUT_INT4, true, tile_base(cfg), out_fp16, remap, s);
     };
@@ -558,6 +571,12 @@ int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStrea
         float ms = 0.0f;
         (void)hipEventElapsedTime(&ms, t0, t1);
         return ms / reps;
+    };
+    // Repeated on the same buffers, the pipelined kernel finds its rows in the memory-side cache;
+    // a program whose buffers change pays for them what 0.7 bytes per sample take at 5 TB/s
+    // (1024 x 64, K = 1024: 130 us repeated, 147 with three sets of buffers in turn).
+    auto later = [&](int cfg) {
+        return cfg == TILE_PIPE ? (float)((double)qc_args->N * qc_args->K * qc_args->batch * 0.7 / 5e9) : 0.0f;
     };
     // first pass: every (configuration, workgroup order), one warm-up launch each
     struct Cand {
@@ -580,7 +599,7 @@ int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStrea
             (cfg == TILE_DIRECT && !worth_direct(a.N, qc_args->K, qc_args->batch)) || time_cand(cfg, 1, 1) < 0.0f)
             continue;
         const float ms = time_cand(cfg, 1, 3);
-        if (ms >= 0.0f) cands.push_back({cfg, 1, ms});
+        if (ms >= 0.0f) cands.push_back({cfg, 1, ms + later(cfg)});
     }
     best.ms = 1e30f;
     best.cfg = kDefaultCfg | flag;
@@ -595,7 +614,7 @@ int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStrea
             for (size_t q = 0; q < nf; ++q) {
                 const size_t i = pass == 0 ? q : nf - 1 - q;
                 const float ms = time_cand(cands[i].cfg, cands[i].remap, 3);
-                sum[i] += ms < 0.0f ? 1e30f : ms;
+                sum[i] += ms < 0.0f ? 1e30f : ms + later(cands[i].cfg);
             }
         for (size_t i = 0; i < nf; ++i)
             if (sum[i] / 2 < best.ms) {
@@ -1228,9 +1247,6 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
     const bool may_pipe = may_route && ftdx::pipe_supported(N, K);
     const bool tune_now = tune && !cached && !explicit_cfg && !precast;
     if (may_route && !cached) cfg = ftdx::choose_kernel(A, N, K, batch_count, fp16);
-    // pre-cast rows: loads two stages ahead (FP16 input 1664 x 16, K = 512: 67 against 73 us;
-    // 4096 x 8, K = 2048: 484 against 489; 1024 x 32, K = 300: 54 both)
-    if (precast && !cached && !explicit_cfg) cfg = ftdx::TILE_128x128_K64_P2;
     uint8_t* frag = nullptr;
     if (may_pipe && (cfg == ftdx::TILE_PIPE || tune_now))
         frag = ftdx::frag_scratch(ctx, ftdx::frag_scratch_bytes(a), s);
@@ -1263,7 +1279,7 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
         }
         ftdx::HerkPlainArgs tp = a;
         tp.batch = t.batch;
-        if (ftdx::autotune(ctx, t, fp16, s, key, best, e3m2 ? ftdx::TILE_BF6 : 0, may_route ? &tp : nullptr, frag) == FTDX_OK) {
+        if (ftdx::autotune(ctx, t, fp16, s, key, best, e3m2 ? ftdx::TILE_BF6 : 0, may_route ? &tp : nullptr, frag, padded) == FTDX_OK) {
             cfg = best.cfg;
             if (ctx->forced_remap < 0) remap = best.xcd_remap;
         }

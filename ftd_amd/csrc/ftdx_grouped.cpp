@@ -206,7 +206,7 @@ int grouped_build_pipe(ftdx_grouped_plan* P, const ftdx_herk_problem* problems, 
         p.N = q.N;
         p.K = q.K;
         p.steps = frag_steps(kq);
-        p.nt = pipe_nontemporal(q.K, out_fp16 != 0);
+        p.nt = pipe_nontemporal(q.N, q.K, out_fp16 != 0);
         p.alpha = q.alpha;
         p.beta = q.beta;
         probs.push_back(p);

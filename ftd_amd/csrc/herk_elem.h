@@ -65,6 +65,10 @@ __device__ __forceinline__ void store_inside(OutT* C, int w, int col, float alph
     uint8_t* base = reinterpret_cast<uint8_t*>(reinterpret_cast<v2*>(C) + tri_index(w, col));
     uint32_t off = (uint32_t)(g4 * w + g4 * (g4 + 1) / 2 + n) * ES;
     const uint32_t step = (uint32_t)(w + g4) * ES;  // row d + g4 -> d + 1 + g4 adds step + (d + 1) ES
+    // Where a kernel holds both forms the compiler would otherwise merge them into one of plain
+    // stores, or compute the offsets and elements of both ahead of the choice and spill them.
+    if constexpr (NT) __asm__ __volatile__("; non-temporal stores" : "+v"(off), "+v"(alpha));
+    else __asm__ __volatile__("; plain stores" : "+v"(off), "+v"(alpha));
 #pragma unroll
     for (int x = 0; x < FM; ++x)
 #pragma unroll
@@ -80,6 +84,7 @@ __device__ __forceinline__ void store_inside(OutT* C, int w, int col, float alph
             }
             off += (q & 3) != 3 ? step + (uint32_t)(d + 1) * ES : 5 * step + (uint32_t)(5 * d + 15) * ES;
         }
+    if constexpr (NT) __asm__ __volatile__("; stored");
 }
 
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));

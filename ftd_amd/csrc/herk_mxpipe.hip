@@ -260,7 +260,7 @@ hipError_t launch_herk_mxpipe(const HerkPlainArgs& a, int fmt, bool out_fp16, hi
     if (a.N <= 0 || a.batch <= 0) return hipSuccess;
     const int tiles = pipe_tiles(a.N), nst = (a.K + 63) / 64;
     if ((int64_t)tiles * a.batch > 0x7FFFFFFF || !mxpipe_supported(a.N, a.K, fmt)) return hipErrorInvalidValue;
-    const bool nt = pipe_nontemporal(a.K, out_fp16);
+    const bool nt = pipe_nontemporal(a.N, a.K, out_fp16);
     if (fmt == MX_FP4_E2M1) {
         if (out_fp16) launch<MX_FP4_E2M1, _Float16>(a, nst, tiles, nt, s);
         else launch<MX_FP4_E2M1, float>(a, nst, tiles, nt, s);

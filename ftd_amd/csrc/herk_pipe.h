@@ -40,7 +40,7 @@ hipError_t launch_qc_frag_rows(const uint8_t* in, uint8_t* out, int N, int K, in
 
 // The HERK over fragment rows: a.A the rows, a.a_bstride their bytes per batch, a.K the
 // samples of one segment (a.nseg of them); packed lower triangle as launch_herk_int4_plain.
-// The rows are paired where pipe_nontemporal(a.K * a.nseg, out_fp16).
+// The rows are paired where pipe_nontemporal(a.N, a.K * a.nseg, out_fp16).
 hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t stream);
 
 // GGP bytes [batches][K][N], any alignment -> fragment rows; the HERK over them with the GGP
@@ -56,7 +56,7 @@ int pipe_tiles(int N);
 int pipe_wg_per_cu();
 
 // Whether the stores of the launch above are non-temporal (samples: of all segments).
-bool pipe_nontemporal(int samples, bool out_fp16);
+bool pipe_nontemporal(int N, int samples, bool out_fp16);
 
 // ---- many problems of different sizes ----
 struct PipeProblem {

@@ -510,11 +510,17 @@ int pipe_tiles(int N) {
 int pipe_wg_per_cu() { return P_WG_PER_CU; }
 
 // Plain stores let the L2 join the partial lines at the ends of the runs, and fill it with
-// output in place of operand rows: they pay where the launch writes more than it multiplies.
-// Both at 4096 inputs x 17, FP32: K = 256 295 (plain) / 382 us (non-temporal), 384 336 / 378,
-// 512 402 / 371, 1024 566 / 423; FP16: 128 142 / 245, 256 202 / 237, 384 245 / 221, 512
-// 286 / 233 us.
-bool pipe_nontemporal(int samples, bool out_fp16) { return samples > (out_fp16 ? 320 : 448); }
+// output in place of operand rows: they pay where the launch writes more than it multiplies,
+// the longer the longer the output's rows.  us, plain / non-temporal (paired rows), buffers in turn:
+//   FP32, K =      128         256         384         512
+//   512 x 400   115 / 134   147 / 146   179 / 156   213 / 181
+//   1664 x 100  269 / 321   293 / 327   386 / 333   452 / 341
+//   4000 x 12   190 / 237   192 / 239   218 / 239   261 / 240
+//   FP16
+//   512 x 400    70 / 86     95 / 100   127 / 118   170 / 156
+//   1664 x 100  156 / 200   220 / 202   274 / 216   322 / 244
+//   4000 x 12    94 / 147   125 / 152   152 / 152   172 / 154
+bool pipe_nontemporal(int N, int samples, bool out_fp16) { return samples > (!out_fp16 && N >= 3000 ? 448 : 320); }
 
 hipError_t launch_qc_frag_rows_multi(const PipeProblem* probs, const ConvBlock* blocks, int nblocks, hipStream_t s) {
     if (nblocks <= 0) return hipSuccess;
@@ -576,7 +582,7 @@ hipError_t launch_herk_pipe(const HerkPlainArgs& a, bool out_fp16, hipStream_t s
     if (blocks > 0x7FFFFFFF || !pipe_supported(a.N, a.K, a.nseg)) return hipErrorInvalidValue;
     const int steps = frag_steps(a.K) * a.nseg;
     const dim3 grid((unsigned)blocks), block(P_THREADS);
-    const bool nt = pipe_nontemporal(a.K * a.nseg, out_fp16);
+    const bool nt = pipe_nontemporal(a.N, a.K * a.nseg, out_fp16);
     if (out_fp16) {
         if (nt)
             hipLaunchKernelGGL((herk_pipe_kernel<_Float16, true>), grid, block, 0, stream, a, steps, tiles);

@@ -1323,23 +1323,27 @@ struct TileRunner {
             return;
         }
         if constexpr (FMT == OUT_LOWER_PACKED) {
-            // A tile inside the matrix and below the diagonal stores straight from its accumulators.
-            // Plain stores, which the L2 joins to whole lines, up to 1024 samples on the larger
-            // tiles; us of staged / non-temporal / plain stores, 128 x 128 tiles: FP16 rows of 1024
-            // x 32, K = 300, FP32 67 / 66 / 54; QC 1664 x 64, K = 128, FP16 129 / 145 / 109; QC
-            // 2048 x 16, K = 512, FP32 89 / 91 / 84; FP16 rows of 4096 x 8, K = 2048, FP16 504 /
-            // 484 / 491.  64 x 64 tiles write shorter runs: the second 235 / 151 / 183, the third
-            // 172 / 140 / 156.
-            if (j.beta == 0.0f && j.row0 + Cfg::TM <= j.N && j.col0 + Cfg::TN <= j.row0) {
+            // A tile inside the matrix and below the diagonal stores straight from its accumulators
+            // where the output is narrow or the samples few; on more samples FP32 rows leave faster
+            // as the staged epilogue's longer runs.  Plain stores, which the L2 joins to whole
+            // lines, up to 320 samples.  us of staged / direct, buffers in turn, 128 x 128 tiles:
+            // FP32 1152 x 66, K = 128 104 / 98; 512 x 100, K = 1024 62 / 66; 1500 x 40, K = 800 168 /
+            // 182; FP16 1664 x 128, K = 128 242 / 200; 1664 x 64, K = 512 209 / 188.  64 x 64 tiles
+            // (not staged, shorter runs) gain at any size: 2048 x 16, K = 512, FP32 172 to 140.
+            const bool direct = j.beta == 0.0f && j.row0 + Cfg::TM <= j.N && j.col0 + Cfg::TN <= j.row0 &&
+                                (!Cfg::EPI_STAGED || sizeof(OutT) == 2 || j.K <= 320);
+            if constexpr (Cfg::EPI_STAGED) {
+                if (!direct) {
+                    epilogue_staged<OutT>(j, lds, acc_re, acc_im, active, wrow0, wcol0, lane, wave);
+                    return;
+                }
+            }
+            if (direct) {
                 OutT* C = static_cast<OutT*>(j.C);
-                if (Cfg::TM < 128 || j.K > 1024) store_inside<OutT, true, true>(C, wrow0, wcol0, j.alpha, acc_re, acc_im, lane);
+                if (Cfg::TM < 128 || j.K > 320) store_inside<OutT, true, true>(C, wrow0, wcol0, j.alpha, acc_re, acc_im, lane);
                 else store_inside<OutT, true, false>(C, wrow0, wcol0, j.alpha, acc_re, acc_im, lane);
                 return;
             }
-        }
-        if constexpr (FMT == OUT_LOWER_PACKED && Cfg::EPI_STAGED) {
-            epilogue_staged<OutT>(j, lds, acc_re, acc_im, active, wrow0, wcol0, lane, wave);
-            return;
         }
         if (!active) return;
 
