@@ -214,7 +214,7 @@ int grouped_build_pipe(ftdx_grouped_plan* P, const ftdx_herk_problem* problems, 
         items += pipe_tiles(q.N);
     }
     size_t free_bytes = 0, all_bytes = 0;
-    if (probs.empty() || items > 0x0FFFFFFF || total > kGroupRowsMax) return FTDX_ERR_UNSUPPORTED;
+    if (probs.empty() || items > 0x07FFFFFF || total > kGroupRowsMax) return FTDX_ERR_UNSUPPORTED;
     if (hipMemGetInfo(&free_bytes, &all_bytes) != hipSuccess || total > free_bytes / 2 ||
         hipMalloc(&P->d_rows, total) != hipSuccess) {
         (void)hipGetLastError();
@@ -257,7 +257,7 @@ int grouped_build_pipe(ftdx_grouped_plan* P, const ftdx_herk_problem* problems, 
     P->items = items;
     P->max_load = *std::max_element(load, load + 8);
     P->mean_load = cost / 8.0;
-    P->num_wg = (int)tiles.size();  // at most 8 items: < 2^31
+    P->num_wg = (int)tiles.size();  // at most 8 per item: < 2^31
     P->conv_blocks = (int)conv.size();
     P->cfg = cfg;
     P->out_fp16 = out_fp16;
