@@ -20,6 +20,7 @@
 #include "ftdx_tune.h"
 #include "herk_fp8.h"
 #include "herk_mx.h"
+#include "herk_chunks.h"
 #include "herk_direct.h"
 #include "herk_grid.h"
 #include "herk_mxpipe.h"
@@ -188,44 +189,12 @@ int device_cu_count() {
     return cus;
 }
 
-// Pre-cast paths (FP16 input, ForceBaseline, E3M2 operands) convert and multiply a chunk
-// of batches at a time: the chunk's operand rows (at most kPrecastChunkBytes) are then
-// still in the memory-side cache when its tiles read them, and the scratch holds one
-// chunk.  Among chunk sizes up to that cap, the one whose launches leave the fewest idle
-// workgroup slots in their last rounds (plus a small cost per launch) wins.
-constexpr size_t kPrecastChunkBytes = size_t(320) << 20;
-
-// batches of `per` scratch bytes each that fit one chunk
-int chunk_cap_bytes(size_t per, int batch, size_t limit = kPrecastChunkBytes) {
-    const size_t cap = per > 0 ? limit / per : (size_t)batch;
-    return (int)std::max<size_t>(1, std::min<size_t>(cap, (size_t)std::max(batch, 1)));
-}
-
 int precast_chunk_cap(int N, int K, int batch) {
     return chunk_cap_bytes((size_t)N * 2 * precast_row_samples(K), batch);
 }
 
 // units_out: output batches per unit of `batch` (a unit is one group of polarization
 // segments on the polarization-sum path)
-int pick_chunk_of(int64_t slots, int64_t tiles, int batch, int cmax) {
-    if (cmax >= batch) return std::max(batch, 1);
-    double best = 1e30;
-    int pick = cmax;
-    for (int c = cmax; c >= 1; --c) {
-        int64_t idle = 0;
-        for (int b0 = 0; b0 < batch; b0 += c) {
-            const int64_t t = tiles * std::min(c, batch - b0);
-            idle += (t + slots - 1) / slots * slots - t;
-        }
-        const double cost = (double)idle / (double)slots + 0.1 * ((batch + c - 1) / c);
-        if (cost < best) {
-            best = cost;
-            pick = c;
-        }
-    }
-    return pick;
-}
-
 int pick_chunk(int cfg, int N, int batch, int cmax, int units_out = 1) {
     const int64_t slots = (int64_t)std::max(device_cu_count(), 1) * tile_config_wg_per_cu(cfg);
     return pick_chunk_of(slots, (int64_t)herk_tiles(cfg, N) * units_out, batch, cmax);
@@ -338,20 +307,6 @@ hipError_t run_padded(ftdx_context* ctx, const HerkPlainArgs& a, int cfg, int ou
 }
 
 // ---- pipelined HERK over E3M2 fragment rows (herk_pipe.h) ----
-// Chunks of batches as on the pre-cast paths, for the same reason; at most 160 MB, so that a
-// chunk's rows and its output share the 256 MB memory-side cache and the next chunk's rows
-// overwrite them there, and at most 80 MB where that makes two chunks of what would be one.  us
-// for 160 / 80 / 48 MB, buffers in turn: 4096 x 96, K = 2048 4116 / 4253 / 4405; 1024 x 200, K = 2048
-// 744 / 891 / 892; 1152 x 66, K = 1024 (117 MB in all) 196 / 180 / 202; 700 x 60, K = 2000, FP16
-// (130 MB) 141 / 137 / 152; 1024 x 64, K = 1024 (101 MB) 150 / 147 / 171.
-constexpr size_t kFragChunkBytes = size_t(160) << 20;
-
-int frag_chunk_cap(int N, int K, int nseg, int batch) {
-    const size_t per = (size_t)frag_rows_bytes(N, K, nseg);
-    const size_t limit = per * (size_t)std::max(batch, 1) <= kFragChunkBytes ? kFragChunkBytes / 2 : kFragChunkBytes;
-    return std::min(chunk_cap_bytes(per, batch, limit), 65535 / std::max(nseg, 1));
-}
-
 size_t frag_scratch_bytes(const HerkPlainArgs& a) {
     const int grp = std::max(a.seg_group, 1);
     return (size_t)frag_rows_bytes(a.N, a.K, a.nseg) * grp * frag_chunk_cap(a.N, a.K, a.nseg * grp, a.batch / grp);
@@ -501,7 +456,7 @@ int choose_kernel(const void* A, int N, int K, int batch, bool fp16) {
 // channels, K = 2 x 1024 89 / 75; 512 x 8, 2 x 512 106 / 102; 100 x 16, 2 x 64 62 / 63).
 bool grid_pipe_pays(const HerkPlainArgs& a) {
     const double st = (double)((a.K + 63) / 64) * a.nseg, t128 = (double)pipe_tiles(a.N) * a.batch;
-    return pipe_supported(a.N, a.K, a.nseg) && t128 <= 0x7FFFFFFF &&
+    return pipe_supported(a.N, a.K, a.nseg) && t128 <= 0x7FFFFFFF && frag_chunk_cap(a.N, a.K, a.nseg, a.batch) > 0 &&
            pipe_us(st, t128, (double)a.N * a.K * a.nseg * a.batch, 2.5) < fused_us(st, t128);
 }
 

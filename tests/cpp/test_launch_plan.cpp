@@ -1,0 +1,36 @@
+// Host-side launch planning of libftdx.so (built with g++ under ASan + UBSan, no GPU): the batches
+// per chunk of the pipelined HERK.  Prints "ALL PASSED" on success.
+#include <cstdio>
+
+#include "herk_chunks.h"
+
+static int g_fail = 0;
+#define CHECK(c)                                                              \
+    do {                                                                      \
+        if (!(c)) {                                                           \
+            std::printf("FAIL %s:%d: %s\n", __FILE__, __LINE__, #c);          \
+            ++g_fail;                                                         \
+        }                                                                     \
+    } while (0)
+
+// Every chunk a loop steps by is at least 1, and a chunk's input batches fit a grid's y dimension;
+// a cap of 0 says that one batch's segments alone do not.
+static void test_chunks() {
+    using namespace ftdx;
+    for (int nseg : {1, 2, 3, 255, 32767, 32768, 65535, 65536, 70000, 1 << 20})
+        for (int batch : {1, 2, 7, 96, 70000}) {
+            const int cap = frag_chunk_cap(64, 16, nseg, batch);
+            CHECK((cap > 0) == (nseg <= 65535));
+            CHECK((int64_t)cap * nseg <= 65535);
+            for (int c : {0, 1, cap}) {
+                const int chunk = pick_chunk_of(512, 3, batch, c);
+                CHECK(chunk >= 1 && chunk <= (c > 1 ? c : 1));
+            }
+        }
+}
+
+int main() {
+    test_chunks();
+    if (g_fail == 0) std::printf("ALL PASSED\n");
+    return g_fail != 0;
+}

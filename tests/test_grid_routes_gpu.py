@@ -1,0 +1,41 @@
+"""ftdx_herk_pol_grid without a forced tile, at the edges of its routes (pipelined kernel, half planes,
+fused tile): bit-exact on integer sums against the CPU oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(N, Ng, seed, cell=2e-3, chan=1):
+    """Baselines of antennas whose UV mostly falls on the grid; frequencies; cell size."""
+    rng = np.random.default_rng(seed)
+    pos = rng.uniform(-0.5, 0.5, (N, 2)) * (0.5 * Ng * cell * 0.2)
+    i, j = np.tril_indices(N)
+    return (pos[i] - pos[j]).astype(np.float32), np.linspace(0.8e9, 1.4e9, chan), cell
+
+
+def _reference(oracle, qc, N, K, chan, pols, uv, freqs, Ng, cell):
+    """The oracle's grid of qc [chan, pols, N, K]."""
+    per = oracle.herk_int64(qc, N, K, chan * pols).reshape(chan, pols, -1, 2).sum(axis=1)
+    assert np.abs(per).max() < 2 ** 24
+    return oracle.pillbox_grid(per.astype(np.float32), uv, freqs, N * (N + 1) // 2, Ng, chan, cell)
+
+
+def test_more_segments_than_a_grid_dimension(oracle, dev):
+    """70000 polarization segments, past the 65535 input batches that one conversion launch takes: the
+    call returns, with the sum of the few segments that are not zero."""
+    import torch
+    from ftd_amd import ftdx
+    N, K, n_pol, Ng = 64, 16, 70000, 64
+    full = [0, 1, 35000, 65535, 65536, 69999]
+    qc = oracle.gen_qc_uniform(5, N * K * len(full)).reshape(len(full), N, K)
+    uv, freqs, cell = _scene(N, Ng, 1)
+    A = torch.zeros((n_pol, N, K), dtype=torch.uint8, device=dev)
+    A[full] = torch.from_numpy(qc).to(dev)
+    grid = torch.zeros((1, Ng, Ng, 2), device=dev)
+    uv_d, f_d = torch.from_numpy(uv).to(dev), torch.from_numpy(freqs).to(dev)
+    ftdx.herk_pol_grid(ftdx.CutlassComplexGemm(), A, N, K, 1, n_pol, uv_d, f_d, grid, Ng, cell)
+    torch.cuda.synchronize()
+    ref = _reference(oracle, qc.reshape(-1), N, K, 1, len(full), uv, freqs, Ng, cell)
+    assert np.abs(ref).sum() > 0
+    assert np.array_equal(grid.cpu().numpy(), ref)
