@@ -1506,10 +1506,14 @@ int ftdx_herk_pol_grid(ftdx_context* ctx, const void* A, int N, int K, int n_cha
     a.freq_offset = freq_offset;
     a.Ng = Ng;
     a.cell = cell_size_rad;
-    const int cfg = ctx->forced_cfg >= 0 ? ftdx::tile_base(ctx->forced_cfg)
-                                         : (ftdx::direct_tile_to_cfg(ctx->direct_tile) >= 0
-                                                ? ftdx::direct_tile_to_cfg(ctx->direct_tile)
-                                                : ftdx::kDefaultCfg);
+    int cfg = ctx->forced_cfg >= 0 ? ftdx::tile_base(ctx->forced_cfg)
+                                   : (ftdx::direct_tile_to_cfg(ctx->direct_tile) >= 0
+                                          ? ftdx::direct_tile_to_cfg(ctx->direct_tile)
+                                          : ftdx::kDefaultCfg);
+    // One wave of a 64 x 64 tile grids all of its rows; a 128 x 128 tile of no more than 128 inputs has
+    // four to share them (us, 64 / 128 tile: 64 x 1, K = 64 49 / 21; 100 x 1, K = 2 x 512 67 / 49; 128 x 1,
+    // K = 2 x 64 52 / 44; from 200 on the smaller tiles win, 2 x 512 x 256 on 1024^2 53 / 67)
+    if (cfg == ftdx::TILE_64x64_K64 && N <= 128) cfg = ftdx::TILE_128x128_K64;
     const int remap = ctx->forced_remap >= 0 ? ctx->forced_remap : ftdx::kDefaultRemap;
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e;

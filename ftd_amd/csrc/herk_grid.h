@@ -56,54 +56,88 @@ __device__ __forceinline__ int64_t grid_cell(int Ng, float x, float y) {
 
 typedef float uv_pair __attribute__((ext_vector_type(2), aligned(4)));
 
-// LDS bytes of one wave below: 16 rows of 32 FN columns, [re, im].
-template <int FN>
-constexpr int grid_lds_bytes() { return 16 * (32 * FN * 8 + 16); }
+// LDS bytes of one wave below: 16 rows of 64 columns, [re, im].
+constexpr int kGridRegion = 16 * (64 * 8 + 16);
 
-// Elements (i, j <= i), i < N, of the block at (w, col), times alpha; Im = 0 on the diagonal.
-// UV in wavelengths = float(uv_m / lambda) (double division).  Whole waves call it.  The block
-// goes through LDS 16 rows at a time so that a loop over elements can serve them all: unrolled
+// Elements (i, j <= i), i < N, of the tile at (row0, col0), times alpha; Im = 0 on the diagonal.
+// UV in wavelengths = float(uv_m / lambda) (double division).  Every wave of the workgroup calls it,
+// W of them in rows of WN, each with the 64 x 64 block of its place (active: it has elements).  The
+// blocks go through LDS 16 rows at a time so that a loop over rows can serve them all: unrolled
 // over the accumulators the cell arithmetic is 64 bodies, past the instruction cache, and the UV
 // loads of few resident waves were waited for one by one.  Eight at a time against four: 128 x 4
 // channels, K = 2 x 512, 68 against 73 us; 1024 x 8 308 against 304.
-template <int FM, int FN>
-__device__ __forceinline__ void grid_block(const GridJob& g, int N, int w, int col, float alpha,
-                                           const v16f (&re)[FM][FN], const v16f (&im)[FM][FN], uint8_t* lds, int lane) {
-    constexpr int COLS = 32 * FN, PITCH = COLS * 8 + 16, BATCH = 8;  // BATCH: UV loads in flight
+// What bounds launches of few tiles is one wave's instructions, about 250 a row.  Where every wave has
+// 64 rows each takes its own; on the diagonal and at the matrix's edge, where some have few or none,
+// the workgroup shares the rows that exist, and rows without an element are skipped (us, each wave its
+// own 64 / shared: 48 x 1 channel, K = 64 40 / 17; 64 x 16, K = 2 x 512 58 / 30; 128 x 16 61 / 54;
+// 256 x 8 73 / 74; 1024 x 8 307 / 300).
+template <int W, int WN, int FM, int FN>
+__device__ __forceinline__ void grid_tile(const GridJob& g, int N, int row0, int col0, bool active, float alpha,
+                                          const v16f (&re)[FM][FN], const v16f (&im)[FM][FN], uint8_t* lds, int wave,
+                                          int lane) {
+    static_assert(FM == 2 && FN == 2 && 16 % W == 0, "blocks of 64 x 64, whole rows per wave");
+    constexpr int PITCH = 64 * 8 + 16, BATCH = 8;  // BATCH: UV loads in flight
+    const bool shared = col0 + WN * 64 > row0 || row0 + W / WN * 64 > N;
     const float half_ng = 0.5f * g.Ng;
     const int64_t sum = mirror_sum(g.Ng);
     const double y = 1.0 / g.lambda;
     const bool plain = !(__builtin_fabs(g.lambda) > 1e-100 && __builtin_fabs(g.lambda) < 1e100);
     const int n = lane & 31, g4 = (lane >> 5) * 4;
+    uint8_t* mine = lds + wave * kGridRegion;
+    // A wave's 16 rows go in groups of R.  Shared: a group or two of every block, of another part of
+    // each, so that a lane still meets at most one element of the diagonal.
+    constexpr int PART = 16 / W, R = PART < BATCH ? PART : BATCH;
+    auto place = [&](int q, int& i, int& j, int& at) {  // group q: first row of its rows, first column, LDS
+        const int r = shared ? q / (PART / R) : wave;
+        const int row = shared ? ((wave + r) & (W - 1)) * PART + q % (PART / R) * R : q * R;
+        i = r / WN * 64 + row;
+        j = col0 + r % WN * 64;
+        at = r * kGridRegion + row * PITCH;
+    };
+    auto wait = [&] {
+        if (shared) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();
+    };
     float* auto_at = nullptr;  // a lane meets at most one element of the diagonal
     float auto_re = 0.0f;
 #pragma unroll
     for (int x = 0; x < FM; ++x)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
+            const int first = x * 32 + h * 16;  // of each block's rows
+            if (row0 + first >= N) continue;    // the same for the workgroup
+            if (active) {
 #pragma unroll
-            for (int y = 0; y < FN; ++y)
+                for (int y = 0; y < FN; ++y)
 #pragma unroll
-                for (int q = 8 * h; q < 8 * h + 8; ++q)
-                    *reinterpret_cast<float2*>(lds + ((q >> 2) * 8 + g4 + (q & 3) - 16 * h) * PITCH + (y * 32 + n) * 8) =
-                        make_float2(re[x][y][q] * alpha, im[x][y][q] * alpha);
-            __builtin_amdgcn_wave_barrier();
+                    for (int q = 8 * h; q < 8 * h + 8; ++q)
+                        *reinterpret_cast<float2*>(mine + ((q >> 2) * 8 + g4 + (q & 3) - 16 * h) * PITCH + (y * 32 + n) * 8) =
+                            make_float2(re[x][y][q] * alpha, im[x][y][q] * alpha);
+            }
+            wait();
 #pragma unroll 1
-            for (int e0 = lane; e0 < 16 * COLS; e0 += 64 * BATCH) {
+            for (int k0 = 0; k0 < 16; k0 += BATCH) {
+                int i0[BATCH / R], j0[BATCH / R], at0[BATCH / R];
                 uv_pair uv[BATCH];
 #pragma unroll
+                for (int q = 0; q < BATCH / R; ++q) {
+                    place(k0 / R + q, i0[q], j0[q], at0[q]);
+                    i0[q] += row0 + first;
+                }
+#pragma unroll
                 for (int b = 0; b < BATCH; ++b) {
-                    const int e = e0 + 64 * b, i = w + x * 32 + h * 16 + e / COLS, j = col + e % COLS;
+                    const int i = i0[b / R] + b % R, j = j0[b / R] + lane;
                     uv[b] = 0.0f;
                     if (i < N && j <= i) uv[b] = *reinterpret_cast<const uv_pair*>(g.uv + 2 * tri_index(i, j));
                 }
 #pragma unroll
                 for (int b = 0; b < BATCH; ++b) {
-                    const int e = e0 + 64 * b, i = w + x * 32 + h * 16 + e / COLS, j = col + e % COLS;
-                    const float2 v = *reinterpret_cast<const float2*>(lds + (e / COLS) * PITCH + (e % COLS) * 8);
+                    const int i = i0[b / R] + b % R, j = j0[b / R] + lane;
+                    if (i >= N || j0[b / R] > i) continue;  // no element in this row
+                    const float2 v = *reinterpret_cast<const float2*>(lds + at0[b / R] + b % R * PITCH + lane * 8);
                     float vim = i == j ? 0.0f : v.y;
                     float *p = nullptr, *c = nullptr;
-                    if (i < N && j <= i) {
+                    if (j <= i) {
                         const float u = over_lambda(uv[b][0], g.lambda, y, plain) / g.cell;
                         const float t = over_lambda(uv[b][1], g.lambda, y, plain) / g.cell;
                         const int64_t at = grid_cell(g.Ng, half_ng + u, half_ng + t);
@@ -125,18 +159,40 @@ __device__ __forceinline__ void grid_block(const GridJob& g, int N, int w, int c
                     if (__ballot(c != nullptr)) grid_add(c, v.x, -vim);
                 }
             }
-            __builtin_amdgcn_wave_barrier();
+            wait();
         }
+    if (!shared) return;  // no diagonal in it
     // Autocorrelations mostly share the centre cell, one address for all their atomics and a
-    // long sum: those of a wave are summed first where they do.
+    // long sum: those of the tile are summed first where they do.
     const uint64_t autos = __ballot(auto_at != nullptr);
-    if (autos == 0) return;
-    const int src = __builtin_ctzll(autos);
-    float* first = reinterpret_cast<float*>(__shfl(reinterpret_cast<uint64_t>(auto_at), src));
-    if (__ballot(auto_at != nullptr && auto_at != first) == 0) {
+    const int src = autos ? __builtin_ctzll(autos) : 0;
+    float* at = reinterpret_cast<float*>(__shfl(reinterpret_cast<uint64_t>(auto_at), src));  // nullptr: none
+    const bool one = __ballot(auto_at != nullptr && auto_at != at) == 0;
+    if (one) {
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) auto_re += __shfl_xor(auto_re, d);
         if (lane != src) auto_at = nullptr;
+    }
+    struct Sum {
+        float* at;
+        float re;
+        int one;
+    }* sums = reinterpret_cast<Sum*>(lds);
+    if (lane == 0) sums[wave] = {at, auto_re, one};
+    __syncthreads();
+    bool same = true;
+    at = nullptr;
+    float total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        const Sum t = sums[w];
+        if (!at) at = t.at;
+        same = same && t.one && (!t.at || t.at == at);
+        total += t.re;
+    }
+    if (same) {
+        auto_at = wave == 0 && lane == 0 ? at : nullptr;
+        auto_re = total;
     }
     grid_add(auto_at, auto_re, 0.0f);
 }

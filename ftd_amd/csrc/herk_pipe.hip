@@ -260,15 +260,15 @@ __device__ __forceinline__ void pipe_tile(uint8_t* lds, const uint8_t* base, int
     const int a = wm * 2 * P_GSTRIDE, bo = (P_GROUPS / 2 + wn * 2) * P_GSTRIDE;
     if (!active) {
         tile_loop<false, false>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
-        if constexpr (FMT == OUT_GRID) __syncthreads();
-        return;
+        if constexpr (FMT != OUT_GRID) return;
+    } else {
+        tile_loop<true, FMT == OUT_UPPER_PACKED || FMT == OUT_HERM_FULL>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
     }
-    tile_loop<true, FMT == OUT_UPPER_PACKED || FMT == OUT_HERM_FULL>(rows, lds, steps / 2, off, lane, wave, a, bo, re, im);
     const bool inside = wcol + 63 < wrow && wrow + 64 <= N;
     if constexpr (FMT == OUT_GRID) {
-        static_assert(4 * grid_lds_bytes<2>() <= P_BUFS * P_STAGE, "gridding regions");
+        static_assert(4 * kGridRegion <= P_BUFS * P_STAGE, "gridding regions");
         __syncthreads();  // the last stage is read
-        grid_block(*grid, N, wrow, wcol, alpha, re, im, lds + wave * grid_lds_bytes<2>(), lane);
+        grid_tile<4, 2>(*grid, N, I * PT, J * PT, active, alpha, re, im, lds, wave, lane);
     } else if constexpr (FMT != OUT_LOWER_PACKED) {
         if (inside) store_ggp_inside<OutT, FMT>(C, N, wrow, wcol, re, im, lane);
         else store_ggp_any<OutT, FMT>(C, N, wrow, wcol, re, im, lane);

@@ -1294,9 +1294,9 @@ struct TileRunner {
             epilogue_beam<OutT>(j, lds, acc_re, acc_im, active, wrow0, wcol0, lane, tid);
             return;
         } else if constexpr (FMT == OUT_GRID) {
-            static_assert(grid_lds_bytes<Cfg::FN>() * Cfg::WAVES_M * Cfg::WAVES_N <= Cfg::LDS_BYTES, "gridding regions");
-            if (active)
-                grid_block(j.grid, j.N, wrow0, wcol0, j.alpha, acc_re, acc_im, lds + wave * grid_lds_bytes<Cfg::FN>(), lane);
+            constexpr int NW = Cfg::WAVES_M * Cfg::WAVES_N;
+            static_assert(kGridRegion * NW <= Cfg::LDS_BYTES, "gridding regions");
+            grid_tile<NW, Cfg::WAVES_N>(j.grid, j.N, j.row0, j.col0, active, j.alpha, acc_re, acc_im, lds, wave, lane);
             return;
         } else if constexpr (GEMM) {
             // B rows hold conj(B), so the HERK product A conj(B)^H = A B^T; lane =

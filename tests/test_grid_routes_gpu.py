@@ -39,3 +39,32 @@ def test_more_segments_than_a_grid_dimension(oracle, dev):
     ref = _reference(oracle, qc.reshape(-1), N, K, 1, len(full), uv, freqs, Ng, cell)
     assert np.abs(ref).sum() > 0
     assert np.array_equal(grid.cpu().numpy(), ref)
+
+
+# a tile's waves share its rows at the diagonal and at the edge: one wave's block and parts of 16 rows
+# (1, 16, 17, 63 .. 65), blocks without rows (100, 130, 193), whole tiles beside them (256, 300)
+@pytest.mark.parametrize("cfg", [-1, 0, 2, 3])
+@pytest.mark.parametrize("N", [1, 16, 17, 63, 64, 65, 100, 128, 130, 193, 256, 300])
+def test_rows_shared_by_a_tile(oracle, dev, cfg, N):
+    """Autocorrelations in one cell (summed over the tile) and in cells of their own, with and without
+    a half plane (one baseline per five cells on), on a grid that is not zero."""
+    import torch
+    from ftd_amd import ftdx
+    K, chan, pols = 80, 2, 2
+    qc = oracle.gen_qc_uniform(N, N * K * chan * pols)
+    ctx = ftdx.CutlassComplexGemm()
+    ctx.set_launch_config(cfg, -1)
+    A = torch.from_numpy(qc).to(dev)
+    for Ng in (33, 700):
+        uv, freqs, cell = _scene(N, Ng, N + 1, chan=chan)
+        f_d = torch.from_numpy(freqs).to(dev)
+        for apart in (False, True):
+            if apart:
+                d = np.arange(N)
+                uv[d * (d + 3) // 2, 0] = (d % 7 - 3) * cell * 0.2
+            ref = _reference(oracle, qc, N, K, chan, pols, uv, freqs, Ng, cell)
+            grid = torch.full((chan, Ng, Ng, 2), 2.0, device=dev)
+            ftdx.herk_pol_grid(ctx, A, N, K, chan, pols, torch.from_numpy(uv).to(dev), f_d, grid, Ng, cell)
+            torch.cuda.synchronize()
+            assert np.abs(ref).max() < 2 ** 24 - 2
+            assert np.array_equal(grid.cpu().numpy(), ref + 2.0), (Ng, apart)
