@@ -86,6 +86,7 @@ struct HerkPlainArgs {
     // n_time_inner).  Defaults: one input batch per output batch.
     int nseg = 1;
     int seg_group = 1;
+    bool plain_stores = false, direct_stores = false;  // set by the launch (the rules below)
     // OUT_GRID (launch_herk_grid): C is the grid [batch][Ng][Ng][2] (c_bstride = 2 Ng^2
     // floats); baseline UV in metres [N(N+1)/2][2] by packed lower index; output batch b
     // uses frequency freq_hz[freq_offset + b] (Hz) and cell size `cell` (radians).
@@ -97,6 +98,27 @@ struct HerkPlainArgs {
     // scratch planes of half_grid_cells(Ng) cells per batch (herk_grid.h), zeroed; nullptr: none
     float* half = nullptr;
 };
+
+// Whether a launch has so few samples for its output that interior tiles store straight from their
+// accumulators, by plain stores: up to 320 of them.  With K segments also where one segment is no more than
+// that and the loop is the bounds-checked one (K % 64 != 0), which leaves the stores more time, or the
+// output stays well inside the memory-side cache.  FP32 us, staged / plain: 1024 x 64, 2 x 320 (269 MB)
+// 122 / 140; 1024 x 64, 2 x 256 105 / 113; 1664 x 16, 2 x 320 (177 MB) 82 / 89; 512 x 64, 2 x 256 (67 MB)
+// 41.6 / 35.5; 1024 x 64, 2 x 200 120 / 113; FP16, non-temporal / plain: 1664 x 16, 2 x 256 (89 MB) 60 / 63;
+// 1024 x 32, 2 x 256 (67 MB) 50.3 / 49.2.
+inline bool plain_stores_pay(const HerkPlainArgs& a, bool out_fp16) {
+    if ((int64_t)a.K * a.nseg <= 320) return true;
+    return a.nseg > 1 && a.K <= 320 && (a.K % 64 != 0 || a.c_bstride * a.batch * (out_fp16 ? 2 : 4) <= 80000000);
+}
+
+// Whether interior tiles may store straight from their accumulators at all: not in up to two rounds of
+// tiles of up to three row blocks, where few are inside and each is waited for.  us, staged / direct:
+// 256 x 64, K = 256, FP32 12.1 / 13.2; 384 x 128, K = 512, FP16 33.0 / 37.9; 256 x 256, K = 640, FP16
+// 36.9 / 41.4; but 512 x 64, K = 256 29.8 / 24.7, 256 x 512, 2 x 200 90 / 85, and E3M2 rows, whose
+// conversion ran before (256 x 256, K = 640, FP16 61 / 59).
+inline bool direct_stores_pay(const HerkPlainArgs& a, int tile_cols, int64_t tiles) {
+    return a.N > 3 * tile_cols || tiles > 1024 || a.precast == 2;
+}
 
 // Lower-triangle tiles per problem for a configuration.
 int herk_tiles(int cfg, int N);

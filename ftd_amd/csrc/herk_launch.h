@@ -56,6 +56,8 @@ herk_int4_fp8_plain_kernel(HerkPlainArgs p, int tiles, int xcd_remap) {
     j.alpha = p.alpha;
     j.beta = p.beta;
     j.lda = p.lda;
+    j.plain_stores = p.plain_stores;
+    j.direct_stores = p.direct_stores;
     if constexpr (MODE == LOAD_MX4D) {
         j.S = p.S + (int64_t)b * p.s_bstride;
         j.s_stage = p.s_stage;
@@ -92,6 +94,8 @@ herk_int4_fp8_grouped_kernel(const GroupProblemDev* __restrict__ probs,
         j.beta = pr.beta;
         j.lda = pr.K;
         j.nseg = 1;
+        j.plain_stores = pr.K <= 320;
+        j.direct_stores = true;
         if constexpr (VEC_ONLY)
             TileRunner<Cfg>::template run<OutT, LOAD_VEC16, OUT_LOWER_PACKED, false>(j, lds);
         else if (pr.vec)
@@ -102,11 +106,13 @@ herk_int4_fp8_grouped_kernel(const GroupProblemDev* __restrict__ probs,
 }
 
 template <class Cfg>
-hipError_t launch_plain_cfg(const HerkPlainArgs& a, bool out_fp16, int xcd_remap,
-                            hipStream_t stream) {
+hipError_t launch_plain_cfg(const HerkPlainArgs& args, bool out_fp16, int xcd_remap, hipStream_t stream) {
+    HerkPlainArgs a = args;
     const int tiles = tri_tiles(a.N, Cfg::TM, Cfg::TN);
     const int64_t blocks = (int64_t)tiles * a.batch;
     if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
+    a.plain_stores = plain_stores_pay(a, out_fp16);
+    a.direct_stores = direct_stores_pay(a, Cfg::TN, blocks);
     const bool vec = (a.K % 16 == 0) && ((reinterpret_cast<uintptr_t>(a.A) & 15u) == 0);
     dim3 grid((unsigned)blocks), block(Cfg::THREADS);
     if (a.precast == 5) {

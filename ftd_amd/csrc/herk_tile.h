@@ -106,6 +106,7 @@ struct TileJob {
     // LOAD_MX4D: this problem's scales (row 0 of stage 0) and the bytes between stages
     const uint8_t* S;
     int64_t s_stage;
+    bool plain_stores, direct_stores;  // plain_stores_pay, direct_stores_pay
     GridJob grid;  // OUT_GRID
 };
 
@@ -1324,14 +1325,14 @@ struct TileRunner {
         }
         if constexpr (FMT == OUT_LOWER_PACKED) {
             // A tile inside the matrix and below the diagonal stores straight from its accumulators
-            // where the output is narrow or the samples few; on more samples FP32 rows leave faster
-            // as the staged epilogue's longer runs.  Plain stores, which the L2 joins to whole
-            // lines, up to 320 samples.  us of staged / direct, buffers in turn, 128 x 128 tiles:
+            // where the output is narrow or the samples few (plain_stores); on more samples FP32 rows leave
+            // faster as the staged epilogue's longer runs.  Plain stores, which the L2 joins to whole
+            // lines, with few samples.  us of staged / direct, buffers in turn, 128 x 128 tiles:
             // FP32 1152 x 66, K = 128 104 / 98; 512 x 100, K = 1024 62 / 66; 1500 x 40, K = 800 168 /
-            // 182; FP16 1664 x 128, K = 128 242 / 200; 1664 x 64, K = 512 209 / 188.  64 x 64 tiles
-            // (not staged, shorter runs) gain at any size: 2048 x 16, K = 512, FP32 172 to 140.
+            // 182; FP16 1664 x 128, K = 128 242 / 200; 1664 x 64, K = 512 209 / 188; 64 x 64 tiles
+            // 1024 x 32, K = 512, FP16 97 / 82.  Launches without room for it stay staged (direct_stores_pay).
             const bool direct = j.beta == 0.0f && j.row0 + Cfg::TM <= j.N && j.col0 + Cfg::TN <= j.row0 &&
-                                (!Cfg::EPI_STAGED || sizeof(OutT) == 2 || j.K <= 320);
+                                (!Cfg::EPI_STAGED || (j.direct_stores && (sizeof(OutT) == 2 || j.plain_stores)));
             if constexpr (Cfg::EPI_STAGED) {
                 if (!direct) {
                     epilogue_staged<OutT>(j, lds, acc_re, acc_im, active, wrow0, wcol0, lane, wave);
@@ -1340,7 +1341,7 @@ struct TileRunner {
             }
             if (direct) {
                 OutT* C = static_cast<OutT*>(j.C);
-                if (Cfg::TM < 128 || j.K > 320) store_inside<OutT, true, true>(C, wrow0, wcol0, j.alpha, acc_re, acc_im, lane);
+                if (Cfg::TM < 128 || !j.plain_stores) store_inside<OutT, true, true>(C, wrow0, wcol0, j.alpha, acc_re, acc_im, lane);
                 else store_inside<OutT, true, false>(C, wrow0, wcol0, j.alpha, acc_re, acc_im, lane);
                 return;
             }
