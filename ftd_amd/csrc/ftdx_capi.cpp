@@ -621,6 +621,12 @@ int grow_precast(ftdx_context* ctx, size_t need, const char* what) {
     return rc;
 }
 
+// The padded rows of a call that the pipelined kernel runs without them: the same call under capture
+// takes the fused tile and can allocate nothing.  Without memory for them it does without.
+void reserve_padded(ftdx_context* ctx, size_t need) {
+    if (grow_precast(ctx, need, "padded rows") != FTDX_OK) (void)hipGetLastError();
+}
+
 // A operand formats of the complex GEMM
 enum GemmInput { GEMM_A_FP16_PLANAR, GEMM_A_INT4, GEMM_A_FP8_INTERLEAVED };
 
@@ -1218,6 +1224,8 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
     if (padded && ((cfg != ftdx::TILE_PIPE && cfg != ftdx::TILE_DIRECT) || tune_now)) {
         int rc = ftdx::grow_precast(ctx, pad_need, "ftdx_herk: scratch");
         if (rc != FTDX_OK) return rc;
+    } else if (padded && cfg == ftdx::TILE_PIPE) {
+        ftdx::reserve_padded(ctx, pad_need);
     }
     if (tune_now) {
         ftdx::TuneEntry best;
@@ -1530,6 +1538,7 @@ int ftdx_herk_pol_grid(ftdx_context* ctx, const void* A, int N, int K, int n_cha
             return hip_fail(e, "ftdx_herk_pol_grid: half grid");
     }
     if (scr && may_pipe) {
+        if (ftdx::pol_rows_padded(A, K, n_pol, cfg)) ftdx::reserve_padded(ctx, ftdx::padded_scratch_bytes(a));
         e = ftdx::run_pipe(scr + half_bytes, a, false, s, true);
     } else if (ftdx::pol_rows_padded(A, K, n_pol, cfg)) {
         // rows padded per chunk of channels, as ftdx_herk does

@@ -1,0 +1,73 @@
+"""Calls that a program captures into a HIP graph after one eager call of the same shape."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+PIPE = 64
+
+
+def _replay(torch, graph, outs, refs, ctx):
+    for _ in range(3):
+        for o in outs:
+            o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for o, r in zip(outs, refs):
+            assert torch.equal(o, r)
+
+
+# rows that 16-byte loads cannot take, by their length and by their address
+@pytest.mark.parametrize("K,shift", [(1000, 0), (1024, 1)])
+@pytest.mark.parametrize("cached", [False, True])
+def test_ragged_rows_after_an_eager_call(oracle, dev, tmp_path, K, shift, cached):
+    """The eager call runs the pipelined kernel, which needs no padded rows; the captured one runs the
+    fused tile on padded rows, in scratch that it cannot allocate."""
+    import torch
+    from ftd_amd import ftdx
+    N, B = 1000, 12
+    ctx = ftdx.CutlassComplexGemm()
+    if cached:
+        path = tmp_path / "tune.txt"
+        ctx.tune_save(str(path))
+        with open(path, "a") as f:
+            f.write(f"herk\t{N}\t{K}\t{B}\t0\t4\t{PIPE}\t1\t1.0\n")
+        assert ctx.tune_load(str(path)) == (1, 0)
+    qc = oracle.gen_qc_uniform(K, N * K * B)
+    buf = torch.zeros(qc.size + shift, dtype=torch.uint8, device=dev)
+    A = buf[shift:]
+    A.copy_(torch.from_numpy(qc))
+    C = torch.zeros((B, N * (N + 1) // 2, 2), device=dev)
+
+    def call():
+        assert ctx.herk(A, C, N, K, B, input=ftdx.InputPrecision.INT4, output=ftdx.OutputPrecision.FP32, tune=False) == 0
+
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        call()
+        torch.cuda.synchronize()
+        ref = C.clone()
+        assert np.array_equal(ref[:1].cpu().numpy(), oracle.herk_f32(qc[:N * K], N, K, 1))
+        with torch.cuda.graph(graph, stream=side):
+            call()
+        _replay(torch, graph, [C], [ref], ctx)
+
+
+def test_ragged_gridding_after_an_eager_call(dev):
+    import torch
+    from ftd_amd import ftdx
+    N, K, chan, pol, Ng, cell = 300, 1000, 3, 2, 512, 2e-3
+    ctx = ftdx.CutlassComplexGemm()
+    A = torch.randint(0, 256, (chan * pol * N * K,), dtype=torch.uint8, device=dev)
+    uv = ((torch.rand((N * (N + 1) // 2, 2), device=dev) - 0.5) * Ng * cell * 0.2).contiguous()
+    freq = torch.linspace(0.8e9, 1.3e9, chan, device=dev, dtype=torch.float64)
+    grid = torch.zeros((chan, Ng, Ng, 2), device=dev)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        ftdx.herk_pol_grid(ctx, A, N, K, chan, pol, uv, freq, grid, Ng, cell)
+        torch.cuda.synchronize()
+        ref = grid.clone()
+        assert float(ref.abs().max()) < 2 ** 24  # integer sums: any order of the atomics
+        with torch.cuda.graph(graph, stream=side):
+            ftdx.herk_pol_grid(ctx, A, N, K, chan, pol, uv, freq, grid, Ng, cell)
+        _replay(torch, graph, [grid], [ref], ctx)
