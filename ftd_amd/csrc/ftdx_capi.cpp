@@ -25,6 +25,7 @@
 #include "herk_grid.h"
 #include "herk_mxpipe.h"
 #include "herk_pipe.h"
+#include "stream_slots.h"
 #include "calib.h"
 #include "stages.h"
 #include "imaging.h"
@@ -56,16 +57,9 @@ struct ftdx_context {
     // pre-cast FP8 operand rows for the unfused / FP16-input paths
     uint8_t* precast = nullptr;
     size_t precast_cap = 0;
-    // fragment rows of the pipelined HERK, one buffer per stream that called it (calls on
-    // different streams may overlap, as the fused tile needs no scratch); a fifth stream
-    // takes the fused tile
-    struct FragScratch {
-        bool used = false;
-        void* stream = nullptr;
-        uint8_t* rows = nullptr;
-        size_t cap = 0;
-    };
-    FragScratch frag[4];
+    // fragment rows of the pipelined HERK and half planes of the gridding, one buffer per stream; a
+    // call without one takes the fused tile, which needs none
+    ftdx::StreamSlots frag;
     // plain-path graph replay (set_direct_herk_graph): small LRU of captured calls
     struct GraphEntry {
         bool used = false;
@@ -314,25 +308,23 @@ size_t frag_scratch_bytes(const HerkPlainArgs& a) {
 
 // Fragment-row scratch of this stream, or NULL where the call has to do without: under
 // capture (a captured call must not depend on a buffer that a later call may replace), with
-// four other streams holding theirs, or when memory is short.
+// four other streams holding theirs, on another device, or when memory is short.
 uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
         return nullptr;
     }
-    ftdx_context::FragScratch* slot = nullptr;
-    for (auto& f : ctx->frag)
-        if (f.used && f.stream == s) slot = &f;
-    for (auto& f : ctx->frag)
-        if (!slot && !f.used) slot = &f;
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) dev = -1;
+    StreamSlot* slot = ctx->frag.pick(ctx->device, dev, s);
     if (!slot) return nullptr;
     if (slot->cap < need) {
         if (slot->rows) {
             if (hipDeviceSynchronize() != hipSuccess) return nullptr;
             (void)hipFree(slot->rows);
         }
-        *slot = ftdx_context::FragScratch();
+        *slot = StreamSlot();
         if (hipMalloc(&slot->rows, need) != hipSuccess) {
             (void)hipGetLastError();
             slot->rows = nullptr;
@@ -905,14 +897,13 @@ int ftdx_end_herk(ftdx_context* ctx) {
     bool any_graph = false;
     for (auto& gph : ctx->graphs) any_graph = any_graph || gph.used;
     bool any_frag = false;
-    for (auto& f : ctx->frag) any_frag = any_frag || f.rows;
+    for (auto& f : ctx->frag.slots) any_frag = any_frag || f.rows;
     if (ctx->mx_codes || ctx->cal_part || ctx->cal_herm || ctx->precast || any_frag ||
         any_graph) {
         (void)hipDeviceSynchronize();
-        for (auto& f : ctx->frag) {
+        for (auto& f : ctx->frag.slots)
             if (f.rows) (void)hipFree(f.rows);
-            f = ftdx_context::FragScratch();
-        }
+        ctx->frag = ftdx::StreamSlots();
         if (ctx->mx_codes) (void)hipFree(ctx->mx_codes);
         if (ctx->cal_part) (void)hipFree(ctx->cal_part);
         if (ctx->cal_herm) (void)hipFree(ctx->cal_herm);

@@ -1,8 +1,9 @@
 // Host-side launch planning of libftdx.so (built with g++ under ASan + UBSan, no GPU): the batches
-// per chunk of the pipelined HERK.  Prints "ALL PASSED" on success.
+// per chunk of the pipelined HERK, and its per-stream scratch slots.  Prints "ALL PASSED" on success.
 #include <cstdio>
 
 #include "herk_chunks.h"
+#include "stream_slots.h"
 
 static int g_fail = 0;
 #define CHECK(c)                                                              \
@@ -29,8 +30,27 @@ static void test_chunks() {
         }
 }
 
+static void* stream(int i) { return reinterpret_cast<void*>((uintptr_t)i); }
+
+// A slot is one stream's of one device: streams of two devices may have the same handle, the null
+// stream always does.
+static void test_slots_of_two_devices() {
+    ftdx::StreamSlots p;
+    ftdx::StreamSlot* s = p.pick(0, 0, stream(0));
+    CHECK(s);
+    s->used = true;
+    s->stream = stream(0);
+    CHECK(p.pick(0, 0, stream(0)) == s);
+    CHECK(p.pick(0, 1, stream(0)) == nullptr);
+    CHECK(p.pick(0, 1, stream(8)) == nullptr);
+    CHECK(p.pick(0, -1, stream(0)) == nullptr);
+    CHECK(p.pick(-1, -1, stream(0)) == nullptr);
+    CHECK(p.pick(0, 0, stream(8)) != s);
+}
+
 int main() {
     test_chunks();
+    test_slots_of_two_devices();
     if (g_fail == 0) std::printf("ALL PASSED\n");
     return g_fail != 0;
 }
