@@ -308,7 +308,7 @@ size_t frag_scratch_bytes(const HerkPlainArgs& a) {
 
 // Fragment-row scratch of this stream, or NULL where the call has to do without: under
 // capture (a captured call must not depend on a buffer that a later call may replace), with
-// four other streams holding theirs, on another device, or when memory is short.
+// four other streams calling, on another device, or when memory is short.
 uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
@@ -319,7 +319,7 @@ uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
     if (hipGetDevice(&dev) != hipSuccess) dev = -1;
     StreamSlot* slot = ctx->frag.pick(ctx->device, dev, s);
     if (!slot) return nullptr;
-    if (slot->cap < need) {
+    if (slot->cap < need || slot->stream != s) {
         if (slot->rows) {
             if (hipDeviceSynchronize() != hipSuccess) return nullptr;
             (void)hipFree(slot->rows);
@@ -332,8 +332,7 @@ uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
         }
         slot->cap = need;
     }
-    slot->used = true;
-    slot->stream = s;
+    ctx->frag.use(slot, s);
     return slot->rows;
 }
 

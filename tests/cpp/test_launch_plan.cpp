@@ -38,8 +38,7 @@ static void test_slots_of_two_devices() {
     ftdx::StreamSlots p;
     ftdx::StreamSlot* s = p.pick(0, 0, stream(0));
     CHECK(s);
-    s->used = true;
-    s->stream = stream(0);
+    p.use(s, stream(0));
     CHECK(p.pick(0, 0, stream(0)) == s);
     CHECK(p.pick(0, 1, stream(0)) == nullptr);
     CHECK(p.pick(0, 1, stream(8)) == nullptr);
@@ -48,9 +47,33 @@ static void test_slots_of_two_devices() {
     CHECK(p.pick(0, 0, stream(8)) != s);
 }
 
+// A program that makes a stream for every few calls keeps getting slots; five streams that take turns do
+// not take them from each other.
+static void test_slots_come_back() {
+    ftdx::StreamSlots p;
+    int served = 0, calls = 0;
+    for (int st = 1; st <= 40; ++st)
+        for (int c = 0; c < 20; ++c, ++calls)
+            if (ftdx::StreamSlot* s = p.pick(0, 0, stream(st))) {
+                p.use(s, stream(st));
+                ++served;
+            }
+    CHECK(served > calls / 4);  // 4 slots of 64 idle calls for streams of 20 calls each
+    ftdx::StreamSlots q;
+    for (int turn = 0; turn < 200; ++turn)
+        for (int st = 1; st <= 5; ++st) {
+            ftdx::StreamSlot* s = q.pick(0, 0, stream(st));
+            CHECK((s != nullptr) == (st <= 4));
+            if (!s) continue;
+            CHECK(!s->used || s->stream == stream(st));
+            q.use(s, stream(st));
+        }
+}
+
 int main() {
     test_chunks();
     test_slots_of_two_devices();
+    test_slots_come_back();
     if (g_fail == 0) std::printf("ALL PASSED\n");
     return g_fail != 0;
 }

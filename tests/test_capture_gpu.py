@@ -71,3 +71,29 @@ def test_ragged_gridding_after_an_eager_call(dev):
         with torch.cuda.graph(graph, stream=side):
             ftdx.herk_pol_grid(ctx, A, N, K, chan, pol, uv, freq, grid, Ng, cell)
         _replay(torch, graph, [grid], [ref], ctx)
+
+
+def test_streams_that_come_and_go(oracle, dev):
+    """A context called from ever new streams: after the first four are idle their memory serves the
+    next ones, and no more than four streams' rows are held."""
+    import torch
+    from ftd_amd import ftdx
+    N, K, B = 1000, 1024, 12  # 18.9 MB of rows a stream
+    qc = oracle.gen_qc_uniform(4, N * K * B)
+    A = torch.from_numpy(qc).to(dev)
+    C = torch.zeros((B, N * (N + 1) // 2, 2), device=dev)
+    ref = oracle.herk_f32(qc[:N * K], N, K, 1)
+    ctx = ftdx.CutlassComplexGemm()
+    streams = [torch.cuda.Stream() for _ in range(9)]
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    for s in streams:
+        for _ in range(30):
+            assert ctx.herk(A, C, N, K, B, input=ftdx.InputPrecision.INT4, output=ftdx.OutputPrecision.FP32, stream=s,
+                            tune=False) == 0
+        torch.cuda.synchronize()
+        assert np.array_equal(C[:1].cpu().numpy(), ref)
+        C.zero_()
+        torch.cuda.synchronize()
+    held = free0 - torch.cuda.mem_get_info()[0]
+    assert held < 4 * 19e6 + 32e6, held
