@@ -320,6 +320,7 @@ uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
     StreamSlot* slot = ctx->frag.pick(ctx->device, dev, s);
     if (!slot) return nullptr;
     if (slot->cap < need || slot->stream != s) {
+        if (ctx->frag.refused(need)) return nullptr;
         if (slot->rows) {
             if (hipDeviceSynchronize() != hipSuccess) return nullptr;
             (void)hipFree(slot->rows);
@@ -328,6 +329,7 @@ uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
         if (hipMalloc(&slot->rows, need) != hipSuccess) {
             (void)hipGetLastError();
             slot->rows = nullptr;
+            ctx->frag.refuse(need);
             return nullptr;
         }
         slot->cap = need;

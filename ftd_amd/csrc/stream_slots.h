@@ -43,6 +43,14 @@ public:
         return pick;
     }
 
+    // After a failed allocation of `need` bytes: no other of that size or more for kIdleCalls calls (each
+    // would cost what the failed one did).
+    bool refused(size_t need) const { return refused_ && need >= refused_ && calls_ - refused_at_ <= kIdleCalls; }
+    void refuse(size_t need) {
+        refused_ = need;
+        refused_at_ = calls_;
+    }
+
     // The call of the last pick has its rows.
     void use(StreamSlot* slot, void* stream) {
         slot->used = true;
@@ -51,7 +59,8 @@ public:
     }
 
 private:
-    uint64_t calls_ = 0;
+    uint64_t calls_ = 0, refused_at_ = 0;
+    size_t refused_ = 0;
 };
 
 }  // namespace ftdx

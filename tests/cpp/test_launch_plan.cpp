@@ -70,8 +70,25 @@ static void test_slots_come_back() {
         }
 }
 
+// An allocation that failed is not tried again on every call.
+static void test_refused_allocations() {
+    ftdx::StreamSlots p;
+    int tries = 0;
+    for (int c = 0; c < 650; ++c) {
+        CHECK(p.pick(0, 0, stream(1)));
+        CHECK(!p.refused(99));
+        if (p.refused(100)) continue;
+        CHECK(c == 0 || !p.refused(200));
+        ++tries;
+        p.refuse(100);
+        CHECK(p.refused(100) && p.refused(200));
+    }
+    CHECK(tries == 10);
+}
+
 int main() {
     test_chunks();
+    test_refused_allocations();
     test_slots_of_two_devices();
     test_slots_come_back();
     if (g_fail == 0) std::printf("ALL PASSED\n");
