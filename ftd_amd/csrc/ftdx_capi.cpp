@@ -316,17 +316,20 @@ uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
         return nullptr;
     }
     int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess) dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) (void)hipGetLastError();
     StreamSlot* slot = ctx->frag.pick(ctx->device, dev, s);
     if (!slot) return nullptr;
     if (slot->cap < need || slot->stream != s) {
         if (ctx->frag.refused(need)) return nullptr;
-        if (slot->rows) {
-            if (hipDeviceSynchronize() != hipSuccess) return nullptr;
-            (void)hipFree(slot->rows);
-        }
+        // another stream or thread may be capturing: only in this mode does an allocation leave that
+        // capture alone, and hipDeviceSynchronize does in none (hipFree waits for the device by itself)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+        if (slot->rows) (void)hipFree(slot->rows);
         *slot = StreamSlot();
-        if (hipMalloc(&slot->rows, need) != hipSuccess) {
+        const hipError_t e = hipMalloc(&slot->rows, need);
+        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) {
             (void)hipGetLastError();
             slot->rows = nullptr;
             ctx->frag.refuse(need);
