@@ -7,6 +7,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <sys/syscall.h>
+#include <unistd.h>
+
 #include <algorithm>
 #include <atomic>
 #include <cstdio>
@@ -93,7 +96,15 @@ namespace ftdx {
 
 namespace {
 thread_local std::string g_last_error;
-thread_local ftdx_context* g_default_ctx = nullptr;
+
+// The context of a thread's stateless calls.  Its scratch goes back when the thread ends; the process's
+// own thread leaves that to the process, and a forked child has no part in its parent's.
+struct DefaultContext {
+    ftdx_context* ctx = nullptr;
+    pid_t pid = 0;
+    ~DefaultContext();
+};
+thread_local DefaultContext g_default;
 
 // Default launch configuration when nothing is tuned or set.
 constexpr int kDefaultCfg = TILE_128x128_K64;
@@ -617,6 +628,26 @@ int grow_precast(ftdx_context* ctx, size_t need, const char* what) {
     return rc;
 }
 
+void free_scratch(ftdx_context* ctx) {
+    for (auto& f : ctx->frag.slots)
+        if (f.rows) (void)hipFree(f.rows);
+    ctx->frag = StreamSlots();
+    for (uint8_t** p : {&ctx->mx_codes, &ctx->cal_part, &ctx->cal_herm, &ctx->precast}) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
+    ctx->mx_codes_cap = ctx->cal_part_cap = ctx->cal_herm_cap = ctx->precast_cap = 0;
+}
+
+// Other threads may be capturing: relaxed mode, and no wait but hipFree's own.
+DefaultContext::~DefaultContext() {
+    if (!ctx || pid != getpid() || syscall(SYS_gettid) == (long)pid) return;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    free_scratch(ctx);
+    delete ctx;
+}
+
 // The padded rows of a call that the pipelined kernel runs without them: the same call under capture
 // takes the fused tile and can allocate nothing.  Without memory for them it does without.
 void reserve_padded(ftdx_context* ctx, size_t need) {
@@ -896,6 +927,7 @@ int ftdx_init_herk(ftdx_context* ctx, int N, int K, int batch_count, void* strea
 }
 
 int ftdx_end_herk(ftdx_context* ctx) {
+    if (!ctx) ctx = ftdx::g_default.ctx;  // of the stateless calls
     if (!ctx) return FTDX_OK;
     ctx->init_N = ctx->init_K = ctx->init_batch = 0;
     bool any_graph = false;
@@ -905,13 +937,7 @@ int ftdx_end_herk(ftdx_context* ctx) {
     if (ctx->mx_codes || ctx->cal_part || ctx->cal_herm || ctx->precast || any_frag ||
         any_graph) {
         (void)hipDeviceSynchronize();
-        for (auto& f : ctx->frag.slots)
-            if (f.rows) (void)hipFree(f.rows);
-        ctx->frag = ftdx::StreamSlots();
-        if (ctx->mx_codes) (void)hipFree(ctx->mx_codes);
-        if (ctx->cal_part) (void)hipFree(ctx->cal_part);
-        if (ctx->cal_herm) (void)hipFree(ctx->cal_herm);
-        if (ctx->precast) (void)hipFree(ctx->precast);
+        ftdx::free_scratch(ctx);
         for (auto& gph : ctx->graphs) {
             if (gph.used && gph.exec) (void)hipGraphExecDestroy(gph.exec);
             gph = ftdx_context::GraphEntry();
@@ -921,12 +947,6 @@ int ftdx_end_herk(ftdx_context* ctx) {
         (void)hipStreamDestroy(ctx->cap_stream);
         ctx->cap_stream = nullptr;
     }
-    ctx->mx_codes = nullptr;
-    ctx->mx_codes_cap = 0;
-    ctx->cal_part = ctx->cal_herm = nullptr;
-    ctx->cal_part_cap = ctx->cal_herm_cap = 0;
-    ctx->precast = nullptr;
-    ctx->precast_cap = 0;
     return FTDX_OK;
 }
 
@@ -2014,7 +2034,7 @@ int ftdx_herk_int4(const void* A, void* C, int N, int K, int batch_count, int ou
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "ftdx_herk_int4: hipGetDevice");
-    ftdx_context*& d = ftdx::g_default_ctx;
+    ftdx_context*& d = ftdx::g_default.ctx;
     if (d && d->device != dev) {
         ftdx_destroy(d);
         d = nullptr;
@@ -2022,6 +2042,7 @@ int ftdx_herk_int4(const void* A, void* C, int N, int K, int batch_count, int ou
     if (!d) {
         int rc = ftdx_create(&d);
         if (rc != FTDX_OK) return rc;
+        ftdx::g_default.pid = getpid();
     }
     return ftdx_herk(d, A, C, N, K, batch_count, FTDX_INPUT_INT4, FTDX_COMPUTE_FP8, output,
                      FTDX_FORMAT_PACKED_TRIANGLE, alpha, beta, stream, 0);

@@ -141,7 +141,8 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
 /* Replaces CutlassComplexGemm::init_herk / end_herk (cutlass_gemm_api.h:601-617).
  * init_herk allocates the scratch that calls of this shape need (staged rows for the
  * pre-cast paths and graph mode, padded rows when K % 16 != 0, E3M2 rows for calls on
- * `stream`), so that they allocate nothing later; end_herk releases it. */
+ * `stream`), so that they allocate nothing later; end_herk releases it (NULL: the scratch of the
+ * calling thread's stateless ftdx_herk_int4 calls, which otherwise goes back when the thread ends). */
 int ftdx_init_herk(ftdx_context* ctx, int N, int K, int batch_count, void* stream);
 int ftdx_end_herk(ftdx_context* ctx);
 
