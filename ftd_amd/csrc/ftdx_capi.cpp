@@ -892,12 +892,12 @@ int ftdx_init_herk(ftdx_context* ctx, int N, int K, int batch_count, void* strea
     if (!ctx) return fail(FTDX_ERR_INVALID_ARG, "ftdx_init_herk: NULL context");
     if (N < 0 || K < 0 || batch_count < 0)
         return fail(FTDX_ERR_INVALID_ARG, "ftdx_init_herk: negative size");
-    // The fused path on 16-byte-aligned rows of K % 16 == 0 needs no scratch.  The
-    // unfused (ForceBaseline) and FP16-input paths stage pre-cast FP8 rows, and the fused
-    // path on rows of K % 16 != 0 zero-padded copies, one chunk of channels at a time:
-    // allocate that now so that later calls (and graph capture) allocate nothing
-    // (cutlass_gemm_api.h:601-617).  Rows at an address that is not 16-byte aligned are
-    // padded too; their scratch is allocated by the first such call unless graph mode
+    // The direct kernel, and the fused tile on 16-byte-aligned rows of K % 16 == 0, need no scratch.
+    // The unfused (ForceBaseline) and FP16-input paths stage pre-cast FP8 rows, the fused
+    // path on rows of K % 16 != 0 zero-padded copies, the pipelined kernel E3M2 fragment rows, one
+    // chunk of channels at a time: allocate that now so that later calls (and graph capture)
+    // allocate nothing (cutlass_gemm_api.h:601-617).  Rows at an address that is not 16-byte
+    // aligned are padded too; their scratch is allocated by the first such call unless graph mode
     // or ForceBaseline already sized it.
     ctx->init_N = N;
     ctx->init_K = K;
@@ -913,9 +913,17 @@ int ftdx_init_herk(ftdx_context* ctx, int N, int K, int batch_count, void* strea
         int rc = ftdx::grow_precast(ctx, need, "ftdx_init_herk: scratch");
         if (rc != FTDX_OK) return rc;
     }
-    // fragment rows of the pipelined path, for calls on this stream (which do without when
-    // there is no memory for them)
-    if (ctx->device >= 0 && ctx->herk_mode == FTDX_HERK_AUTO && ctx->forced_cfg < 0 &&
+    // fragment rows for calls on this stream (which do without when there is no memory for them), where
+    // INT4 calls of either output run the pipelined kernel, by the tuning cache or untuned
+    bool pipe = false;
+    for (int fp16 = 0; fp16 <= 1; ++fp16) {
+        ftdx::TuneEntry e;
+        if (ctx->tune.find({N, K, batch_count, fp16, K % 16 != 0 ? 4 : 1}, e))
+            pipe = pipe || e.cfg == ftdx::TILE_PIPE;
+        else
+            pipe = pipe || ftdx::choose_kernel(nullptr, N, K, batch_count, fp16 != 0) == ftdx::TILE_PIPE;
+    }
+    if (pipe && ctx->device >= 0 && ctx->herk_mode == FTDX_HERK_AUTO && ctx->forced_cfg < 0 &&
         ctx->direct_tile == FTDX_DIRECT_TILE_AUTO && batch_count > 0 && ftdx::pipe_supported(N, K)) {
         ftdx::HerkPlainArgs a{};
         a.N = N;
