@@ -578,12 +578,22 @@ int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStrea
                 const float ms = time_cand(cands[i].cfg, cands[i].remap, 3);
                 sum[i] += ms < 0.0f ? 1e30f : ms + later(cands[i].cfg);
             }
-        for (size_t i = 0; i < nf; ++i)
-            if (sum[i] / 2 < best.ms) {
-                best.ms = sum[i] / 2;
+        for (size_t i = 0; i < nf; ++i) {
+            cands[i].ms = sum[i] / 2;
+            if (cands[i].ms < best.ms) {
+                best.ms = cands[i].ms;
                 best.cfg = cands[i].cfg;
                 best.xcd_remap = cands[i].remap;
             }
+        }
+        float alt = 1e30f;
+        if (best.cfg == TILE_PIPE)
+            for (const Cand& c : cands)
+                if (c.cfg != TILE_PIPE && c.ms < alt) {
+                    alt = c.ms;
+                    best.alt_cfg = c.cfg;
+                    best.alt_remap = c.remap;
+                }
     }
     (void)hipEventDestroy(t0);
     (void)hipEventDestroy(t1);
@@ -1234,8 +1244,15 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
     uint8_t* frag = nullptr;
     if (may_pipe && (cfg == ftdx::TILE_PIPE || tune_now))
         frag = ftdx::frag_scratch(ctx, ftdx::frag_scratch_bytes(a), s);
-    if ((cfg == ftdx::TILE_PIPE && !frag) ||
-        (cfg == ftdx::TILE_DIRECT && !(may_route && ftdx::direct_supported(N, K, batch_count))))
+    if (cfg == ftdx::TILE_PIPE && !frag) {
+        ftdx::TuneEntry e;
+        cfg = ftdx::TILE_128x128_K64_P2;
+        if (cached && ctx->tune.find(key, e) && e.alt_cfg >= 0) {
+            cfg = e.alt_cfg;
+            if (ctx->forced_remap < 0) remap = e.alt_remap;
+        }
+    }
+    if (cfg == ftdx::TILE_DIRECT && !(may_route && ftdx::direct_supported(N, K, batch_count)))
         cfg = ftdx::TILE_128x128_K64_P2;
     const int Kp = ftdx::precast_row_samples(K);
     const size_t rows_need = (size_t)N * ftdx::precast_chunk_cap(N, K, batch_count) * 2 * Kp;

@@ -1,7 +1,7 @@
 // ftdx_tune.cpp -- tuning cache file I/O (format: see ftdx_tune.h).
 //
 //   # ftdx-tune <fingerprint>
-//   herk <N> <K> <batch> <out_fp16> <vec> <cfg> <xcd_remap> <ms>     (tab-separated)
+//   herk <N> <K> <batch> <out_fp16> <vec> <cfg> <xcd_remap> <ms> [<alt_cfg> <alt_remap>]   (tab-separated)
 #include "ftdx_tune.h"
 
 #include <unistd.h>
@@ -71,7 +71,9 @@ int TuneCache::load(const std::string& path, int* skipped) {
             continue;
         }
         std::string extra;
-        if (ss >> extra) {
+        if (!(ss >> std::ws).eof() &&
+            (e.cfg != TILE_PIPE || !(ss >> e.alt_cfg >> e.alt_remap) ||
+             !(valid_tile_config(e.alt_cfg) || e.alt_cfg == TILE_DIRECT) || (ss >> extra))) {
             ++bad;
             continue;
         }
@@ -99,7 +101,9 @@ bool TuneCache::save(const std::string& path) const {
             const TuneKey& k = kv.first;
             const TuneEntry& e = kv.second;
             out << "herk\t" << k.N << '\t' << k.K << '\t' << k.batch << '\t' << k.out_fp16 << '\t'
-                << k.vec << '\t' << e.cfg << '\t' << e.xcd_remap << '\t' << e.ms << "\n";
+                << k.vec << '\t' << e.cfg << '\t' << e.xcd_remap << '\t' << e.ms;
+            if (e.alt_cfg >= 0) out << '\t' << e.alt_cfg << '\t' << e.alt_remap;
+            out << "\n";
         }
         if (!out) {
             out.close();

@@ -20,6 +20,10 @@ struct TuneEntry {
     int cfg = 0;
     int xcd_remap = 1;
     float ms = 0.0f;
+    // where cfg needs scratch that a call may have to do without (the pipelined kernel): the fastest that
+    // needs none; -1: not timed
+    int alt_cfg = -1;
+    int alt_remap = 1;
 };
 
 class TuneCache {
