@@ -534,13 +534,10 @@ int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStrea
         (void)hipEventElapsedTime(&ms, t0, t1);
         return ms / reps;
     };
-    // Repeated on the same buffers, the pipelined kernel finds its rows in the memory-side cache;
-    // a program whose buffers change pays for them what 0.7 bytes per sample take at 5 TB/s
-    // (1024 x 64, K = 1024: 130 us repeated, 147 with three sets of buffers in turn).
     auto later = [&](int cfg) {
-        return cfg == TILE_PIPE ? (float)((double)qc_args->N * qc_args->K * qc_args->batch * 0.7 / 5e9) : 0.0f;
+        return cfg == TILE_PIPE ? (float)pipe_cold_ms((int64_t)qc_args->N * qc_args->K * qc_args->batch) : 0.0f;
     };
-    // first pass: every (configuration, workgroup order), one warm-up launch each
+    // first pass: every (configuration, workgroup order), one warm-up launch each; ms includes later(cfg)
     struct Cand {
         int cfg, remap;
         float ms;
@@ -595,6 +592,7 @@ int autotune(ftdx_context* ctx, const HerkPlainArgs& a0, bool out_fp16, hipStrea
                     best.alt_remap = c.remap;
                 }
     }
+    if (!cands.empty()) best.ms -= later(best.cfg);  // the entry's time is the measured one
     (void)hipEventDestroy(t0);
     (void)hipEventDestroy(t1);
     if (scratch) (void)hipFree(scratch);

@@ -61,4 +61,10 @@ inline int frag_chunk_cap(int N, int K, int nseg, int batch) {
     return std::min(chunk_cap_bytes(per, batch, limit), 65535 / std::max(nseg, 1));
 }
 
+// Repeated on the same buffers, as the autotuner runs it, the conversion finds inputs of up to 100 MB in
+// the memory-side cache; a program whose buffers change pays for them what 0.45 bytes per sample take at
+// 5 TB/s.  us more with three sets of buffers in turn: 512 x 100, K = 1024 (52 MB) 4.6, 1024 x 64, K = 1024
+// (67 MB) 5.9; 1024 x 64, K = 2048 (134 MB) -0.2, 1024 x 128 (268 MB) -2.4, 4096 x 96 (805 MB) -2.5.
+inline double pipe_cold_ms(int64_t samples) { return samples <= 100000000 ? (double)samples * 0.45 / 5e9 : 0.0; }
+
 }  // namespace ftdx

@@ -86,8 +86,18 @@ static void test_refused_allocations() {
     CHECK(tries == 10);
 }
 
+// Inputs that no cache holds cost the same on every pass.
+static void test_cold_inputs() {
+    CHECK(ftdx::pipe_cold_ms((int64_t)4096 * 2048 * 96) == 0.0);
+    CHECK(ftdx::pipe_cold_ms(268435456) == 0.0);
+    const double ms = ftdx::pipe_cold_ms(1024 * 1024 * 64);
+    CHECK(ms > 0.004 && ms < 0.008);
+    CHECK(ftdx::pipe_cold_ms(0) == 0.0);
+}
+
 int main() {
     test_chunks();
+    test_cold_inputs();
     test_refused_allocations();
     test_slots_of_two_devices();
     test_slots_come_back();
