@@ -467,14 +467,16 @@ bool grid_pipe_pays(const HerkPlainArgs& a) {
            pipe_us(st, t128, (double)a.N * a.K * a.nseg * a.batch, 2.5) < fused_us(st, t128);
 }
 
-// Whether a half plane (herk_grid.h) saves more scattered atomics than its own passes cost: from
-// one baseline per five cells on, and up to 256 MB of it.  us without / with, baselines per cell:
-// 1024 x 8 channels on 1024^2 (0.50) 498 / 353; 512 x 8 on 512^2 (0.50) 133 / 106; 1536 x 2 on
-// 2048^2 (0.28) 268 / 227; 700 x 1 on 1000^2 (0.25) 74 / 65; 512 x 8 on 1024^2 (0.13) 141 / 146
-// (with the slower first form of the closing pass).
+// Whether a half plane (herk_grid.h) saves more scattered atomics than zeroing it and its closing pass
+// cost: from one baseline per eight cells on, up to 256 MB of it, where the atomics bound the launch: not in
+// a few tiles of less than 256 inputs.  us without / with, baselines per cell: 1024 x 8 channels on 1024^2
+// (0.50) 453 / 293, on 2048^2 (0.125) 487 / 407, on 2896^2 (0.06) 569 / 538; 512 x 8 on 700^2 (0.27) 129 / 98,
+// on 1024^2 (0.125) 126 / 114, on 1448^2 (0.06) 138 / 147; 256 x 8 on 512^2 (0.125) 71 / 67, on 604^2 (0.09)
+// 72 / 75; 200 x 8 on 284^2 (0.25) 50 / 52; 64 x 16 on 100^2 (0.21) 26 / 30; 200 x 64 on 400^2 (0.126) 146 / 133.
 bool half_grid_pays(int N, int Ng, int n_chan) {
+    const int64_t baselines = (int64_t)N * (N + 1) / 2;
     const size_t plane = (size_t)half_grid_cells(Ng) * 8;
-    return 5 * ((int64_t)N * (N + 1) / 2) >= (int64_t)Ng * Ng && n_chan <= 65535 &&
+    return 8 * baselines >= (int64_t)Ng * Ng && (N >= 256 || baselines * n_chan >= 1000000) && n_chan <= 65535 &&
            plane <= (size_t(256) << 20) / n_chan;
 }
 

@@ -68,3 +68,55 @@ def test_rows_shared_by_a_tile(oracle, dev, cfg, N):
             torch.cuda.synchronize()
             assert np.abs(ref).max() < 2 ** 24 - 2
             assert np.array_equal(grid.cpu().numpy(), ref + 2.0), (Ng, apart)
+
+
+# even and odd grids on both sides of one baseline per eight cells; few inputs with enough channels and not
+@pytest.mark.parametrize("N,K,chan,Ng", [(256, 64, 3, 363), (256, 64, 3, 362), (300, 600, 2, 65), (300, 40, 2, 602),
+                                         (100, 16, 200, 40), (100, 16, 197, 40), (255, 64, 2, 64)])
+def test_half_planes_at_their_line(oracle, dev, N, K, chan, Ng):
+    """Baselines on the grid's edge (no mirror cell) and exactly between two cells (rounding away from
+    zero is not symmetric about the centre), wavelengths of 1 and 2 m and others."""
+    import torch
+    from ftd_amd import ftdx
+    pols, cell, light = 2, 2e-3, 299792458.0
+    qc = oracle.gen_qc_uniform(N + Ng, N * K * chan * pols)
+    rng = np.random.default_rng(Ng)
+    uv = (rng.integers(-2 * Ng, 2 * Ng + 1, (N * (N + 1) // 2, 2)) * (0.25 * cell)).astype(np.float32)
+    d = np.arange(N)
+    uv[d * (d + 3) // 2] = 0.0
+    freqs = np.resize([light, 0.5 * light, 1.3e9], chan)
+    ref = _reference(oracle, qc, N, K, chan, pols, uv, freqs, Ng, cell)
+    grid = torch.full((chan, Ng, Ng, 2), 3.0, device=dev)
+    ftdx.herk_pol_grid(ftdx.CutlassComplexGemm(), torch.from_numpy(qc).to(dev), N, K, chan, pols,
+                       torch.from_numpy(uv).to(dev), torch.from_numpy(freqs).to(dev), grid, Ng, cell)
+    torch.cuda.synchronize()
+    assert np.abs(ref).max() < 2 ** 24 - 3
+    assert np.array_equal(grid.cpu().numpy(), ref + 3.0)
+
+
+@pytest.mark.parametrize("Ng", [512, 1024])  # 168 MB of half planes; 671 MB, so none
+@pytest.mark.parametrize("K", [1008, 1000])
+def test_gridding_in_chunks(dev, Ng, K):
+    """More channels than one 160 MB chunk of fragment rows: each chunk grids its own channels, at their
+    frequencies, into their planes.  Equal to a forced tile's grid, whose sums are exact too (+-1 voltages)."""
+    import torch
+    from ftd_amd import ftdx
+    N, chan, pols = 1024, 120, 2  # 3.1 MB of rows per channel
+    gen = torch.Generator(device=dev).manual_seed(K)
+    A = torch.tensor([0x11, 0x19, 0x91, 0x99], dtype=torch.uint8, device=dev)[
+        torch.randint(0, 4, (chan * pols * N * K,), generator=gen, device=dev)]
+    uv, _, cell = _scene(N, Ng, 3)
+    uv_d = torch.from_numpy(uv).to(dev)
+    freqs = torch.linspace(0.7e9, 1.4e9, chan + 1, dtype=torch.float64, device=dev)
+    grids = []
+    for cfg in (-1, 0):
+        ctx = ftdx.CutlassComplexGemm()
+        ctx.set_launch_config(cfg, -1)
+        grids.append(torch.zeros((chan, Ng, Ng, 2), device=dev))
+        ftdx.herk_pol_grid(ctx, A, N, K, chan, pols, uv_d, freqs, grids[-1], Ng, cell, freq_offset=1)
+        torch.cuda.synchronize()
+        ctx.close()
+    assert float(grids[0].abs().max()) < 2 ** 24
+    for c in range(chan):
+        assert torch.equal(grids[0][c], grids[1][c]), c
+    assert not torch.equal(grids[0][0], grids[0][chan - 1])
