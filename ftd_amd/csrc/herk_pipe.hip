@@ -13,9 +13,10 @@
 //   * operands one 32-sample step ahead in a second register set, across the barrier too: a
 //     stage's first step is read during the previous stage, whose barrier already published
 //     it, so no MFMA waits for an LDS read that was not issued a step earlier.
-// Stores go to the packed rows straight from the accumulators: 32-lane runs, plain (not
-// non-temporal) so that the L2 joins the partial lines of neighbouring runs (1664 inputs x
-// 128, K = 128: 303 against 478 us; 64-byte write requests within 1% of the output bytes).
+// Stores go to the packed rows straight from the accumulators.  With few samples they are runs of 32
+// lanes, plain, so that the L2 joins the partial lines of neighbouring runs (1664 inputs x 128, K = 128,
+// FP32: 303 against 478 us non-temporal; written bytes within 2% of the output's); with more, runs of 64
+// elements from paired rows, non-temporal (pipe_nontemporal below has both sides).
 #include "herk_common.h"
 #include "herk_elem.h"
 #include "herk_grid.h"

@@ -127,12 +127,16 @@ int ftdx_destroy(ftdx_context* ctx);
  * over the waves of a workgroup, larger ones convert each chunk of channels to 6-bit E3M2 operand
  * rows (every QC value is exact in E3M2, results are those of the FP8 tile bit for bit) and run a
  * pipelined kernel over them, and the rest the fused FP8 tile.  The rows live in the context, at
- * most 160 MB (or one channel's) for each of up to four streams that called it; a call without them --
- * under stream capture, from a fifth stream, or when memory is short -- takes the fused tile.
+ * most 160 MB (or one channel's, up to 2 GiB) for each of up to four streams that call it, the
+ * largest any call of the stream needed (ftdx_herk_pol_grid's included); a stream that 64 calls of
+ * others went past loses them to the next.  A call without them -- under stream capture, from a
+ * fifth stream, on another device than the context's, or when memory is short -- takes the fused
+ * tile: the fastest kernel without scratch that tuning found for the shape, else 128 x 128.
  * The fused tile copies rows of K % 16 != 0, or at an address that is not 16-byte aligned,
  * zero-padded (K rounded up to 16, or to the tile's stage) into the context's scratch (at
- * most 320 MB per chunk of channels); the FP16-input, ForceBaseline and E3M2
- * paths stage converted rows there.  The scratch grows on first need unless
+ * most 320 MB per chunk of channels; the first eager call of such a shape sizes it also where it
+ * runs the pipelined kernel, so that the same call may be captured afterwards); the FP16-input,
+ * ForceBaseline and E3M2 paths stage converted rows there.  The scratch grows on first need unless
  * ftdx_init_herk sized it. */
 int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch_count,
               int input, int compute, int output, int format, float alpha, float beta,
@@ -141,7 +145,8 @@ int ftdx_herk(ftdx_context* ctx, const void* A, void* C, int N, int K, int batch
 /* Replaces CutlassComplexGemm::init_herk / end_herk (cutlass_gemm_api.h:601-617).
  * init_herk allocates the scratch that calls of this shape need (staged rows for the
  * pre-cast paths and graph mode, padded rows when K % 16 != 0, E3M2 rows for calls on
- * `stream`), so that they allocate nothing later; end_herk releases it (NULL: the scratch of the
+ * `stream` where INT4 calls of the shape run the pipelined kernel), so that they allocate nothing
+ * later, tuning apart; end_herk releases it (NULL: the scratch of the
  * calling thread's stateless ftdx_herk_int4 calls, which otherwise goes back when the thread ends). */
 int ftdx_init_herk(ftdx_context* ctx, int N, int K, int batch_count, void* stream);
 int ftdx_end_herk(ftdx_context* ctx);
@@ -177,11 +182,11 @@ int ftdx_set_launch_config(ftdx_context* ctx, int tile_config, int xcd_remap);
  * skipped.  `loaded` / `skipped` may be NULL. */
 int ftdx_tune_load(ftdx_context* ctx, const char* path, int* loaded, int* skipped);
 int ftdx_tune_save(ftdx_context* ctx, const char* path);
-/* Launch configuration ftdx_herk would use now for this shape without tuning
- * (explicit setting, else cache entry, else the default).  A cache entry may also hold 64 (the
- * pipelined kernel over E3M2 rows) or 65 (the K-splitting kernel for small problems), which
- * ftdx_set_launch_config does not take; without an entry or a setting INT4 calls choose between
- * them and the fused tile by size. */
+/* The setting for this shape: the explicit one, else the cache entry's, else the default tile.  It is
+ * what ftdx_herk runs, but for INT4 calls with neither, which choose between the pipelined kernel, the
+ * K-splitting kernel and the fused tile by size.  An entry may hold 64 (the pipelined kernel over E3M2
+ * rows) or 65 (the K-splitting kernel): those two are not tiles, and ftdx_set_launch_config refuses
+ * them; a context without a setting runs them from the same entry. */
 int ftdx_herk_query_config(ftdx_context* ctx, int N, int K, int batch_count, int output,
                            int* tile_config, int* xcd_remap);
 
@@ -434,8 +439,11 @@ int ftdx_pillbox_grid(const void* vis_tri, int vis_output, const float* baseline
  * zeroes the grid.  Equal to ftdx_herk_pol_reduce (n_time_inner = 1) followed by
  * ftdx_pillbox_grid (Nf = n_chan) whenever the FP32 cell sums are exact (integer
  * visibilities, |partial sums| < 2^24); otherwise equal up to the order of the adds.
- * Rows of K % 16 != 0 or at an unaligned address are padded first, as in
- * ftdx_herk_pol_reduce. */
+ * Without a forced tile large calls run the pipelined kernel over E3M2 rows, as ftdx_herk, and calls of
+ * many baselines per cell add pairs of mirror cells once, to half planes that a closing pass adds to the
+ * grid: at most 256 MB of them, beside the rows in the same per-stream scratch.  Other calls, and
+ * those without scratch, pad rows of K % 16 != 0 or at an unaligned address first, as
+ * ftdx_herk_pol_reduce does. */
 int ftdx_herk_pol_grid(ftdx_context* ctx, const void* A, int N, int K, int n_chan, int n_pol,
                        const float* baseline_uv_m, const double* freq_hz, float* uv_grid, int Ng,
                        int freq_offset, float cell_size_rad, float alpha, void* stream);
