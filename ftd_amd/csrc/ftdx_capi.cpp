@@ -317,15 +317,18 @@ size_t frag_scratch_bytes(const HerkPlainArgs& a) {
     return (size_t)frag_rows_bytes(a.N, a.K, a.nseg) * grp * frag_chunk_cap(a.N, a.K, a.nseg * grp, a.batch / grp);
 }
 
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone) return false;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Fragment-row scratch of this stream, or NULL where the call has to do without: under
 // capture (a captured call must not depend on a buffer that a later call may replace), with
 // four other streams calling, on another device, or when memory is short.
 uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    if (capturing(s)) return nullptr;
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) (void)hipGetLastError();
     StreamSlot* slot = ctx->frag.pick(ctx->device, dev, s);
@@ -1099,7 +1102,10 @@ int ftdx_herk_mx(ftdx_context* ctx, const void* A, void* C, int N, int K, int ba
     const int fmt = ftdx::mx_format(compute);
     if (ctx->forced_cfg < 0 && ftdx::mxpipe_takes(N, K, batch_count, fmt)) {
         const int64_t per = ftdx::mxfrag_rows_bytes(N, K, fmt);
-        const int cap = std::min(ftdx::chunk_cap_bytes((size_t)per, batch_count), 65535);
+        int cap = std::min(ftdx::chunk_cap_bytes((size_t)per, batch_count), 65535);
+        // a captured call cannot allocate: smaller chunks in what eager calls of other shapes left
+        if ((size_t)per * cap > ctx->mx_codes_cap && ctx->mx_codes_cap >= (size_t)per && ftdx::capturing(s))
+            cap = (int)(ctx->mx_codes_cap / (size_t)per);
         int rc = ftdx::ensure_scratch(ctx->mx_codes, ctx->mx_codes_cap, (size_t)per * cap, "ftdx_herk_mx: scratch");
         if (rc != FTDX_OK) return rc;
         e = ftdx::run_mxpipe(ctx->mx_codes, A, C, N, K, batch_count, cap, input, fmt, ctx->mx_rounding,

@@ -131,3 +131,30 @@ def test_eager_calls_beside_a_capture(dev, grow):
     assert torch.equal(y, x + 1.0)
     assert bool((large[1][:, 0] == torch.tensor([4096.0, 0.0], device=dev)).all())
     assert bool((large[1][..., 0] == 4096.0).all())
+
+
+def test_block_scaled_call_after_a_larger_one(dev):
+    """A captured block-scaled call gets along with the scratch that an eager call of another, larger shape
+    left: smaller chunks where its own would be more."""
+    import torch
+    from ftd_amd import ftdx
+    ctx = ftdx.CutlassComplexGemm()
+    kw = dict(input=ftdx.InputPrecision.INT4, compute=ftdx.ComputePrecision.FP6, output="fp16")
+    gen = torch.Generator(device=dev).manual_seed(2)
+
+    def qc(n):
+        return torch.randint(0, 256, (n,), generator=gen, dtype=torch.uint8, device=dev)
+
+    N, K, B = 8192, 16384, 2  # one channel's fragments (210 MB) are a chunk
+    big = torch.zeros((B, N * (N + 1) // 2, 2), dtype=torch.float16, device=dev)
+    ftdx.herk_mx(ctx, qc(N * K * B), N, K, B, C=big, **kw)
+    N, K, B = 1024, 1024, 200  # 328 MB in chunks of its own
+    A = qc(N * K * B)
+    C, ref = (torch.zeros((B, N * (N + 1) // 2, 2), dtype=torch.float16, device=dev) for _ in range(2))
+    ftdx.herk_mx(ftdx.CutlassComplexGemm(), A, N, K, B, C=ref, **kw)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            ftdx.herk_mx(ctx, A, N, K, B, C=C, **kw)
+        _replay(torch, graph, [C], [ref], ctx)
