@@ -112,12 +112,12 @@ inline bool plain_stores_pay(const HerkPlainArgs& a, bool out_fp16) {
 }
 
 // Whether interior tiles may store straight from their accumulators at all: not in up to two rounds of
-// tiles of up to three row blocks, where few are inside and each is waited for.  us, staged / direct:
-// 256 x 64, K = 256, FP32 12.1 / 13.2; 384 x 128, K = 512, FP16 33.0 / 37.9; 256 x 256, K = 640, FP16
-// 36.9 / 41.4; but 512 x 64, K = 256 29.8 / 24.7, 256 x 512, 2 x 200 90 / 85, and E3M2 rows, whose
-// conversion ran before (256 x 256, K = 640, FP16 61 / 59).
+// tiles (one of E3M2 rows, whose conversion ran before) of up to three row blocks, where few are inside and
+// each is waited for.  us, staged / direct: 256 x 64, K = 256, FP32 12.1 / 13.2; 384 x 128, K = 512, FP16
+// 33.0 / 37.9; 256 x 256, K = 640, FP16 36.9 / 41.4, E3M2 61 / 59; 256 x 128, K = 256, E3M2 27.1 / 28.3; but
+// 512 x 64, K = 256 29.8 / 24.7, 256 x 512, 2 x 200 90 / 85.
 inline bool direct_stores_pay(const HerkPlainArgs& a, int tile_cols, int64_t tiles) {
-    return a.N > 3 * tile_cols || tiles > 1024 || a.precast == 2;
+    return a.N > 3 * tile_cols || tiles > (a.precast == 2 ? 512 : 1024);
 }
 
 // Lower-triangle tiles per problem for a configuration.

@@ -34,7 +34,8 @@ hipError_t launch_mx_quantize_rows(const void* X, const void* X2, int input, int
 
 // Dense E2M1 operand rows (LOAD_MX4D): rows_out [rows][nblkp][2][16] code bytes (Re part,
 // Im part), row pitch nblkp * 32 bytes; scales [rows / nrow][nblkp / 4][nrow][8], the
-// (Re, Im) E8M0 bytes of each 4-block stage.  nblkp = mx_dense_blocks(K), a multiple of 4.
+// (Re, Im) E8M0 bytes of each 4-block stage.  nblkp = mx_dense_blocks(K), a multiple of 4.  For calls
+// with a forced tile, and those whose fragments are too large for the pipelined form.
 int mx_dense_blocks(int K);
 hipError_t launch_mx_quantize_dense(const void* X, int input, int rounding, uint8_t* rows_out, uint8_t* scales,
                                     int64_t rows, int64_t nrow, int K, hipStream_t s);

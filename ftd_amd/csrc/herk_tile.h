@@ -79,6 +79,8 @@ __device__ __forceinline__ void wait_vmcnt() {
 // LOAD_MX4D: dense E2M1 rows (OPF_MX4D), interior tiles of 64-sample-stage configurations
 // only: each 128-byte stage row holds 4 blocks of 32 samples (16 code bytes of Re, then Im),
 // and TileJob::S holds the scales, [stage][row][8]: (Re, Im) bytes of the stage's 4 blocks.
+// The HERK takes the LOAD_MX modes for a forced tile, and where the fragments of the pipelined form
+// (mxpipe_takes in ftdx_capi.cpp) are too large; the GEMM's FP6 / FP4 compute always takes LOAD_MX6 / LOAD_MX4.
 enum LoadMode { LOAD_VEC16 = 0, LOAD_BYTES = 1, LOAD_FP8 = 2, LOAD_BF6 = 3, LOAD_MX6 = 4, LOAD_MX4 = 5,
                 LOAD_MX4D = 6 };
 
@@ -1099,7 +1101,8 @@ struct TileRunner {
     // issued right after the barrier that opens stage s, into the buffer of stage s - 1,
     // which every wave finished reading before that barrier.  The barrier is written out
     // (wait for this wave's loads of stage s + 1 only, then s_barrier): the release fence
-    // of __syncthreads() would also wait for the loads of stage s + 2.
+    // of __syncthreads() would also wait for the loads of stage s + 2.  The 256 x 128 configurations run
+    // it, which the GEMM takes when they are forced (its default is the 128 x 128 tile).
     static constexpr int DMA3_LDS = 3 * DSTAGE;
     static constexpr bool DMA3_OK = DMA_OK && Cfg::WG_PER_CU == 1 && DMA3_LDS <= 160 * 1024;
 
