@@ -60,6 +60,8 @@ struct ftdx_context {
     // pre-cast FP8 operand rows for the unfused / FP16-input paths
     uint8_t* precast = nullptr;
     size_t precast_cap = 0;
+    size_t pad_refused = 0;         // bytes of padded rows that reserve_padded found no memory for
+    bool precast_captured = false;  // a program's captured calls use the buffer
     // fragment rows of the pipelined HERK and half planes of the gridding, one buffer per stream; a
     // call without one takes the fused tile, which needs none
     ftdx::StreamSlots frag;
@@ -205,11 +207,24 @@ int pick_chunk(int cfg, int N, int batch, int cmax, int units_out = 1) {
     return pick_chunk_of(slots, (int64_t)herk_tiles(cfg, N) * units_out, batch, cmax);
 }
 
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone) return false;
+    (void)hipGetLastError();
+    return true;
+}
+
+// A launch that reads ctx->precast on st: under the program's own capture, every replay will.
+void note_precast_use(ftdx_context* ctx, hipStream_t st) {
+    if (!ctx->precast_captured && st != ctx->cap_stream && capturing(st)) ctx->precast_captured = true;
+}
+
 // The pre-cast path of one call: per chunk of batches, convert A's rows into the
 // context's scratch (FP8 planar rows, or E3M2 rows when bf6), then run the tile over
 // them.  The scratch must hold N * precast_chunk_cap(...) rows of 2 * Kp bytes.
 hipError_t run_precast(ftdx_context* ctx, const HerkPlainArgs& a, int input, bool bf6, int cfg, bool fp16,
                        int remap, hipStream_t st) {
+    note_precast_use(ctx, st);
     const int Kp = precast_row_samples(a.K);
     const int chunk = pick_chunk(cfg, a.N, a.batch, precast_chunk_cap(a.N, a.K, a.batch));
     const int64_t in_bytes = (int64_t)a.N * a.K * (input == FTDX_INPUT_FP16 ? 4 : 1);
@@ -289,6 +304,7 @@ int padded_chunk_cap(int N, int K, int batch) {
 template <class Launch>
 hipError_t run_padded(ftdx_context* ctx, const HerkPlainArgs& a, int cfg, int out_elem, hipStream_t st,
                       Launch&& launch) {
+    note_precast_use(ctx, st);
     const int Kq = padded_row_samples(a.K, cfg);
     const int grp = std::max(a.seg_group, 1), in_per = a.nseg * grp;
     const int units = a.batch / grp;
@@ -317,11 +333,20 @@ size_t frag_scratch_bytes(const HerkPlainArgs& a) {
     return (size_t)frag_rows_bytes(a.N, a.K, a.nseg) * grp * frag_chunk_cap(a.N, a.K, a.nseg * grp, a.batch / grp);
 }
 
-bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone) return false;
-    (void)hipGetLastError();
-    return true;
+// Frees `old`, allocates `need` bytes: nullptr if there is no memory.  Another stream or thread may be
+// capturing: only in relaxed mode does an allocation leave that capture alone, and hipDeviceSynchronize
+// does in none (hipFree waits for the device by itself).
+uint8_t* replace_scratch(uint8_t* old, size_t need) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (old) (void)hipFree(old);
+    uint8_t* p = nullptr;
+    if (hipMalloc(&p, need) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+    }
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return p;
 }
 
 // Fragment-row scratch of this stream, or NULL where the call has to do without: under
@@ -335,17 +360,9 @@ uint8_t* frag_scratch(ftdx_context* ctx, size_t need, hipStream_t s) {
     if (!slot) return nullptr;
     if (slot->cap < need || slot->stream != s) {
         if (ctx->frag.refused(need)) return nullptr;
-        // another stream or thread may be capturing: only in this mode does an allocation leave that
-        // capture alone, and hipDeviceSynchronize does in none (hipFree waits for the device by itself)
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-        if (slot->rows) (void)hipFree(slot->rows);
+        uint8_t* const old = slot->rows;
         *slot = StreamSlot();
-        const hipError_t e = hipMalloc(&slot->rows, need);
-        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            slot->rows = nullptr;
+        if (!(slot->rows = replace_scratch(old, need))) {
             ctx->frag.refuse(need);
             return nullptr;
         }
@@ -628,16 +645,18 @@ int ensure_scratch(uint8_t*& p, size_t& cap, size_t need, const char* what) {
 
 // Grows the pre-cast operand buffer; captured graphs of the pre-cast path point at
 // the old buffer, so they are dropped when it moves.
+void drop_precast_graphs(ftdx_context* ctx) {
+    for (auto& gph : ctx->graphs)
+        if (gph.used && gph.mode != 0) {
+            (void)hipGraphExecDestroy(gph.exec);
+            gph = ftdx_context::GraphEntry();
+        }
+}
+
 int grow_precast(ftdx_context* ctx, size_t need, const char* what) {
     const uint8_t* before = ctx->precast;
     int rc = ensure_scratch(ctx->precast, ctx->precast_cap, need, what);
-    if (rc == FTDX_OK && before && before != ctx->precast) {
-        for (auto& gph : ctx->graphs)
-            if (gph.used && gph.mode != 0) {
-                (void)hipGraphExecDestroy(gph.exec);
-                gph = ftdx_context::GraphEntry();
-            }
-    }
+    if (rc == FTDX_OK && before && before != ctx->precast) drop_precast_graphs(ctx);
     return rc;
 }
 
@@ -649,7 +668,8 @@ void free_scratch(ftdx_context* ctx) {
         if (*p) (void)hipFree(*p);
         *p = nullptr;
     }
-    ctx->mx_codes_cap = ctx->cal_part_cap = ctx->cal_herm_cap = ctx->precast_cap = 0;
+    ctx->mx_codes_cap = ctx->cal_part_cap = ctx->cal_herm_cap = ctx->precast_cap = ctx->pad_refused = 0;
+    ctx->precast_captured = false;
 }
 
 // Other threads may be capturing: relaxed mode, and no wait but hipFree's own.
@@ -662,9 +682,15 @@ DefaultContext::~DefaultContext() {
 }
 
 // The padded rows of a call that the pipelined kernel runs without them: the same call under capture
-// takes the fused tile and can allocate nothing.  Without memory for them it does without.
+// takes the fused tile and can allocate nothing.  A buffer that captured calls use stays where it is.
+// Without memory for the rows the call does without, and a size that failed is not tried again before
+// the scratch is given back.
 void reserve_padded(ftdx_context* ctx, size_t need) {
-    if (grow_precast(ctx, need, "padded rows") != FTDX_OK) (void)hipGetLastError();
+    if (need <= ctx->precast_cap || ctx->precast_captured || (ctx->pad_refused && need >= ctx->pad_refused)) return;
+    ctx->precast = replace_scratch(ctx->precast, need);
+    ctx->precast_cap = ctx->precast ? need : 0;
+    if (!ctx->precast) ctx->pad_refused = need;
+    drop_precast_graphs(ctx);
 }
 
 // A operand formats of the complex GEMM
@@ -689,6 +715,7 @@ int gemm_run(ftdx_context* ctx, const uint8_t* brows, GemmInput kind, const void
     const int64_t rows = (int64_t)M * batch;
     int rc = grow_precast(ctx, (size_t)rows * Kp * 2 + 16, "gemm: A rows");
     if (rc != FTDX_OK) return rc;
+    note_precast_use(ctx, s);
     hipError_t e = hipSuccess;
     if (K > 0) {
         if (kind == GEMM_A_FP16_PLANAR)
@@ -1466,6 +1493,7 @@ int ftdx_correlate_ftd(ftdx_context* ctx, const void* raw, void* tri_fp32, int n
                                                            : ftdx::direct_tile_to_cfg(ctx->direct_tile),
                                       n_ant, (int)batch);
     const int remap = ctx->forced_remap >= 0 ? ctx->forced_remap : 1;
+    ftdx::note_precast_use(ctx, static_cast<hipStream_t>(stream));
     hipError_t e = ftdx::run_ftd_payload(static_cast<const uint8_t*>(raw), static_cast<float*>(tri_fp32),
                                          ctx->precast, n_ant, n_chan, n_time, n_time_inner, n_pol,
                                          twos != 0, cfg, remap, static_cast<hipStream_t>(stream));

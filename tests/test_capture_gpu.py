@@ -100,9 +100,10 @@ def test_streams_that_come_and_go(oracle, dev):
 
 
 @pytest.mark.parametrize("grow", [False, True])
-def test_eager_calls_beside_a_capture(dev, grow):
+@pytest.mark.parametrize("K", [2048, 2040])
+def test_eager_calls_beside_a_capture(dev, grow, K):
     """A capture in progress (global mode) survives eager calls on another stream that need scratch for
-    the first time, or more of it than before."""
+    the first time, or more of it than before; K = 2040: rows that the fused tile would pad."""
     import torch
     from ftd_amd import ftdx
     ctx = ftdx.CutlassComplexGemm()
@@ -117,7 +118,7 @@ def test_eager_calls_beside_a_capture(dev, grow):
         return A, C, lambda: ctx.herk(A, C, N, K, B, input=ftdx.InputPrecision.INT4, output=ftdx.OutputPrecision.FP32,
                                       stream=other, tune=False)
 
-    small, large = call(2048, 2048, 2), call(2048, 2048, 4)  # the pipelined kernel's
+    small, large = call(2048, K, 2), call(2048, K, 4)  # the pipelined kernel's
     if grow:
         assert small[2]() == 0
         torch.cuda.synchronize()
@@ -129,8 +130,8 @@ def test_eager_calls_beside_a_capture(dev, grow):
     graph.replay()
     torch.cuda.synchronize()
     assert torch.equal(y, x + 1.0)
-    assert bool((large[1][:, 0] == torch.tensor([4096.0, 0.0], device=dev)).all())
-    assert bool((large[1][..., 0] == 4096.0).all())
+    assert bool((large[1][:, 0] == torch.tensor([2.0 * K, 0.0], device=dev)).all())
+    assert bool((large[1][..., 0] == 2.0 * K).all())
 
 
 def test_block_scaled_call_after_a_larger_one(dev):
@@ -158,3 +159,33 @@ def test_block_scaled_call_after_a_larger_one(dev):
         with torch.cuda.graph(graph, stream=side):
             ftdx.herk_mx(ctx, A, N, K, B, C=C, **kw)
         _replay(torch, graph, [C], [ref], ctx)
+
+
+def test_padded_rows_of_a_captured_call_stay(oracle, dev):
+    """A captured call on padded rows keeps its scratch: larger eager calls, which run the pipelined kernel,
+    leave it where the replays read and write it."""
+    import torch
+    from ftd_amd import ftdx
+    ctx = ftdx.CutlassComplexGemm()
+
+    def make(N, K, B):
+        qc = oracle.gen_qc_uniform(K + B, N * K * B)
+        A, C = torch.from_numpy(qc).to(dev), torch.zeros((B, N * (N + 1) // 2, 2), device=dev)
+        return C, lambda: ctx.herk(A, C, N, K, B, input=ftdx.InputPrecision.INT4, output=ftdx.OutputPrecision.FP32,
+                                   tune=False), qc
+
+    C, call, qc = make(1000, 1000, 12)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        assert call() == 0
+        torch.cuda.synchronize()
+        ref = C.clone()
+        assert np.array_equal(ref[:1].cpu().numpy(), oracle.herk_f32(qc[:10 ** 6], 1000, 1000, 1))
+        with torch.cuda.graph(graph, stream=side):
+            assert call() == 0
+        for K, B in ((1500, 20), (1999, 24)):
+            D, big, _ = make(1000, K, B)
+            assert big() == 0
+            junk = [torch.full((1 << 22,), 0x5A, dtype=torch.uint8, device=dev) for _ in range(16)]
+            _replay(torch, graph, [C], [ref], ctx)
+            assert all(bool((j == 0x5A).all()) for j in junk)
